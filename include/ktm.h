@@ -293,8 +293,9 @@ int ktm_poststack_adjoint(const ktm_plan *plan, const float *image, const float 
  *   I[X][h][t] = sum over traces of class h in aperture of the CLOSED filtered
  *                trace at q, Catmull-Rom cubic interpolation (C1 in q);
  *   J          = sum_{X,t} sum_{h<nh-1} (I[X][h+1][t] - I[X][h][t])^2.
- * dJ/dV comes from a hand-written backward pass that recomputes traveltimes
- * per time chunk of `chunk` (<= 256) samples instead of storing them. */
+ * dJ/dV is hand-written: per time chunk of `chunk` (<= 256) samples the
+ * derivative of each offset class's image is summed beside the image itself,
+ * and nothing is stored per contribution. */
 typedef struct ktm_vgrad ktm_vgrad;
 int ktm_vgrad_create(ktm_vgrad **out, const ktm_config *cfg, int ns, float dt, int nt_nodes,
                      int nx_nodes, int chunk);

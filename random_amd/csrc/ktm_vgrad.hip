@@ -20,15 +20,16 @@
  *
  * k_vgrad: one workgroup owns one image column X and one time chunk of
  * `chunk` (<= 256) samples, one lane per sample.  The offset classes stream
- * in order: pass 1 sums class h+1 (Kahan) while the lane holds I[h-1..h]
- * of its sample in registers, adds its share of J (FP64), and with dJ/dI[h]
- * known pass 2 walks class h's traces again and recomputes each traveltime
- * to accumulate
- *   dJ/dv(X,t) = sum_h dJ/dI[h][t] sum_c F'(q_c) dq_c/dv.
- * Nothing per contribution is stored: the time chunk and a window of three
- * classes bound the working set to registers.  Traces are binned on the host
- * by (offset class, CMP inline coordinate), so a column's traces of one class
- * are a contiguous range; every wave walks the ranges itself (gates
+ * in order: one pass over the traces of class h+1 sums I[h+1] (Kahan) and,
+ * when the gradient is wanted, S[h+1] = sum_c F'(q_c) (a/s1 + b/s2)_c, while
+ * the lane holds I[h-1..h] and S[h] of its sample in registers; it adds its
+ * share of J (FP64), and with dJ/dI[h] known
+ *   dJ/dv(X,t) = sum_h (dJ/dI[h][t] kfac S[h]), kfac = -1/(v^3 dt).
+ * S does not depend on dJ/dI, so the traveltimes and the taps are formed once
+ * per contribution for both.  Nothing per contribution is stored: the time
+ * chunk and a window of three classes bound the working set to registers.
+ * Traces are binned on the host by (offset class, CMP inline coordinate), so
+ * a column's traces of one class are a contiguous range; every wave walks the ranges itself (gates
  * lane-parallel, ballot, then the passing traces in order) and needs no
  * barrier.  At bind, k_vg_tables lays the geometry and the traces out in
  * that order, each trace zero-padded (one sample before, five after): the
@@ -199,22 +200,25 @@ __global__ void k_vg_tables(const float *__restrict__ prep, int64_t row,
     }
 }
 
-/* One pass over the traces of class h for this lane's sample t.  The
+/* One pass over the traces of one class for this lane's sample t.  The
  * traveltime is formed as q = t + m/dt with the moveout
  *   m = a r / (s1 + th) + b r / (s2 + th),  s1 = sqrt(th^2 + a r),  th = t dt / 2,
  * (equal to (s1 + s2)/dt - t), so FP32 rounds the moveout and not the whole
  * traveltime: ulp(m) instead of ulp(q) (1e-4 samples at q ~ 2000).
- * FWD: returns the Kahan sum of F(q); otherwise sum F'(q) (a/s1 + b/s2).
+ * Returns the Kahan sum of F(q); with GRAD also S = sum F'(q) (a/s1 + b/s2)
+ * from the same traveltimes and taps: 7 VALU instructions more per
+ * contribution where a second pass over the class repeated all 41.
  * lo..hi are positions in the binned order, so they index sgeom and taps
  * directly.  The interval T = t + floor(min(m/dt, ns + 2 - t)) stays in
  * [0, ns + 2] for every lane (m >= 0; inactive lanes have r = 0). */
-template <bool FWD>
+template <bool GRAD>
 __device__ __forceinline__ float vg_class_pass(const VgArgs &a, int lo, int hi, float IX,
                                                float r, float th, float t2, int t, int lane,
-                                               float2 *sAB)
+                                               float2 *sAB, float &S)
 {
     const float dmax = (float)(a.ns + 2 - t);   /* q clamped to ns + 2: a zero interval */
     float acc = 0.0f, cmp = 0.0f;
+    S = 0.0f;
     for (int b0 = lo; b0 < hi; b0 += VG_WAVE) {
         const int k = b0 + lane;
         float ga = 0.0f, gb = 0.0f;
@@ -266,7 +270,7 @@ __device__ __forceinline__ float vg_class_pass(const VgArgs &a, int lo, int hi, 
                 const float d = fminf(__builtin_fmaf(ar, w1, br * w2) * a.rdt, dmax);
                 const float Df = floorf(d);
                 uu[c] = d - Df;
-                dqv[c] = __builtin_fmaf(A, i1, B * i2);
+                if (GRAD) dqv[c] = __builtin_fmaf(A, i1, B * i2);
                 /* taps T-1..T+2 at a 32-bit byte offset from the trace's
                  * (scalar) row base */
                 cf[c] = *(const vg_f4 *)(Fr + (uint32_t)(t + (int)Df) * 4u);
@@ -274,14 +278,11 @@ __device__ __forceinline__ float vg_class_pass(const VgArgs &a, int lo, int hi, 
 #pragma unroll
             for (int c = 0; c < VG_G; ++c) {
                 if (c < nb) {
-                    if (FWD) {
-                        const float y = cr_eval<false>(cf[c], uu[c]) - cmp;
-                        const float s = acc + y;
-                        cmp = (s - acc) - y;
-                        acc = s;
-                    } else {
-                        acc = __builtin_fmaf(cr_eval<true>(cf[c], uu[c]), dqv[c], acc);
-                    }
+                    const float y = cr_eval<false>(cf[c], uu[c]) - cmp;
+                    const float s = acc + y;
+                    cmp = (s - acc) - y;
+                    acc = s;
+                    if (GRAD) S = __builtin_fmaf(cr_eval<true>(cf[c], uu[c]), dqv[c], S);
                 }
             }
         }
@@ -289,6 +290,12 @@ __device__ __forceinline__ float vg_class_pass(const VgArgs &a, int lo, int hi, 
     return acc;
 }
 
+/* Bound by VALU issue (the moveout and the cubic of every contribution; two
+ * reciprocal square roots and two reciprocals of it at a quarter of the
+ * rate).  J + dJ/dV of 48,000 traces x 2001 samples into 1000 columns x 64
+ * classes: 47.1 ms with a second pass per class for the gradient, 26.7 ms
+ * with S summed beside I (55 VGPRs, 8 waves per SIMD either way), same bits. */
+template <bool GRAD>
 __global__ void __launch_bounds__(VG_NT) k_vgrad(const VgArgs a)
 {
     __shared__ double sRed[VG_NT / VG_WAVE];
@@ -326,29 +333,29 @@ __global__ void __launch_bounds__(VG_NT) k_vgrad(const VgArgs a)
 
     /* The offset classes stream in order: the lane holds I[h-1..h+1] of its
      * sample, the objective share adds (I[h+1] - I[h])^2, and as soon as
-     * dJ/dI[h] = 2 ((I[h] - I[h-1]) - (I[h+1] - I[h])) is known the second
-     * pass recomputes class h's traveltimes for dJ/dv.  No per-class array,
-     * so no LDS bounds the occupancy. */
+     * dJ/dI[h] = 2 ((I[h] - I[h-1]) - (I[h+1] - I[h])) is known it weighs
+     * S[h] into dJ/dv.  No per-class array, so no LDS bounds the occupancy. */
     double jl = 0.0;
-    float dprev = 0.0f, g = 0.0f;
-    float Ih = vg_class_pass<true>(a, rg[0], rg[1], IX, r, th, t2, t, lane, sABw[wv]);
+    float dprev = 0.0f, g = 0.0f, Sh = 0.0f;
+    float Ih = vg_class_pass<GRAD>(a, rg[0], rg[1], IX, r, th, t2, t, lane, sABw[wv], Sh);
     if (!act) Ih = 0.0f;
     for (int h = 0; h < a.nh; ++h) {
-        float In = 0.0f, dn = 0.0f;
+        float In = 0.0f, dn = 0.0f, Sn = 0.0f;
         if (h + 1 < a.nh) {
-            In = vg_class_pass<true>(a, rg[2 * h + 2], rg[2 * h + 3], IX, r, th, t2, t, lane, sABw[wv]);
+            In = vg_class_pass<GRAD>(a, rg[2 * h + 2], rg[2 * h + 3], IX, r, th, t2, t, lane,
+                                     sABw[wv], Sn);
             if (!act) In = 0.0f;
             dn = In - Ih;
         }
         jl += (double)dn * (double)dn;
         if (a.cig && act) a.cig[((int64_t)X * a.nh + h) * a.ns + t] = Ih;
-        if (a.gv) {
+        if (GRAD) {
             const float rh = 2.0f * (dprev - dn);
-            const float S = vg_class_pass<false>(a, rg[2 * h], rg[2 * h + 1], IX, r, th, t2, t, lane, sABw[wv]);
-            g = __builtin_fmaf(rh, S, g);
+            g = __builtin_fmaf(rh, Sh, g);
         }
         dprev = dn;
         Ih = In;
+        Sh = Sn;
     }
     for (int o = VG_WAVE / 2; o > 0; o >>= 1) jl += __shfl_down(jl, o);
     if (lane == 0) sRed[wv] = jl;
@@ -358,7 +365,7 @@ __global__ void __launch_bounds__(VG_NT) k_vgrad(const VgArgs a)
         for (int w = 0; w < VG_NT / VG_WAVE; ++w) s += sRed[w];
         a.part[tile] = s;
     }
-    if (a.gv && act) a.gv[(int64_t)X * a.ns + t] = kfac * g;
+    if (GRAD && act) a.gv[(int64_t)X * a.ns + t] = kfac * g;
 }
 
 /* ------------------------------------------------------------------------ */
@@ -584,7 +591,10 @@ extern "C" int ktm_vgrad_eval(ktm_vgrad *p, const float *V, double *J, double *d
     if (a.run < 1) a.run = 1;
     const int64_t span = 8 * (int64_t)a.run;
     const int64_t nblk = ((int64_t)ntiles + span - 1) / span * span;
-    hipLaunchKernelGGL(k_vgrad, dim3((unsigned)nblk), dim3(VG_NT), 0, st, a);
+    if (dJdV)
+        hipLaunchKernelGGL(k_vgrad<true>, dim3((unsigned)nblk), dim3(VG_NT), 0, st, a);
+    else
+        hipLaunchKernelGGL(k_vgrad<false>, dim3((unsigned)nblk), dim3(VG_NT), 0, st, a);
     VG_TRY(hipGetLastError());
     if (dJdV) {
         const int64_t n1 = (int64_t)p->nxp * p->nt_nodes;

@@ -11,8 +11,8 @@ writes one common-image gather of nh offset classes per column and
 
 measures how far the gathers are from flat.  ``VelocityGradient`` evaluates
 J and dJ/dV on the GPU: one workgroup owns (column, time chunk), streams the
-offset classes through registers and recomputes the traveltimes for the
-backward pass instead of storing them.  Binding copies the traces into a
+offset classes through registers and sums each class's image and its
+velocity derivative in one pass, storing nothing per contribution.  Binding copies the traces into a
 table the plan holds, binned by (offset class, CMP) and zero-padded.  The reference has no such operator
 (its nearest-node velocity, Kirchhoff.c:1357-1358,1376, and floor(dsr/dt),
 1384, have zero derivative almost everywhere).
