@@ -529,8 +529,9 @@ struct MigArgs {
     int ns, nh, nxp, nyp, nx, ny, jobs_y, nvel_xl, nsm;
     int tiles_x, ntiles, tx_cols, ty_cols, run;
     int rx0, ry0, rx1, ry1;          /* migrated region [rx0,rx1) x [ry0,ry1) */
-    /* Kahan variants: the block's 512-trace chunks dealt round-robin to
-     * nparts parts (chunk c to part c mod nparts), part = blockIdx.z, so that
+    int align16;                     /* prep (and so every row) 16-byte aligned */
+    /* Kahan variants: the block's chunks of a workgroup's thread count of
+     * traces dealt round-robin to nparts parts (chunk c to part c mod nparts), part = blockIdx.z, so that
      * every part spans the whole survey and its workgroups carry like loads;
      * part 0 adds into km/fold/comp, part p > 0 writes its sums into
      * parts + (p-1) * 3 * part_n, region layout [X-rx0][Y-ry0][h][t] */
@@ -629,91 +630,149 @@ __device__ __forceinline__ float clamp_ns(float q, float hi)
     return __builtin_amdgcn_fmed3f(q, 0.0f, hi);
 }
 
-/* Slots whose traveltime chains the exact path evaluates side by side
- * under one test for the rare path (K divisible by it, else 2) */
-#ifndef KTM_SLOT_GROUP
-#define KTM_SLOT_GROUP 2
-#endif
+/* The exact variants' form of q, in units of nsh = ns + 1/2: with
+ * rsn = RN(1/(v2 dt^2 nsh^2)) and tqn = RN(t^2/(4 nsh^2)) (double, rounded
+ * once)
+ *   p = RN( sqrt_hw(fma(dIS2, rsn, tqn)) + sqrt_hw(fma(dIR2, rsn, tqn)) ),
+ * q = p nsh without rounding.  The radicand's two constants carry one
+ * rounding each, at most u of a sum of non-negative terms, and the FMA u: 2u,
+ * as above (rs and the FMA), so |p nsh - Q| <= 7u Q holds unchanged.  p is
+ * limited to 1 by the clamp modifier of its sum, at no cost (a v_med3 is a
+ * quarter-rate instruction): a limited sample has Q > ns for certain, its
+ * index is ns, and half a sample from an integer it is never ambiguous. */
+__device__ __forceinline__ float fast_rsn(float v2, float dt, float nsh)
+{
+    return (float)(1.0 / ((double)v2 * (double)dt * (double)dt * ((double)nsh * (double)nsh)));
+}
+__device__ __forceinline__ float fast_tqn(int t, float nsh)
+{
+    const double r = (double)t / (2.0 * (double)nsh);
+    return (float)(r * r);
+}
+__device__ __forceinline__ float fast_p(float dIS2, float dIR2, float rsn, float tqn)
+{
+    return __builtin_amdgcn_fmed3f(__builtin_amdgcn_sqrtf(__builtin_fmaf(dIS2, rsn, tqn)) +
+                                       __builtin_amdgcn_sqrtf(__builtin_fmaf(dIR2, rsn, tqn)),
+                                   0.0f, 1.0f);
+}
 
-/* Queue of the speculative exact path: items per lane and staged batch (a
- * lane's further ambiguous samples of the batch take the inline exact path) */
-#define KTM_SPEC_Q 1
+/* floor(q), q = p nsh, by one rounding: M = RN(q + (2^23 - 1/2)) holds
+ * 2^23 + floor(q) in its mantissa when M >= 2^23, i.e. for q >= 1/4 (a tie,
+ * q an integer, gives that integer or the one below; it is always
+ * ambiguous); center = floor + 1/2 exactly; dev = q - center in
+ * [-1/2, 1/2].  low: q may be below 1/4 (only t = 0 can be), where M is
+ * raised to 2^23. */
+#define KTM_FLOOR_MAGIC 8388607.5f
+#define KTM_FLOOR_BITS 0x4B000000u     /* bits of 2^23 */
+struct FloorP { float M, center, dev; };
+__device__ __forceinline__ FloorP floor_p(float p, float nsh, bool low)
+{
+    FloorP r;
+    r.M = __builtin_fmaf(p, nsh, KTM_FLOOR_MAGIC);
+    if (low) r.M = fmaxf(r.M, 8388608.0f);
+    r.center = r.M - KTM_FLOOR_MAGIC;
+    r.dev = __builtin_fmaf(p, nsh, -r.center);
+    return r;
+}
+__device__ __forceinline__ int floor_T(const FloorP &f)
+{
+    return (int)(__float_as_uint(f.M) - KTM_FLOOR_BITS);
+}
+/* An integer within eps (q + 1) of q: the distance to the nearest integer is
+ * 1/2 - |dev|, so |dev| >= 1/2 - eps (q + 1) (the rounding of dev, 3e-8, is
+ * inside the 8u against 7u of the bound).  The kernel takes the threshold at
+ * the largest q that the trace can have in the wave's samples: one value per
+ * trace instead of an FMA per sample, for a few more ambiguous samples. */
+__device__ __forceinline__ float ambiguous_from(float q) { return 0.5f - KTM_FAST_EPS_S * (q + 1.0f); }
 
 /* The reference traveltime index of a sample with every rule of the exact
  * path: the fast form, and where an integer lies within its error bound the
- * reference arithmetic, ns when the sample is past the trace for certain. */
-__device__ __forceinline__ int reference_T(float dIS2, float dIR2, float rs, float tq, float t2,
-                                           float v2, float dt, float rdt, int ns)
+ * reference arithmetic.  low as in floor_p. */
+__device__ __forceinline__ int reference_T(float dIS2, float dIR2, float rsn, float tqn, float t2,
+                                           float v2, float dt, float rdt, int ns, bool low)
 {
-    constexpr float EPS = KTM_FAST_EPS_S;
-    const float nsf = (float)ns;
-    const float q = fast_qs(dIS2, dIR2, rs, tq);
-    const float qc = clamp_ns(q, nsf);
-    if (!fast_ambiguous(qc, EPS)) return fast_T(qc);
-    if (q - nsf >= __builtin_fmaf(q, EPS, EPS)) return ns;
+    const float nsh = (float)ns + 0.5f;
+    const float p = fast_p(dIS2, dIR2, rsn, tqn);
+    const FloorP f = floor_p(p, nsh, low);
+    if (fabsf(f.dev) < ambiguous_from(p * nsh)) return floor_T(f);
     return exact_T(dIS2, dIR2, t2, v2, 1.0f / v2, dt, rdt, ns);
 }
 
-/* One workgroup = 8 waves = NCOL image columns x W time segments.  Each lane
+typedef __attribute__((address_space(3))) float lds_float;
+typedef __attribute__((address_space(3))) void lds_void;
+typedef __attribute__((address_space(1))) const void global_void;
+
+/* One workgroup = NW waves = NCOL image columns x W time segments.  Each lane
  * owns K samples t = seg*64K + 64k + lane of its column: the image values
- * (km, fold count, Kahan compensation) and the fast path's rs = RN(1/(v^2
- * dt^2)) and tq = t^2/4 stay in registers for the whole launch.  Traces
- * stream through LDS in trace order: a chunk of 512 is filtered to those
- * whose CMP can reach the tile (ordered compaction), then staged 8 at a
- * time; per staged trace the aperture and slab gates of every column are
- * evaluated lane-parallel (one lane per trace) and the passing traces are
- * walked in order.
+ * (km, fold count, Kahan compensation) and the per-sample constants of the
+ * traveltime stay in registers for the whole launch.
+ *
+ * Traces stream through LDS in trace order.  Blocks of NT traces are filtered
+ * to those whose CMP can reach the tile (ordered compaction into a list);
+ * the aperture and slab gates of the next 64 of the list are evaluated
+ * lane-parallel (lane j = trace j), and the passing ones are walked in order.
+ * Rows are staged C at a time into a ring of three such chunks by loads that
+ * write LDS directly: chunk q + 1 is in flight while chunk q is used, so the
+ * loads' latency is hidden, no register holds a staged row, and one barrier
+ * per chunk separates the two (the third slot keeps the previous chunk for
+ * the re-summation below).
  *
  * Traveltime index, two variants:
  * - exact (the FP32 reference path, and the Kahan modes unless FASTIDX): the
- *   reference's index, resolved speculatively.  The fast form's floor(q) is
- *   used at once; a sample whose q lies within the form's error bound of an
+ *   reference's index, resolved speculatively.  The fast form's floor is
+ *   used at once; a sample whose p ns lies within the form's error bound of an
  *   integer (and is not past the trace for certain) is added with that index
- *   and queued in LDS with the running sum before the add (one per lane and
- *   batch; a lane's further ambiguous samples take the inline exact path).
- *   At the end of the staged batch one wave-wide pass computes the reference
- *   index of every lane's queued sample together (the exact arithmetic used
- *   to run for the whole wave per ambiguous lane and slot); where it differs
- *   from the fast one (a few percent of them) the sample's running sum is
- *   rebuilt from the saved value through the batch's later traces in order,
- *   so every sample receives its additions in the reference's order and the
- *   result equals the inline exact path's bit for bit.  v^2 of the column's
- *   samples stays in LDS for the reference arithmetic.
+ *   and remembered with the running sum before the add (one per lane and
+ *   window of two chunks; a lane's further ambiguous samples take the inline
+ *   exact path).  At the end of the window one wave-wide pass computes the
+ *   reference index of every lane's remembered sample together; where it
+ *   differs from the fast one (a few percent of them) the sample's running sum
+ *   is rebuilt from the saved value through the window's later traces in
+ *   order, so every sample receives its additions in the reference's order
+ *   and the result equals the inline exact path's bit for bit.
  * - FASTIDX: T = floor(min(q, ns)) of the fast form alone (CLOSED and 16-bit
  *   modes, whose contract is an error bound against FP64): no ambiguity
- *   test; fold is summed from a row V[T] = (T < ns) staged once in LDS (an
- *   address add and a float add per sample instead of a compare and a carry
- *   add, both quarter-rate on gfx950).
- * q is clamped at ns, so in the exact variants a sample at or past the end of
- * the trace lands on an integer and takes the rare branch, where the samples
- * that do not count towards fold are counted: the common path has no compare
- * for fold.  Every variant fits 128 VGPRs (4 waves per SIMD, two workgroups
- * per CU, one staging while the other computes; the Kahan exact variant
- * spills a few 64-bit addresses that are reloaded once per chunk of 512
- * traces). */
-template <int K, int W, int B, bool KAHAN, bool FASTIDX>
-__global__ void __launch_bounds__(8 * KTM_WAVE) __attribute__((amdgpu_waves_per_eu(4, 4)))
+ *   test.
+ * A sample past the trace reads the zero F[ns] and does not count for fold.
+ * With the gates each lane bounds, for its trace and every slot of the wave,
+ * the largest q (the traveltime at the slot's largest constants): slots before
+ * the first whose bound reaches the end of the trace need no count (and,
+ * relaxed index, no clamp), and the bound over all slots sets the trace's
+ * ambiguity threshold.
+ * Bound by VALU issue.  In this mixed stream every VALU instruction takes a
+ * SIMD about 4 cycles and a square root 8 (the doubled FMA and add rate of a
+ * pure stream does not appear: 17.3 instructions per 64 contributions of
+ * which 2.07 roots took 79 cycles), so what counts is their number: two FMA, two
+ * roots, the clamped sum, three for floor and distance, the LDS address, the
+ * add into the image, and 2/3 of an instruction for the test (14.5 in all with
+ * the gates, the staging and the ambiguous samples).  Against rows staged
+ * through registers between two barriers and every sample past the trace on
+ * the rare path: 16,000 traces x 1500 samples into 400 x 400 columns 295 ->
+ * 253 ms, 20,000 BF16-stored x 1251 into 150 x 150 222 -> 187 ms, the
+ * 40-shot line 3.75 -> 2.85 ms, 12 classes x 2503 samples x 500 columns 10.9 ->
+ * 6.75 ms.  12 waves of K = 8 (six per SIMD) measured the same as 8 of K = 12
+ * with 1500 samples, 16 waves in one workgroup 15 % slower (all of a CU's waves
+ * at one barrier); slot groups of 2, 4 and 6 within 3 % of 3. */
+template <int K, int W, int NW, int C, int EU, bool KAHAN, bool FASTIDX>
+__global__ void __launch_bounds__(NW * KTM_WAVE) __attribute__((amdgpu_waves_per_eu(EU, EU)))
 k_migrate(const MigArgs a)
 {
-    constexpr int NCOL = 8 / W;             /* image columns per workgroup */
-    constexpr int NW = NCOL * W;            /* waves per workgroup (8) */
+    constexpr int NCOL = NW / W;            /* image columns per workgroup */
     constexpr int NT = NW * KTM_WAVE;
+    constexpr int WPR = NW / C;             /* waves that stage one row of a chunk */
     constexpr bool SPEC = !FASTIDX;
-    static_assert(B <= 16 && K <= 16, "queue items pack the slot and the trace in 4 bits each");
+    constexpr int G = K % 3 ? 4 : 3;        /* slots side by side */
+    static_assert(NW % C == 0 && 2 * C <= 16 && K < 16 && K % G == 0 && KTM_WAVE % (2 * C) == 0,
+                  "remembered samples pack the slot and the trace in 4 bits each");
     extern __shared__ float4 lds4[];
     const int ldl = (int)a.row;             /* LDS row = prepared row (floats) */
-    float *sF = reinterpret_cast<float *>(lds4);            /* [B][ldl] */
-    float *sG = sF + B * ldl;                               /* [B][8]   */
-    int *sSel = reinterpret_cast<int *>(sG + B * 8);        /* [NT]     */
-    int *sCnt = sSel + NT;                                  /* [NW]     */
-    /* exact index: v^2 per sample [NCOL][W*K*64], then the speculation
-     * queue [NW][KTM_SPEC_Q][64] of uint2 (running sum before the add,
-     * slot | trace << 4 | index << 8 | mismatch << 31: the fast index when
-     * queued, the reference's once resolved); fast index: V[T], [ldl] */
-    float *sV2 = reinterpret_cast<float *>(sCnt + NW);
-    uint2 *sQ = reinterpret_cast<uint2 *>(sV2 + NCOL * (W * K * KTM_WAVE));
+    float *sF = reinterpret_cast<float *>(lds4);            /* [3][C][ldl]  */
+    float2 *sMax = reinterpret_cast<float2 *>(sF + 3 * C * ldl);   /* [NW][K] largest rs, tq */
+    int *sSel = reinterpret_cast<int *>(sMax + NW * K);     /* [64 + C + NT] */
+    int *sCnt = sSel + KTM_WAVE + C + NT;                   /* [NW]     */
 
-    const int tid = threadIdx.x, lane = tid & (KTM_WAVE - 1), wv = tid / KTM_WAVE;
+    const int tid = threadIdx.x, lane = tid & (KTM_WAVE - 1);
+    const int wv = __builtin_amdgcn_readfirstlane(tid / KTM_WAVE);
     /* XCD-aware tile order: consecutive workgroup ids go to different XCDs.
      * Each XCD takes runs of a.run consecutive tiles (a row of tiles in 3-D:
      * neighbouring columns share traces in its L2) and the runs are dealt
@@ -736,7 +795,9 @@ k_migrate(const MigArgs a)
     const float scx = a.slab_cx[job], scy = a.slab_cy[job];
     const float sthr = a.slab_x2thr[job];
     const int ns = a.ns;
-    const float nsf = (float)ns;
+    const float nsf = (float)ns, nsh = nsf + 0.5f;
+    /* M - past is 0 or less for an index below ns, 1 for ns */
+    const float past = 8388608.0f + (nsf - 1.0f);
 
     /* conservative tile test: the CMP must be within aperture of some
      * column of the tile (exact per-column gates follow) */
@@ -748,42 +809,39 @@ k_migrate(const MigArgs a)
     const float reach = a.aperture * 1.0001f + sqrtf(hx * hx + hy * hy) + 1.0f;
     const float reach2 = reach * reach;
 
-    /* exact variants: v^2 of this column's samples in LDS for the exact path */
-    float *sV2c = sV2 + cw * (W * K * KTM_WAVE);
-    if (FASTIDX) {
-        for (int c = tid; c < ldl; c += NT) sV2[c] = c < ns ? 1.0f : 0.0f;
-    }
-    uint2 *sQw = sQ + wv * (KTM_SPEC_Q * KTM_WAVE);
     const int64_t pix = (((int64_t)Xc * a.nyp + Yc) * a.nh + h) * ns;
-    const int64_t vbase = ((int64_t)a.velx[Xc] * a.nvel_xl + a.vely[Yc]) * a.nsm;
+    const float *vel = a.vel2 + ((int64_t)a.velx[Xc] * a.nvel_xl + a.vely[Yc]) * a.nsm;
     float rs[K], tq[K], acc[K], cmp[K];
-    int cnt[FASTIDX ? 1 : K];               /* passing traces with T >= ns, per slot */
-    float vcnt[FASTIDX ? K : 1];            /* passing traces with T < ns, per slot */
+    float cnt[K];                           /* passing traces with T >= ns, per slot */
 #pragma unroll
     for (int k = 0; k < K; ++k) {
         const int tl = seg * K * KTM_WAVE + k * KTM_WAVE + lane;
-        if (!FASTIDX) cnt[FASTIDX ? 0 : k] = 0;
-        if (FASTIDX) vcnt[FASTIDX ? k : 0] = 0.0f;
+        cnt[k] = 0.0f;
         cmp[k] = 0.0f;
         if (tl < ns) {
-            const float v2 = a.vel2[vbase + a.t1[tl]];
-            if (!FASTIDX) sV2c[tl] = v2;
-            rs[k] = fast_rs(v2, a.dt);
-            tq[k] = fast_tq(tl);
+            const float v2 = vel[a.t1[tl]];
+            rs[k] = FASTIDX ? fast_rs(v2, a.dt) : fast_rsn(v2, a.dt, nsh);
+            tq[k] = FASTIDX ? fast_tq(tl) : fast_tqn(tl, nsh);
             acc[k] = col_ok && part == 0 ? a.km[pix + tl] : 0.0f;
             if (KAHAN && col_ok && part == 0) cmp[k] = a.comp[pix + tl];
         } else {
-            if (!FASTIDX) sV2c[tl] = 1.0f;
             /* padding lane: q = 0.5, never flagged by the ambiguity test; it
              * reads F[0] (and V[0]) into values that are not stored */
             rs[k] = 0.0f;
-            tq[k] = 0.0625f;
+            tq[k] = FASTIDX ? 0.0625f : 0.0625f / (nsh * nsh);
             acc[k] = 0.0f;
         }
+        /* the slot's largest constants over the wave */
+        float mr = rs[k], mt = tq[k];
+        for (int d = KTM_WAVE / 2; d >= 1; d >>= 1) {
+            mr = fmaxf(mr, __shfl_xor(mr, d));
+            mt = fmaxf(mt, __shfl_xor(mt, d));
+        }
+        if (lane == 0) sMax[wv * K + k] = make_float2(mr, mt);
     }
 
     /* Kahan variants: the taps are summed onto y = -c in plain FP32 over
-     * KTM_KAHAN_FOLD staged batches (at most KTM_KAHAN_FOLD * B terms, error
+     * KTM_KAHAN_FOLD windows (at most KTM_KAHAN_FOLD * 2C terms, error
      * <= (terms - 1) u times their magnitudes) and added to the image with one
      * compensated step, which keeps the compensated error bound of order
      * u * sum |f| at a fraction of the per-tap cost.  Plain variants add
@@ -801,245 +859,266 @@ k_migrate(const MigArgs a)
             acc[k] = s;
         }
     };
-    /* the squared source and receiver distances of staged trace j from this
-     * column, as the gate evaluation forms them */
-    auto staged_dist = [&](int j, float &dIS2, float &dIR2) __attribute__((always_inline)) {
-        const float4 g0 = reinterpret_cast<const float4 *>(sG + j * 8)[0];
-        const float ax = IX - g0.x, ay = IY - g0.y, bx = IX - g0.z, by = IY - g0.w;
-        dIS2 = ax * ax + ay * ay;
-        dIR2 = bx * bx + by * by;
-    };
 
     uint32_t npass = 0;
-    const int n4 = ldl / 4;
-    const int64_t cbeg = KAHAN ? (int64_t)part * NT : 0;
     const int64_t cstep = KAHAN ? a.nparts * NT : NT;
-    const int64_t cend = a.ntr;
-    for (int64_t c0 = cbeg; c0 < cend; c0 += cstep) {
-        /* ---- select the traces of this chunk that can reach the tile, in order ---- */
-        const int64_t i = c0 + tid;
-        bool pred = false;
-        if (i < cend) {
-            const ktm_trace_geom g = a.geom[i];
-            const float dx = g.cmpx - ccx, dy = g.cmpy - ccy;
-            pred = g.off == h && dx * dx + dy * dy <= reach2;
-        }
-        const uint64_t m = __ballot(pred);
-        const int pre = __popcll(m & ((1ull << lane) - 1ull));
-        if (lane == 0) sCnt[wv] = __popcll(m);
-        __syncthreads();
-        int base = 0, total = 0;
-#pragma unroll
-        for (int q = 0; q < NW; ++q) {
-            const int v = sCnt[q];
-            base += q < wv ? v : 0;
-            total += v;
-        }
-        if (pred) sSel[base + pre] = tid;
-        __syncthreads();
-
-        for (int b0 = 0; b0 < total; b0 += B) {
-            const int nb = min(B, total - b0);
-            /* ---- stage nb traces (filtered samples + geometry) into LDS ---- */
-            for (int j = 0; j < nb; ++j) {
-                const int64_t ti = c0 + sSel[b0 + j];
-                const float4 *src = reinterpret_cast<const float4 *>(a.prep + ti * a.row);
-                for (int c = tid; c < n4; c += NT)
-                    reinterpret_cast<float4 *>(sF + j * ldl)[c] = src[c];
+    int64_t c0 = KAHAN ? (int64_t)part * NT : 0;
+    /* the list of traces that can reach the tile, in order: sSel[head, n) */
+    int head = 0, n = 0;
+    auto refill = [&]() __attribute__((always_inline)) {
+        while (n - head < KTM_WAVE + C && c0 < a.ntr) {
+            if (head) {                          /* the rest to the front */
+                const int left = n - head;       /* < 64 + C <= NT */
+                const int v = tid < left ? sSel[head + tid] : 0;
+                __syncthreads();
+                if (tid < left) sSel[tid] = v;
+                head = 0;
+                n = left;
             }
-            if (tid < nb * 2) {
-                const int j = tid >> 1, half = tid & 1;
-                const int64_t ti = c0 + sSel[b0 + j];
-                reinterpret_cast<float4 *>(sG + j * 8)[half] =
-                    reinterpret_cast<const float4 *>(a.geom + ti)[half];
+            const int64_t i = c0 + tid;
+            bool pred = false;
+            if (i < a.ntr) {
+                const ktm_trace_geom g = a.geom[i];
+                const float dx = g.cmpx - ccx, dy = g.cmpy - ccy;
+                pred = g.off == h && dx * dx + dy * dy <= reach2;
             }
+            const uint64_t m = __ballot(pred);
+            const int pre = __popcll(m & ((1ull << lane) - 1ull));
+            if (lane == 0) sCnt[wv] = __popcll(m);
             __syncthreads();
+            int base = n, total = 0;
+#pragma unroll
+            for (int q = 0; q < NW; ++q) {
+                const int v = sCnt[q];
+                base += q < wv ? v : 0;
+                total += v;
+            }
+            if (pred) sSel[base + pre] = (int)i;
+            n += __builtin_amdgcn_readfirstlane(total);
+            c0 += cstep;
+            __syncthreads();
+        }
+    };
+    /* start the loads of this wave's share of a chunk, part of the row of
+     * trace ti, into ring slot s: WPR waves per row, 1 KiB pieces, lane l's 16
+     * bytes to the piece's base + 16 l */
+    const int rowbytes = ldl * (int)sizeof(float), jrow = wv / WPR;
+    auto issue = [&](int ti, int s) __attribute__((always_inline)) {
+        const char *src = reinterpret_cast<const char *>(a.prep + (int64_t)ti * a.row);
+        char *dst = reinterpret_cast<char *>(sF + (s * C + jrow) * ldl);
+        if (a.align16) {
+            for (int o = (wv % WPR) * 1024; o < rowbytes; o += WPR * 1024) {
+                const uint32_t lo = (uint32_t)lane * 16u;
+                if (o + 1024 <= rowbytes || o + (int)lo < rowbytes)
+                    __builtin_amdgcn_global_load_lds((global_void *)(src + o + lo),
+                                                     (lds_void *)(dst + o), 16, 0, 0);
+            }
+        } else {                            /* rows that start at any float */
+            for (int o = (wv % WPR) * 256; o < rowbytes; o += WPR * 256) {
+                const uint32_t lo = (uint32_t)lane * 4u;
+                if (o + (int)lo < rowbytes)
+                    __builtin_amdgcn_global_load_lds((global_void *)(src + o + lo),
+                                                     (lds_void *)(dst + o), 4, 0, 0);
+            }
+        }
+    };
 
-            if (col_ok) {
-                /* gates and distances of Kirchhoff.c:1334-1354 for every staged
-                 * trace at once (lane j = trace j), on squared distances with
-                 * the exact thresholds of ktm_gate_threshold */
-                float g_is = 0.0f, g_ir = 0.0f;
-                bool gp = false;
-                if (lane < nb) {
-                    staged_dist(lane, g_is, g_ir);
-                    const float4 g1 = reinterpret_cast<const float4 *>(sG + lane * 8)[1];
-                    const float cx = IX - g1.x, cy = IY - g1.y;
-                    const float ex = scx - g1.x, ey = scy - g1.y;
-                    gp = ex * ex + ey * ey < sthr && cx * cx + cy * cy < a.ap_x2thr;
-                }
-                const uint64_t pm_batch = __ballot(gp);
-                uint64_t pm = pm_batch;
-                npass += __popcll(pm);
-                int qn = 0;                         /* queued samples of this lane (plain) */
-                /* Hot loop, Kirchhoff.c:1374-1399: the tap F[T] of slot k for
-                 * one trace (and, fast index, V[T] for fold). */
-                auto tap = [&](int k, int j, float dIS2, float dIR2, const float *Fr) __attribute__((always_inline)) {
-                    const float q = fast_qs(dIS2, dIR2, rs[k], tq[k]);
-                    const float qc = clamp_ns(q, nsf);
-                    int T = fast_T(qc);
+    refill();
+    int slot = 0;                               /* ring slot of the current chunk */
+    if (head + jrow < n) issue(__builtin_amdgcn_readfirstlane(sSel[head + jrow]), 0);
+    while (n > head) {
+        /* gates and distances of Kirchhoff.c:1334-1354 for the next 64 traces
+         * at once (lane j = trace j), on squared distances with the exact
+         * thresholds of ktm_gate_threshold */
+        const int nb = min(KTM_WAVE, n - head);
+        float g_is = 0.0f, g_ir = 0.0f;
+        int g_ti = 0;
+        bool gp = false;
+        if (lane < nb) {
+            g_ti = sSel[head + lane];
+            const float4 *gg = reinterpret_cast<const float4 *>(a.geom + g_ti);
+            const float4 g0 = gg[0], g1 = gg[1];
+            const float ax = IX - g0.x, ay = IY - g0.y, bx = IX - g0.z, by = IY - g0.w;
+            g_is = ax * ax + ay * ay;
+            g_ir = bx * bx + by * by;
+            const float cx = IX - g1.x, cy = IY - g1.y;
+            const float ex = scx - g1.x, ey = scy - g1.y;
+            gp = ex * ex + ey * ey < sthr && cx * cx + cy * cy < a.ap_x2thr;
+        }
+        const uint64_t pm = col_ok ? __ballot(gp) : 0ull;
+        npass += __popcll(pm);
+        /* the slots that cannot reach the end of lane j's trace, the first
+         * kend: their largest q (FMA and v_sqrt_f32 to 1 ulp each, so 1e-5
+         * covers their rounding) is below ns - 1; and the trace's ambiguity
+         * threshold, kend in its low 4 bits (which lower it by < 1e-6, taken
+         * off first) */
+        int kend = K;
+        float qm = 0.0f;
+#pragma unroll
+        for (int k = K - 1; k >= 0; --k) {
+            const float2 mx = sMax[wv * K + k];
+            const float q = FASTIDX ? fast_qs(g_is, g_ir, mx.x, mx.y)
+                                    : nsh * fast_p(g_is, g_ir, mx.x, mx.y);
+            kend = q * 1.00001f < nsf - 1.0f ? kend : k;
+            qm = fmaxf(qm, q);
+        }
+        const uint32_t g_lim =
+            (__float_as_uint(ambiguous_from(qm * 1.00001f) - 1.0e-6f) & ~15u) | (uint32_t)kend;
+        /* the lane's remembered sample of the window: slot | trace << 4 |
+         * index << 8 (-1: none) and the sum before it */
+        int qi = -1;
+        float qs = 0.0f;
+        for (int q = 0; q * C < nb; ++q) {
+            /* chunk q has arrived and every wave is done with chunk q - 1,
+             * so with the slot that chunk q + 1 goes to */
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+            const int nslot = slot == 2 ? 0 : slot + 1;
+            const int jn = (q + 1) * C + jrow;      /* this wave's row of chunk q + 1 */
+            if (head + jn < n)
+                issue(jn < KTM_WAVE ? __builtin_amdgcn_readlane(g_ti, jn)
+                                    : __builtin_amdgcn_readfirstlane(sSel[head + jn]), nslot);
+
+            uint32_t pmc = (uint32_t)(pm >> (q * C)) & ((1u << C) - 1u);
+            const float *ring = sF + slot * C * ldl;
+            while (pmc) {
+                const int j = __builtin_ctz(pmc);    /* traces in order */
+                pmc &= pmc - 1u;
+                const float dIS2 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(g_is), q * C + j));
+                const float dIR2 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(g_ir), q * C + j));
+                const uint32_t lim = (uint32_t)__builtin_amdgcn_readlane((int)g_lim, q * C + j);
+                const int kend = (int)(lim & 15u);
+                const float *Fr = ring + j * ldl;
+                /* Hot loop, Kirchhoff.c:1374-1399: G slots at a time, their
+                 * chains side by side */
+                const uint32_t fr = (uint32_t)(uintptr_t)(lds_float *)Fr;
+#pragma unroll
+                for (int k = 0; k < K; k += G) {
+                    uint32_t ad[G];
                     if (FASTIDX) {
-                        /* V sits (sV2 - Fr) floats from F: one address add */
-                        const float *Fp = Fr + T;
-                        vcnt[FASTIDX ? k : 0] += Fp[sV2 - Fr];
-                        return *Fp;
-                    }
-                    constexpr float EPS = KTM_FAST_EPS_S;
-                    if (fast_ambiguous(qc, EPS)) {
-                        if (q - nsf >= __builtin_fmaf(q, EPS, EPS)) {
-                            T = ns;   /* Q >= ns as well: past the trace */
-                            cnt[FASTIDX ? 0 : k] += 1;
-                        } else if (SPEC && qn < KTM_SPEC_Q) {
-                            /* speculate: floor(q) now, the reference index at
-                             * the end of the batch */
-                            sQw[qn * KTM_WAVE + lane] = make_uint2(
-                                __float_as_uint(KAHAN ? y[KAHAN ? k : 0] : acc[k]),
-                                (uint32_t)(k | (j << 4) | (T << 8)));
-                            ++qn;
-                        } else {
-                            const int tl = seg * K * KTM_WAVE + k * KTM_WAVE + lane;
-                            const float v2 = sV2c[tl];
-                            T = exact_T(dIS2, dIR2, a.t2[tl], v2, 1.0f / v2, a.dt, a.rdt, ns);
-                            cnt[FASTIDX ? 0 : k] += T >= ns ? 1 : 0;
-                        }
-                    }
-                    return Fr[T];
-                };
-                /* the rare path of tap() for slot k: ambiguous or past the trace */
-                auto rare = [&](int k, int j, float q, float dIS2, float dIR2, int &T) __attribute__((always_inline)) {
-                    constexpr float EPS = KTM_FAST_EPS_S;
-                    if (q - nsf >= __builtin_fmaf(q, EPS, EPS)) {
-                        T = ns;   /* Q >= ns as well: past the trace */
-                        cnt[FASTIDX ? 0 : k] += 1;
-                    } else if (SPEC && qn < KTM_SPEC_Q) {
-                        sQw[qn * KTM_WAVE + lane] = make_uint2(
-                            __float_as_uint(KAHAN ? y[KAHAN ? k : 0] : acc[k]),
-                            (uint32_t)(k | (j << 4) | (T << 8)));
-                        ++qn;
-                    } else {
-                        const int tl = seg * K * KTM_WAVE + k * KTM_WAVE + lane;
-                        const float v2 = sV2c[tl];
-                        T = exact_T(dIS2, dIR2, a.t2[tl], v2, 1.0f / v2, a.dt, a.rdt, ns);
-                        cnt[FASTIDX ? 0 : k] += T >= ns ? 1 : 0;
-                    }
-                };
-                while (pm) {
-                    const int j = __builtin_ctzll(pm);   /* traces in order */
-                    pm &= pm - 1ull;
-                    const float dIS2 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(g_is), j));
-                    const float dIR2 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(g_ir), j));
-                    const float *Fr = sF + j * ldl;
-                    constexpr int G = K % KTM_SLOT_GROUP == 0 ? KTM_SLOT_GROUP : 2;
-                    if (FASTIDX || (K % G)) {
+                        float qg[G];
 #pragma unroll
-                        for (int k = 0; k < K; ++k) {
-                            const float f = tap(k, j, dIS2, dIR2, Fr);
-                            if (KAHAN) y[KAHAN ? k : 0] = y[KAHAN ? k : 0] + f;
-                            else acc[k] = acc[k] + f;
-                        }
-                    } else {
-                        /* exact index, G slots per branch: their chains run
-                         * side by side, one test guards their rare paths */
-#pragma unroll
-                        for (int k = 0; k < K; k += G) {
-                            constexpr float EPS = KTM_FAST_EPS_S;
-                            float qg[G];
-                            int Tg[G];
-                            bool ag[G], any = false;
+                        for (int i = 0; i < G; ++i) qg[i] = fast_qs(dIS2, dIR2, rs[k + i], tq[k + i]);
+                        if (k + G > kend) {
 #pragma unroll
                             for (int i = 0; i < G; ++i) {
-                                qg[i] = fast_qs(dIS2, dIR2, rs[k + i], tq[k + i]);
-                                const float qc = clamp_ns(qg[i], nsf);
-                                Tg[i] = fast_T(qc);
-                                ag[i] = fast_ambiguous(qc, EPS);
-                                any = any || ag[i];
+                                cnt[k + i] += qg[i] >= nsf ? 1.0f : 0.0f;
+                                qg[i] = clamp_ns(qg[i], nsf);
                             }
-                            if (any) {
+                        }
 #pragma unroll
-                                for (int i = 0; i < G; ++i)
-                                    if (ag[i]) rare(k + i, j, qg[i], dIS2, dIR2, Tg[i]);
-                            }
+                        for (int i = 0; i < G; ++i) ad[i] = ((uint32_t)fast_T(qg[i]) << 2) + fr;
+                    } else {
+                        float pg[G];
+                        FloorP fg[G];
+                        float far = 0.0f;       /* largest distance from the middle */
+#pragma unroll
+                        for (int i = 0; i < G; ++i) {
+                            pg[i] = fast_p(dIS2, dIR2, rs[k + i], tq[k + i]);
+                            fg[i] = floor_p(pg[i], nsh, k + i == 0);
+                            ad[i] = (__float_as_uint(fg[i].M) << 2) + (fr - 4u * KTM_FLOOR_BITS);
+                            far = i ? fmaxf(far, fabsf(fg[i].dev)) : fabsf(fg[i].dev);
+                        }
+                        if (k + G > kend) {
+                            /* past the trace, 0 or 1 */
+#pragma unroll
+                            for (int i = 0; i < G; ++i)
+                                cnt[k + i] += __builtin_amdgcn_fmed3f(fg[i].M - past, 0.0f, 1.0f);
+                        }
+                        const float thr = __uint_as_float(lim);
+                        if (far >= thr) {
+                            const int jw = (q & 1) * C + j;
 #pragma unroll
                             for (int i = 0; i < G; ++i) {
-                                const float f = Fr[Tg[i]];
-                                if (KAHAN) y[KAHAN ? k + i : 0] = y[KAHAN ? k + i : 0] + f;
-                                else acc[k + i] = acc[k + i] + f;
+                                if (!(fabsf(fg[i].dev) >= thr)) continue;
+                                const int kk = k + i;
+                                const int T = floor_T(fg[i]);
+                                if (qi < 0) {
+                                    /* speculate: the fast index now, the
+                                     * reference's at the end of the window */
+                                    qi = kk | (jw << 4) | (T << 8);
+                                    qs = KAHAN ? y[KAHAN ? kk : 0] : acc[kk];
+                                    continue;
+                                }
+                                const int tl = seg * K * KTM_WAVE + kk * KTM_WAVE + lane;
+                                const float v2 = vel[a.t1[tl]];
+                                const int Te = exact_T(dIS2, dIR2, a.t2[tl], v2, 1.0f / v2, a.dt, a.rdt, ns);
+                                cnt[kk] += (Te >= ns ? 1.0f : 0.0f) - (T >= ns ? 1.0f : 0.0f);
+                                ad[i] = ((uint32_t)Te << 2) + fr;
                             }
                         }
                     }
-                }
-                if (SPEC && __ballot(qn > 0)) {
-                    /* ---- resolve the queued samples: one pass per queue
-                     * depth, every lane's item of that depth together ---- */
-                    bool redo = false;
-                    for (int r = 0; r < KTM_SPEC_Q; ++r) {
-                        if (!__ballot(qn > r)) break;
-                        if (qn > r) {
-                            uint2 e = sQw[r * KTM_WAVE + lane];
-                            const int k = (int)(e.y & 15u), j = (int)((e.y >> 4) & 15u);
-                            const int tl = seg * K * KTM_WAVE + k * KTM_WAVE + lane;
-                            const int Tf = (int)((e.y >> 8) & 0x7fffu);
-                            float dIS2, dIR2;
-                            staged_dist(j, dIS2, dIR2);
-                            const float v2 = sV2c[tl];
-                            const int Te = exact_T(dIS2, dIR2, a.t2[tl], v2, 1.0f / v2, a.dt,
-                                                   a.rdt, ns);
-                            if (Te >= ns) {
 #pragma unroll
-                                for (int kk = 0; kk < K; ++kk)
-                                    if (kk == k) cnt[FASTIDX ? 0 : kk] += 1;
-                            }
-                            e.y = (e.y & 0xffu) | ((uint32_t)Te << 8) |
-                                  (Te != Tf ? 0x80000000u : 0u);
-                            sQw[r * KTM_WAVE + lane] = e;
-                            redo = redo || Te != Tf;
-                        }
+                    for (int i = 0; i < G; ++i) {
+                        const float f = *(lds_float *)(uintptr_t)ad[i];
+                        if (KAHAN) y[KAHAN ? k + i : 0] = y[KAHAN ? k + i : 0] + f;
+                        else acc[k + i] = acc[k + i] + f;
                     }
-                    /* ---- rebuild the sums whose queued index was wrong: from
-                     * the sum before the earliest wrong one, through the
-                     * batch's later passing traces in order (rare) ---- */
-                    if (__ballot(redo) && redo) {
-                        uint32_t done = 0;              /* slots rebuilt */
-                        for (int r = 0; r < qn; ++r) {
-                            const uint2 e = sQw[r * KTM_WAVE + lane];
-                            const int k = (int)(e.y & 15u), j = (int)((e.y >> 4) & 15u);
-                            if (!(e.y & 0x80000000u) || (done >> k & 1u)) continue;
-                            done |= 1u << k;
-                            const int tl = seg * K * KTM_WAVE + k * KTM_WAVE + lane;
-                            const float v2 = sV2c[tl];
-                            float rsk = 0.0f;
-#pragma unroll
-                            for (int kk = 0; kk < K; ++kk)
-                                if (kk == k) rsk = rs[kk];
-                            const float tqk = fast_tq(tl), t2k = a.t2[tl];
-                            float s = __uint_as_float(e.x) +
-                                      sF[j * ldl + (int)((e.y >> 8) & 0x7fffu)];
-                            uint64_t later = pm_batch & ~((2ull << j) - 1ull);
-                            while (later) {
-                                const int jj = __builtin_ctzll(later);
-                                later &= later - 1ull;
-                                float dIS2, dIR2;
-                                staged_dist(jj, dIS2, dIR2);
-                                const int T = reference_T(dIS2, dIR2, rsk, tqk, t2k, v2, a.dt,
-                                                          a.rdt, ns);
-                                s = s + sF[jj * ldl + T];
-                            }
-#pragma unroll
-                            for (int kk = 0; kk < K; ++kk) {
-                                if (kk != k) continue;
-                                if (KAHAN) y[KAHAN ? kk : 0] = s;
-                                else acc[kk] = s;
-                            }
-                        }
-                    }
-                }
-                if (KAHAN && ++nfold == KTM_KAHAN_FOLD) {
-                    nfold = 0;
-                    fold_y();
                 }
             }
-            __syncthreads();
+            const bool wend = (q & 1) || (q + 1) * C >= nb;     /* end of the window */
+            if (SPEC && wend && __ballot(qi >= 0)) {
+                /* ---- the reference index of every lane's remembered sample ---- */
+                const int w0 = (q & ~1) * C;         /* the window's first trace */
+                /* row of the window's trace jw: the previous slot holds the
+                 * first chunk when the current one is the second */
+                const int pslot = slot == 0 ? 2 : slot - 1;
+                auto row_of = [&](int jw) __attribute__((always_inline)) {
+                    const int s = (q & 1) && jw < C ? pslot : slot;
+                    return sF + (s * C + (jw & (C - 1))) * ldl;
+                };
+                const int jw = (qi >> 4) & 15, k = qi & 15;
+                const float dIS2 = __shfl(g_is, w0 + (qi >= 0 ? jw : 0));
+                const float dIR2 = __shfl(g_ir, w0 + (qi >= 0 ? jw : 0));
+                const int tl = seg * K * KTM_WAVE + k * KTM_WAVE + lane;
+                int Te = 0;
+                float v2 = 1.0f, t2 = 0.0f;
+                bool redo = false;
+                if (qi >= 0) {
+                    v2 = vel[a.t1[tl]];
+                    t2 = a.t2[tl];
+                    Te = exact_T(dIS2, dIR2, t2, v2, 1.0f / v2, a.dt, a.rdt, ns);
+                    redo = Te != (qi >> 8);
+                }
+                if (__ballot(redo)) {
+                    /* ---- rebuild the sums whose index was wrong: from the
+                     * sum before it through the window's later passing
+                     * traces in order (rare) ---- */
+                    float s = 0.0f, rsk = 0.0f;
+                    if (redo) s = qs + row_of(jw)[Te];
+#pragma unroll
+                    for (int kk = 0; kk < K; ++kk)
+                        if (kk == k) rsk = rs[kk];
+                    uint32_t later = (uint32_t)(pm >> w0) & ((1u << (2 * C)) - 1u);
+                    while (later) {
+                        const int jj = __builtin_ctz(later);
+                        later &= later - 1u;
+                        const float es = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(g_is), w0 + jj));
+                        const float er = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(g_ir), w0 + jj));
+                        const float *Fr = row_of(jj);
+                        if (redo && jj > jw)
+                            s = s + Fr[reference_T(es, er, rsk, fast_tqn(tl, nsh), t2, v2, a.dt,
+                                                   a.rdt, ns, tl == 0)];
+                    }
+#pragma unroll
+                    for (int kk = 0; kk < K; ++kk) {
+                        if (!redo || kk != k) continue;
+                        if (KAHAN) y[KAHAN ? kk : 0] = s;
+                        else acc[kk] = s;
+                        cnt[kk] +=
+                            (Te >= ns ? 1.0f : 0.0f) - ((qi >> 8) >= ns ? 1.0f : 0.0f);
+                    }
+                }
+                qi = -1;
+            }
+            if (KAHAN && wend && ++nfold == KTM_KAHAN_FOLD) {
+                nfold = 0;
+                fold_y();
+            }
+            slot = nslot;
         }
+        head += nb;
+        refill();
     }
     if (KAHAN && nfold) fold_y();
 
@@ -1053,8 +1132,7 @@ k_migrate(const MigArgs a)
             const int t = seg * K * KTM_WAVE + k * KTM_WAVE + lane;
             if (t < ns) {
                 pk[rpix + t] = acc[k];
-                pk[a.part_n + rpix + t] = FASTIDX ? vcnt[FASTIDX ? k : 0]
-                                                  : (float)((int)npass - cnt[FASTIDX ? 0 : k]);
+                pk[a.part_n + rpix + t] = (float)npass - cnt[k];
                 pk[2 * a.part_n + rpix + t] = -y[KAHAN ? k : 0];
             }
         }
@@ -1068,9 +1146,7 @@ k_migrate(const MigArgs a)
                 a.km[pix + t] = acc[k];
                 /* fold adds the passing traces whose sample was inside the
                  * trace (Kirchhoff.c:1387-1396) */
-                a.fold[pix + t] = a.fold[pix + t] +
-                                  (FASTIDX ? vcnt[FASTIDX ? k : 0]
-                                           : (float)((int)npass - cnt[FASTIDX ? 0 : k]));
+                a.fold[pix + t] = a.fold[pix + t] + ((float)npass - cnt[k]);
                 if (KAHAN) a.comp[pix + t] = -y[KAHAN ? k : 0];
             }
         }
@@ -1311,14 +1387,12 @@ __global__ void k_selftest_traveltime(const float4 *__restrict__ in, int64_t n, 
     const float4 in4 = in[i];
     const int t = (int)in4.z;
     const float4 v = make_float4(in4.x, in4.y, (float)(0.25 * t * t * dt * dt), in4.w);
-    const float r = 1.0f / v.w, rdt = 1.0f / dt;
+    const float rdt = 1.0f / dt;
     const float q = fast_qs(v.x, v.y, fast_rs(v.w, dt), fast_tq(t));
     /* the decision procedure of k_migrate */
-    const float nsf = (float)ns, qc = fminf(q, nsf);
-    int T = fast_T(qc);
-    if (fast_ambiguous(qc, KTM_FAST_EPS_S))
-        T = q - nsf >= __builtin_fmaf(q, KTM_FAST_EPS_S, KTM_FAST_EPS_S)
-                ? ns : exact_T(v.x, v.y, v.z, v.w, r, dt, rdt, ns);
+    const float nsf = (float)ns, nsh = nsf + 0.5f;
+    const int T = reference_T(v.x, v.y, fast_rsn(v.w, dt, nsh), fast_tqn(t, nsh), v.z, v.w, dt, rdt,
+                              ns, t == 0);
     /* the reference computed independently of exact_T: the compiler's
      * correctly rounded division and double square root */
     const float s1 = v.z + v.x / v.w, s2 = v.z + v.y / v.w;
@@ -2170,57 +2244,50 @@ extern "C" int ktm_image_reset(const ktm_plan *p, float *km, float *fold, float 
     return KTM_OK;
 }
 
-/* kernel choice: K sample slots per lane and W waves per column cover ns */
+/* kernel choice */
 typedef void (*mig_fn)(const MigArgs);
+struct MigShape {
+    mig_fn fn;
+    int K, W, NW, C;    /* samples per lane, waves per column, waves, rows per chunk */
+};
 
-/* B traces staged per batch (8: two workgroups per CU fit the LDS); accum
- * is KTM_ACCUM_PLAIN or KTM_ACCUM_KAHAN, optionally with KTM_INDEX_FAST */
-template <int K, int W, int B_ = 8>
-static mig_fn pick_accum(int accum, int *B)
+/* accum is KTM_ACCUM_PLAIN or KTM_ACCUM_KAHAN, optionally with KTM_INDEX_FAST */
+template <int K, int W, int NW, int C, int EU = 4>
+static MigShape pick_accum(int accum)
 {
-    *B = B_;
     const bool kahan = (accum & ~KTM_INDEX_FAST) == KTM_ACCUM_KAHAN;
+    MigShape m = {nullptr, K, W, NW, C};
     if (accum & KTM_INDEX_FAST)
-        return kahan ? k_migrate<K, W, B_, true, true> : k_migrate<K, W, B_, false, true>;
-    return kahan ? k_migrate<K, W, B_, true, false> : k_migrate<K, W, B_, false, false>;
+        m.fn = kahan ? k_migrate<K, W, NW, C, EU, true, true> : k_migrate<K, W, NW, C, EU, false, true>;
+    else
+        m.fn = kahan ? k_migrate<K, W, NW, C, EU, true, false> : k_migrate<K, W, NW, C, EU, false, false>;
+    return m;
 }
 
-/* W waves share one image column (each owns K*64 consecutive samples);
- * a workgroup is 8 waves, so it covers 8/W columns. */
-static mig_fn pick_migrate(int ns, int accum, int64_t wgs8, int *W, int *K, int *B)
+/* W waves share one image column (each owns K*64 consecutive samples); a
+ * workgroup of NW waves covers NW/W columns. */
+static MigShape pick_migrate(int ns, int accum, int64_t wgs8)
 {
     /* wgs8: workgroups of 8 columns (x offset classes) in the region.  An
      * image too small to give every CU two workgroups at the default layout
      * takes twice the waves per column with half the samples per lane: on
      * the 800-column, 1001-sample line 3.77 ms against 4.79 ms (the 1536-
      * sample layout gained nothing from 6 x 4 on a 1600-column line). */
-    if (ns <= 512) {
-        if (wgs8 < 512) { *W = 2; *K = 4; return pick_accum<4, 2>(accum, B); }
-        *W = 1; *K = 8; return pick_accum<8, 1>(accum, B);
-    }
-    if (ns <= 1024) {
-        if (2 * wgs8 < 512) { *W = 4; *K = 4; return pick_accum<4, 4>(accum, B); }
-        *W = 2; *K = 8; return pick_accum<8, 2>(accum, B);
-    }
-    /* (the Kahan K = 12 variant runs at 0.97x the plain one; four waves of
-     * K = 6 per column measured 0.72x, of K = 8 0.63x, before the Kahan sums
-     * were blocked per batch) */
-    if (ns <= 1536) { *W = 2; *K = 12; return pick_accum<12, 2>(accum, B); }
-    if (ns <= 2048) { *W = 4; *K = 8; return pick_accum<8, 4>(accum, B); }
-    if (ns <= 3072) { *W = 4; *K = 12; return pick_accum<12, 4>(accum, B); }
-    /* one column per workgroup (8 waves of K*64 samples) for long traces,
-     * with fewer traces staged per batch so the rows fit the LDS */
-    if (ns <= 4096) { *W = 8; *K = 8; return pick_accum<8, 8>(accum, B); }
-    *W = 8; *K = 12;
-    return pick_accum<12, 8, 5>(accum, B);
+    if (ns <= 512) return wgs8 < 512 ? pick_accum<4, 2, 8, 4>(accum) : pick_accum<8, 1, 8, 4>(accum);
+    if (ns <= 1024) return 2 * wgs8 < 512 ? pick_accum<4, 4, 8, 4>(accum) : pick_accum<8, 2, 8, 4>(accum);
+    if (ns <= 1536) return pick_accum<12, 2, 8, 4>(accum);
+    if (ns <= 2048) return pick_accum<8, 4, 16, 4>(accum);
+    if (ns <= 3072) return pick_accum<12, 4, 16, 4>(accum);
+    /* fewer rows per chunk for long traces, so that the ring fits the LDS */
+    if (ns <= 4096) return pick_accum<8, 8, 16, 2>(accum);
+    return pick_accum<12, 8, 16, 2>(accum);
 }
 
-/* Tiles of the region [rx0,rx1) x [ry0,ry1) at W waves per column: 8/W
- * columns, a row on a 2-D line, as square as possible in 3-D. */
-static void tile_layout(const ktm_setup *s, int W, MigArgs *a)
+/* Tiles of the region [rx0,rx1) x [ry0,ry1): ncol columns, a row on a 2-D
+ * line, as square as possible in 3-D. */
+static void tile_layout(const ktm_setup *s, int ncol, MigArgs *a)
 {
-    const int ncol = 8 / W;
-    a->tx_cols = s->nyp == 1 ? ncol : (ncol == 8 ? 4 : ncol == 4 ? 2 : ncol);
+    a->tx_cols = s->nyp == 1 ? ncol : (ncol == 8 ? 4 : ncol == 6 ? 3 : ncol == 4 ? 2 : ncol);
     a->ty_cols = ncol / a->tx_cols;
     a->tiles_x = (a->rx1 - a->rx0 + a->tx_cols - 1) / a->tx_cols;
     const int tiles_y = (a->ry1 - a->ry0 + a->ty_cols - 1) / a->ty_cols;
@@ -2253,10 +2320,9 @@ static int parts_workspace(ktm_plan *p)
     MigArgs a;
     memset(&a, 0, sizeof a);
     a.rx1 = s->nxp; a.ry1 = s->nyp;
-    int W = 1, K = 8, B = 8;
-    (void)pick_migrate(s->ns, KTM_ACCUM_KAHAN, ((int64_t)s->nxp * s->nyp + 7) / 8 * s->nh, &W, &K,
-                       &B);
-    tile_layout(s, W, &a);
+    const MigShape m = pick_migrate(s->ns, KTM_ACCUM_KAHAN,
+                                    ((int64_t)s->nxp * s->nyp + 7) / 8 * s->nh);
+    tile_layout(s, m.NW / m.W, &a);
     int n = parts_for((int64_t)a.ntiles * s->nh);
     const uint64_t per = 3ull * sizeof(float) * (uint64_t)s->nxp * s->nyp * s->nh * s->ns;
     if (n > 1 && (uint64_t)(n - 1) * per > KTM_PARTS_MAX_BYTES)
@@ -2388,7 +2454,7 @@ static int migrate_block(const ktm_plan *p, const void *prepared, int dtype, int
     }
     MigArgs a;
     memset(&a, 0, sizeof a);
-    a.prep = F; a.geom = geom; a.ntr = ntr; a.row = p->row;
+    a.prep = F; a.align16 = ((uintptr_t)F & 15u) == 0; a.geom = geom; a.ntr = ntr; a.row = p->row;
     a.km = km; a.fold = fold; a.comp = comp;
     a.vel2 = p->d_vel2; a.t1 = p->d_t1; a.velx = p->d_velx; a.vely = p->d_vely;
     a.t2 = p->d_t2; a.colx = p->d_colx; a.coly = p->d_coly;
@@ -2406,11 +2472,11 @@ static int migrate_block(const ktm_plan *p, const void *prepared, int dtype, int
         a.rx0 = (job / p->cfg.jobs_y) * s->nx; a.rx1 = a.rx0 + s->nx;
         a.ry0 = (job % p->cfg.jobs_y) * s->ny; a.ry1 = a.ry0 + s->ny;
     }
-    int W = 1, K = 8, B = 8;
     const int64_t ncols_region = (int64_t)(a.rx1 - a.rx0) * (a.ry1 - a.ry0);
-    mig_fn fn = pick_migrate(s->ns, accum, (ncols_region + 7) / 8 * s->nh, &W, &K, &B);
-    tile_layout(s, W, &a);
-    const int nthreads = 8 * KTM_WAVE;
+    const MigShape m = pick_migrate(s->ns, accum, (ncols_region + 7) / 8 * s->nh);
+    const mig_fn fn = m.fn;
+    tile_layout(s, m.NW / m.W, &a);
+    const int nthreads = m.NW * KTM_WAVE;
     /* compensated sums of a small region: the traces in parts */
     int nparts = 1;
     a.part_n = ncols_region * s->nh * s->ns;
@@ -2422,14 +2488,9 @@ static int migrate_block(const ktm_plan *p, const void *prepared, int dtype, int
         if (nparts > nchunks) nparts = (int)nchunks;     /* no part without a chunk */
     }
     a.nparts = nparts;
-    /* staged rows + geometry, selection list and counts, and: v^2 per sample
-     * and the speculation queue (exact index) or the fold row V (fast index) */
-    const bool fast = (accum & KTM_INDEX_FAST) != 0;
-    const size_t tail = fast ? sizeof(float) * (size_t)p->row
-                             : sizeof(float) * (size_t)(8 * K * KTM_WAVE) +
-                                   sizeof(uint2) * (size_t)(8 * KTM_SPEC_Q * KTM_WAVE);
-    const size_t lds = sizeof(float) * (size_t)(B * p->row + B * 8) +
-                       sizeof(int) * (size_t)(nthreads + 8) + tail;
+    /* the ring of rows, the slots' largest constants, the trace list, counts */
+    const size_t lds = sizeof(float) * (size_t)(3 * m.C * p->row + 2 * m.NW * m.K) +
+                       sizeof(int) * (size_t)(KTM_WAVE + m.C + nthreads + m.NW);
     if (lds > 160 * 1024) return KTM_ERR_UNSUPPORTED;
     /* runs of a row of tiles, but at least 8 runs per XCD */
     a.run = a.ntiles / 64 < a.tiles_x ? a.ntiles / 64 : a.tiles_x;
@@ -2439,14 +2500,23 @@ static int migrate_block(const ktm_plan *p, const void *prepared, int dtype, int
     if (nblk > 0x7fffffffLL) return KTM_ERR_UNSUPPORTED;
     const dim3 grid((unsigned)nblk, (unsigned)s->nh, (unsigned)nparts);
     HIP_TRY(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL(fn, grid, dim3(nthreads), lds, hs, a);
-    if (nparts > 1) {
-        const int64_t nb = (a.part_n + 255) / 256;
-        hipLaunchKernelGGL(k_merge_parts, dim3((unsigned)(nb < 8192 ? nb : 8192)), dim3(256), 0, hs,
-                           a, nparts);
+    /* at most 2^24 traces a launch: the kernels count a sample's passing
+     * traces in floats */
+    for (int64_t i0 = 0; i0 < ntr; i0 += 1 << 24) {
+        MigArgs b = a;
+        b.ntr = ntr - i0 < (1 << 24) ? ntr - i0 : (1 << 24);
+        b.prep = a.prep + i0 * a.row;
+        b.geom = a.geom + i0;
+        hipLaunchKernelGGL(fn, grid, dim3(nthreads), lds, hs, b);
+        if (nparts > 1) {
+            const int64_t nb = (a.part_n + 255) / 256;
+            hipLaunchKernelGGL(k_merge_parts, dim3((unsigned)(nb < 8192 ? nb : 8192)), dim3(256), 0,
+                               hs, b, nparts);
+        }
+        if (counter)
+            hipLaunchKernelGGL(k_count_outside, dim3((unsigned)((b.ntr + 255) / 256)), dim3(256), 0,
+                               hs, b);
     }
-    if (counter)
-        hipLaunchKernelGGL(k_count_outside, dim3((unsigned)((ntr + 255) / 256)), dim3(256), 0, hs, a);
     HIP_TRY(hipGetLastError());
     return KTM_OK;
 }

@@ -194,3 +194,37 @@ def test_compensated_and_16bit_long_traces(cuda, ns):
         print(f"  dtype {dtype}: relL2 vs FP64 {r:.2e}", flush=True)
         assert n == n64 and np.array_equal(fold.cpu().numpy(), fold64.astype(np.float32))
         assert r <= tol
+
+
+@pytest.mark.parametrize("ns", [301, 1003, 1500, 2047, 2600, 3500, 5000])
+@pytest.mark.parametrize("ntr", [1, 3, 5, 64, 67, 69, 133, 515, 1089])
+def test_trace_list_and_ring_boundaries_bitexact(cuda, ns, ntr):
+    """Trace counts around the steps of the trace stream of every lane layout
+    (rows staged 2 or 4 at a time, gates 64 at a time, blocks of 512 or 1024
+    traces filtered into the list), with every third trace outside the
+    offset classes and zero-offset traces on a column (q < 1 at t = 0)."""
+    print(f"case: {ntr} traces x {ns} samples", flush=True)
+    sv = small_line(ns, nshots=55, nrecv_side=10, ncols=9, jobs_x=1, nh=1, dh=110.0)
+    co = sv.coords[np.random.default_rng(ntr).permutation(sv.ntr)[:ntr]].copy()
+    co[::4, 2] = co[::4, 0] = 625 * (1 + np.arange(co[::4].shape[0]) % 7)
+    sv.coords = co
+    tr = np.random.default_rng(ns).standard_normal((ntr, ns)).astype(np.float32)
+    bitexact_case(sv, tr, cuda)
+
+
+def test_prepared_rows_at_any_float(cuda):
+    """Prepared rows that start 4 bytes past a 16-byte boundary migrate to the
+    same bits as aligned ones."""
+    print("case: prepared rows 4 bytes past a 16-byte boundary", flush=True)
+    sv = small_line(700)
+    plan = Plan(sv.cfg, sv.ns, sv.dt, sv.vel)
+    tr = torch.from_numpy(surveys.traces_numpy(sv)).to(cuda)
+    prepared, geom = plan.prep(tr, torch.from_numpy(sv.coords).to(cuda))
+    km, fold, _ = plan.new_image(device=cuda)
+    plan.migrate_block(prepared, geom, km, fold)
+    odd = torch.empty(prepared.numel() + 1, device=cuda)[1:].view_as(prepared)
+    odd.copy_(prepared)
+    assert odd.data_ptr() % 16 == 4
+    km2, fold2, _ = plan.new_image(device=cuda)
+    plan.migrate_block(odd, geom, km2, fold2)
+    assert bool(km.any()) and torch.equal(km, km2) and torch.equal(fold, fold2)
