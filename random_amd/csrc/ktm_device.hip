@@ -211,125 +211,212 @@ __device__ __forceinline__ float decode_word(uint32_t u)
     return SRC == SRC_SEGY_IBM ? ibm_word(w) : __uint_as_float(w);
 }
 
+/* the same for N words: where no exponent reaches 2^128 (one test for all)
+ * the power of 16 is finite and the product of ibm_word is one exact scaling,
+ * fraction x 2^(4 (exponent - 64) - 24), rounded once */
+template <int SRC, int N>
+__device__ __forceinline__ void decode_words(const uint32_t *u, float *x)
+{
+    if (SRC != SRC_SEGY_IBM) {
+#pragma unroll
+        for (int m = 0; m < N; ++m) x[m] = decode_word<SRC>(u[m]);
+        return;
+    }
+    uint32_t big = 0u;
+#pragma unroll
+    for (int m = 0; m < N; ++m) big = max(big, u[m] & 0x7fu);   /* the exponent, as stored */
+    if (__ballot(big >= 96u)) {
+#pragma unroll
+        for (int m = 0; m < N; ++m) x[m] = decode_word<SRC>(u[m]);
+    } else {
+#pragma unroll
+        for (int m = 0; m < N; ++m) {
+            const uint32_t w = __builtin_bswap32(u[m]);
+            const float v = __builtin_amdgcn_ldexpf((float)(w & 0x00ffffffu), 4 * (int)(u[m] & 0x7fu) - 280);
+            x[m] = __uint_as_float((__float_as_uint(v) & 0x7fffffffu) | (w & 0x80000000u));
+        }
+    }
+}
+
 template <int SRC>
 __device__ __forceinline__ float load_sample(const TraceSrc &s, int64_t i, int t)
 {
     return decode_word<SRC>(load_word<SRC>(s, i, t));
 }
 
-/* REFERENCE mode: one lane per trace runs the two FP32 running sums of
- * Kirchhoff.c:1314-1324 in a single pass, keeping the last five values of
- * the double integral p[] in registers, and emits
+/* REFERENCE mode: the two FP32 running sums of Kirchhoff.c:1314-1324 per
+ * trace, emitting
  *   F[T] = (float)(-2.0*p[T] + p[T-2] + p[T+2])         (Kirchhoff.c:1392)
- * as soon as p[T+2] exists (F[t-2] at step t).  p[-1] = p[1] and p[-2] =
- * p[2] are the mirror pad of Kirchhoff.c:1327-1328.  A workgroup is one
- * wave of 64 traces; samples pass through LDS in tiles of 64 so that every
- * global load and store is one contiguous 256-byte run of a trace row (a
- * lane walking its own row would touch 64 rows per instruction). */
+ * as soon as p[T+2] exists (F[t-2] at step t), p[] the double integral of
+ * which the last five values stay in registers.  p[-1] = p[1] and p[-2] =
+ * p[2] are the mirror pad of Kirchhoff.c:1327-1328.
+ *
+ * A workgroup takes 64 traces.  Its first wave runs the recurrence, one lane
+ * per trace, and nothing else: one step is a double add between two
+ * conversions (the chain), the second sum and F.  Two helper waves feed it
+ * through LDS, a tile of PREP_TS steps ahead: they load the samples
+ * (PREP_AHEAD tiles ahead, two traces x 32 samples per instruction), decode
+ * them, divide by 4 t2[t] (the increment of integral 1 does not depend on the
+ * running sum), and store the F of the tile before.  Tile i's steps are
+ * t = 32 (i - 1) + 2 ..., so its F start at a multiple of 32.  One barrier
+ * per tile.
+ * Bound by the recurrence's chain for few traces and by memory for a full
+ * block: 50,000 IBM records of 1500 samples 319 -> 170 us (3.6 TB/s), 96
+ * traces of 501 74 -> 20 us, against one wave that did all of it with a full
+ * double division per sample.  Of the same block with 4 helper waves 180 us,
+ * 8 200, tiles of 16 steps 250, and with the division in the recurrence wave
+ * and tiles of 64 steps 350. */
 #define PREP_TS 32
+#define PREP_HELPERS 2
+#define PREP_AHEAD 2        /* tiles in flight */
+#define PREP_NT (KTM_WAVE * (1 + PREP_HELPERS))
 template <int SRC>
-__global__ void __launch_bounds__(KTM_WAVE)
+__global__ void __launch_bounds__(PREP_NT)
 k_prep_ref(const TraceSrc src, int64_t ntr, int ns, int64_t row, float dt,
            const float *__restrict__ t2, float *__restrict__ out)
 {
-    /* s_inc[j][k]: the increment of integral 1 at t = t0 + k of trace j,
-     * (double)tr[t] / (4 t2[t]) (Kirchhoff.c:1314); at t = 0 the sample
-     * itself.  It does not depend on the running sum, so it is computed in
-     * the load phase, lane-parallel, and the sequential recurrence is left
-     * with one double add and two conversions per step.  Loads and stores
-     * move two traces x 32 samples per instruction (128-byte runs). */
-    __shared__ double s_inc[KTM_WAVE][PREP_TS + 1];
-    __shared__ float s_out[KTM_WAVE][PREP_TS + 1];
-    const int lane = threadIdx.x;
-    const int sub = lane & (PREP_TS - 1), half = lane / PREP_TS;
+    /* slot (b, j, k), b the tile's parity: the increment of integral 1 at the
+     * tile's step k of trace j, (double)tr[t] / (4 t2[t]) (Kirchhoff.c:1314),
+     * at t = 0 the sample itself; then, in its place, F of that step.  A
+     * helper lane reads the F and writes the increment two tiles on of the
+     * same slots, so one pair of buffers holds both. */
+    union Slot { double inc; float f; };
+    __shared__ Slot s[2][KTM_WAVE][PREP_TS + 1];
+    constexpr int PER = PREP_TS / PREP_HELPERS;                 /* samples per helper lane */
+    constexpr int STEP = KTM_WAVE * PREP_HELPERS / PREP_TS;     /* traces per helper pass */
     const int64_t tr0 = (int64_t)blockIdx.x * KTM_WAVE;
     const int ntl = (int)min((int64_t)KTM_WAVE, ntr - tr0);
-    const int64_t i = tr0 + (lane < ntl ? lane : 0);
-    const float last = load_sample<SRC>(src, i, ns - 1);
-    float q = 0.0f, p = 0.0f;
-    float pm1 = 0.0f, pm2 = 0.0f, pm3 = 0.0f, pm4 = 0.0f;
-    /* unconditional loads at clamped (in-bounds) positions, so that all 32
-     * are in flight before the first wait; out-of-range values are replaced
-     * after the decode.  The next tile's words are loaded as soon as this
-     * tile's are decoded, so their latency overlaps the recurrence. */
-    uint32_t wv[KTM_WAVE / 2];
-    float t2v;
-    {
-        const int tc = sub < ns ? sub : ns - 1;
+    const int ntiles = (ns + PREP_TS - 1) / PREP_TS + 1;        /* steps up to ns + 1 */
+    if (threadIdx.x < KTM_WAVE) {
+        /* ---- the recurrence: tile i in phase i ---- */
+        const int lane = threadIdx.x;
+        const float last = load_sample<SRC>(src, tr0 + (lane < ntl ? lane : 0), ns - 1);
+        float q = 0.0f, p = 0.0f;
+        double dm1 = 0.0, dm2 = 0.0, dm3 = 0.0, dm4 = 0.0, d0 = 0.0;   /* p[t-1..t-4], p[t] */
+        __syncthreads();
+        for (int i = 0; i < ntiles; ++i) {
+            const int t0 = (i - 1) * PREP_TS + 2;
+            Slot *sl = s[i & 1][lane];
+            if (t0 >= 4 && t0 + PREP_TS <= ns) {
+                /* interior tile: every step is the t >= 4, t < ns case */
+                double iv[PREP_TS];
 #pragma unroll
-        for (int m = 0; m < KTM_WAVE / 2; ++m)
-            wv[m] = load_word<SRC>(src, tr0 + min(2 * m + half, ntl - 1), tc);
-        t2v = t2[tc];
+                for (int k = 0; k < PREP_TS; ++k) iv[k] = sl[k].inc;
+#pragma unroll
+                for (int k = 0; k < PREP_TS; ++k) {
+                    q = (float)((double)q + iv[k]);
+                    dm4 = dm3; dm3 = dm2; dm2 = dm1; dm1 = d0;
+                    p = p + q;
+                    d0 = (double)p;
+                    sl[k].f = (float)(-2.0 * dm2 + dm4 + d0);
+                }
+            } else {
+                const int s_end = min(PREP_TS, ns + 2 - t0);
+                for (int k = max(0, -t0); k < s_end; ++k) {
+                    const int tk = t0 + k;
+                    if (tk == 0) {
+                        q = (float)sl[k].inc;   /* integral 1 at t */
+                        p = q;                  /* integral 2 at t */
+                        d0 = (double)p;
+                        continue;
+                    }
+                    if (tk < ns)
+                        q = (float)((double)q + sl[k].inc);
+                    else
+                        q = q + last / dt / dt / (float)tk / (float)tk;
+                    dm4 = dm3; dm3 = dm2; dm2 = dm1; dm1 = d0;
+                    p = p + q;
+                    d0 = (double)p;
+                    if (tk == 2)
+                        sl[k].f = (float)(-2.0 * dm2 + d0 + d0);
+                    else if (tk == 3)
+                        sl[k].f = (float)(-2.0 * dm2 + dm2 + d0);
+                    else if (tk >= 4)
+                        sl[k].f = (float)(-2.0 * dm2 + dm4 + d0);
+                }
+            }
+            __syncthreads();
+        }
+        return;
     }
-    for (int t0 = 0; t0 < ns + 2; t0 += PREP_TS) {
-        const int t = t0 + sub;
-        const double den = t < ns && t > 0 ? 4.0 * (double)t2v : 1.0;
-        float xv[KTM_WAVE / 2];
+    /* ---- helpers: lane (sub, tb) moves step sub of traces tb, tb + STEP .. */
+    const int hid = threadIdx.x - KTM_WAVE;
+    const int sub = hid & (PREP_TS - 1), tb = hid / PREP_TS;
+    uint32_t wv[PREP_AHEAD][PER];       /* tile i in place i % PREP_AHEAD */
+    float t2v[PREP_AHEAD];
+    /* the workgroup's first record and output row; 32-bit offsets from there */
+    const uint32_t *sp = reinterpret_cast<const uint32_t *>(src.p) + tr0 * src.rec_words +
+                         (SRC == SRC_F32 ? 0 : 60);
+    float *op = out + tr0 * row;
+    const uint32_t rw = (uint32_t)src.rec_words, orow = (uint32_t)row;
+    const bool full = ntl == KTM_WAVE;
+    /* unconditional loads at clamped (in-bounds) positions, all in flight
+     * together; out-of-range values are replaced after the decode */
+    auto load = [&](int i, int a) __attribute__((always_inline)) {
+        const int t = (i - 1) * PREP_TS + 2 + sub, tc = min(max(t, 0), ns - 1);
+        if (full) {
+            const uint32_t o = (uint32_t)tb * rw + (uint32_t)tc;
 #pragma unroll
-        for (int m = 0; m < KTM_WAVE / 2; ++m)
-            xv[m] = t < ns ? decode_word<SRC>(wv[m]) : 0.0f;
+            for (int m = 0; m < PER; ++m) wv[a][m] = (sp + (uint32_t)(m * STEP) * rw)[o];
+        } else {
 #pragma unroll
-        for (int m = 0; m < KTM_WAVE / 2; ++m)
-            s_inc[2 * m + half][sub] = t == 0 ? (double)xv[m] : (double)xv[m] / den;
-        if (t0 + PREP_TS < ns + 2) {
-            const int tn = t0 + PREP_TS + sub;
-            const int tc = tn < ns ? tn : ns - 1;
-#pragma unroll
-            for (int m = 0; m < KTM_WAVE / 2; ++m)
-                wv[m] = load_word<SRC>(src, tr0 + min(2 * m + half, ntl - 1), tc);
-            t2v = t2[tc];
+            for (int m = 0; m < PER; ++m)
+                wv[a][m] = sp[(uint32_t)min(tb + m * STEP, ntl - 1) * rw + (uint32_t)tc];
         }
-        __syncthreads();
-        const int s_end = min(PREP_TS, ns + 2 - t0);
-        if (t0 >= 4 && t0 + PREP_TS <= ns) {
-            /* interior tile: every step is the t >= 4, t < ns case; unrolled
-             * so that the LDS reads and the F arithmetic overlap the
-             * recurrence (one double add and two conversions per step) */
-            double inc[PREP_TS];
+        t2v[a] = t2[tc];
+    };
+    auto feed = [&](int i, int a) __attribute__((always_inline)) {
+        const int t = (i - 1) * PREP_TS + 2 + sub;
+        const double den = t > 0 && t < ns ? 4.0 * (double)t2v[a] : 1.0;
+        const double rden = 1.0 / den;
+        float x[PER];
+        decode_words<SRC, PER>(wv[a], x);
+        if (i < 2 || i * PREP_TS + 2 > ns) {
 #pragma unroll
-            for (int k = 0; k < PREP_TS; ++k) inc[k] = s_inc[lane][k];
+            for (int m = 0; m < PER; ++m) x[m] = t >= 0 && t < ns ? x[m] : 0.0f;
+        }
 #pragma unroll
-            for (int k = 0; k < PREP_TS; ++k) {
-                q = (float)((double)q + inc[k]);
-                pm4 = pm3; pm3 = pm2; pm2 = pm1; pm1 = p;
-                p = p + q;
-                s_out[lane][k] = (float)(-2.0 * (double)pm2 + (double)pm4 + (double)p);
-            }
-        } else for (int k = 0; k < s_end; ++k) {
-            const int tk = t0 + k;
-            const double inc = s_inc[lane][k];
-            if (tk == 0) {
-                q = (float)inc;   /* integral 1 at t */
-                p = q;            /* integral 2 at t */
-                continue;
-            }
-            if (tk < ns)
-                q = (float)((double)q + inc);
-            else
-                q = q + last / dt / dt / (float)tk / (float)tk;
-            pm4 = pm3; pm3 = pm2; pm2 = pm1; pm1 = p;
-            p = p + q;
-            /* window: pm4..p = p[t-4]..p[t]; F[t-2] goes to s_out[.][k] */
-            if (tk == 2)
-                s_out[lane][k] = (float)(-2.0 * (double)pm2 + (double)p + (double)p);
-            else if (tk == 3)
-                s_out[lane][k] = (float)(-2.0 * (double)pm2 + (double)pm2 + (double)p);
-            else if (tk >= 4)
-                s_out[lane][k] = (float)(-2.0 * (double)pm2 + (double)pm4 + (double)p);
+        for (int m = 0; m < PER; ++m)
+            /* x / den correctly rounded from RN(1/den), zeros, infinities,
+             * NaN and a zero den as the division gives them */
+            s[i & 1][tb + m * STEP][sub].inc = __builtin_amdgcn_div_fixup(
+                div_cr((double)x[m], den, rden), den, (double)x[m]);
+    };
+    /* F of tile i, T = 32 (i - 1) + sub, and zeros from ns to the row's end */
+    auto store = [&](int i) __attribute__((always_inline)) {
+        const int T = (i - 1) * PREP_TS + sub;
+        const uint32_t o = (uint32_t)tb * orow + (uint32_t)T;
+        if (full && i > 0 && i * PREP_TS <= ns) {
+#pragma unroll
+            for (int m = 0; m < PER; ++m)
+                (op + (uint32_t)(m * STEP) * orow)[o] = s[i & 1][tb + m * STEP][sub].f;
+            return;
         }
-        __syncthreads();
-        const int T = t0 - 2 + sub;           /* F index held in s_out[.][sub] */
-        if (sub < s_end && T >= 0 && T < ns) {
-#pragma unroll 8
-            for (int m = 0; m < KTM_WAVE / 2; ++m) {
-                const int j = 2 * m + half;
-                if (j < ntl) out[(tr0 + j) * row + T] = s_out[j][sub];
-            }
+        if (T < 0 || T >= row) return;
+#pragma unroll
+        for (int m = 0; m < PER; ++m) {
+            const int j = tb + m * STEP;
+            if (j < ntl) op[(uint32_t)(m * STEP) * orow + o] = T < ns ? s[i & 1][j][sub].f : 0.0f;
         }
-        __syncthreads();
+    };
+#pragma unroll
+    for (int a = 0; a < PREP_AHEAD; ++a) load(a, a);
+    feed(0, 0);
+    __syncthreads();
+    for (int i0 = 0; i0 < ntiles; i0 += PREP_AHEAD) {
+#pragma unroll
+        for (int a = 0; a < PREP_AHEAD; ++a) {
+            const int i = i0 + a;
+            if (i >= ntiles) break;
+            /* phase i: tile i's registers are free, tile i + 1 is fed */
+            load(i + PREP_AHEAD, a);
+            store(i - 1);
+            if (i + 1 < ntiles) feed(i + 1, (a + 1) % PREP_AHEAD);
+            __syncthreads();
+        }
     }
-    for (int j = 0; j < ntl; ++j)
-        for (int64_t T = ns + lane; T < row; T += KTM_WAVE) out[(tr0 + j) * row + T] = 0.0f;
+    store(ntiles - 1);
+    store(ntiles);                          /* the row's end past the last tile */
 }
 
 /* CLOSED mode: F as the 3-tap filter of x[t] = trace[min(t,ns-1)] * w[t].
@@ -433,6 +520,7 @@ __device__ __forceinline__ float f16_to_f32(uint16_t u)
  * 32 samples per load (max is exact in any order); the sequential
  * error-feedback sweep stages 32-sample tiles through LDS like k_prep_ref,
  * one lane per trace. */
+#define QUANT_TS 32
 #define QA1 1.625f
 #define QA2 (-1.625f)
 #define QA3 1.5f
@@ -444,19 +532,19 @@ __global__ void __launch_bounds__(KTM_WAVE)
 k_quantize(const TraceSrc src, int64_t ntr, int ns, int64_t row, uint16_t *__restrict__ q,
            ktm_trace_geom *__restrict__ geom)
 {
-    __shared__ float s_in[KTM_WAVE][PREP_TS + 1];
-    __shared__ uint16_t s_q[KTM_WAVE][PREP_TS + 2];
+    __shared__ float s_in[KTM_WAVE][QUANT_TS + 1];
+    __shared__ uint16_t s_q[KTM_WAVE][QUANT_TS + 2];
     __shared__ float s_scale[KTM_WAVE];
     const int lane = threadIdx.x;
-    const int sub = lane & (PREP_TS - 1), half = lane / PREP_TS;
+    const int sub = lane & (QUANT_TS - 1), half = lane / QUANT_TS;
     const int64_t tr0 = (int64_t)blockIdx.x * KTM_WAVE;
     const int ntl = (int)min((int64_t)KTM_WAVE, ntr - tr0);
     for (int m = 0; m < KTM_WAVE / 2; ++m) {
         const int j = min(2 * m + half, ntl - 1);
         float mx = 0.0f;
 #pragma unroll 8
-        for (int t = sub; t < ns; t += PREP_TS) mx = fmaxf(mx, fabsf(load_sample<SRC>(src, tr0 + j, t)));
-        for (int o = PREP_TS / 2; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+        for (int t = sub; t < ns; t += QUANT_TS) mx = fmaxf(mx, fabsf(load_sample<SRC>(src, tr0 + j, t)));
+        for (int o = QUANT_TS / 2; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
         if (sub == 0) s_scale[2 * m + half] = mx;
     }
     __syncthreads();
@@ -464,7 +552,7 @@ k_quantize(const TraceSrc src, int64_t ntr, int ns, int64_t row, uint16_t *__res
     const float scale = m_own > 0.0f ? m_own : 1.0f;
     const float inv = 1.0f / scale;
     float e1 = 0.0f, e2 = 0.0f, e3 = 0.0f, e4 = 0.0f, e5 = 0.0f, e6 = 0.0f;   /* e[t-1] .. */
-    for (int t0 = 0; t0 < ns; t0 += PREP_TS) {
+    for (int t0 = 0; t0 < ns; t0 += QUANT_TS) {
         const int t = t0 + sub;
         const int tc = t < ns ? t : ns - 1;
         uint32_t wv[KTM_WAVE / 2];
@@ -474,13 +562,13 @@ k_quantize(const TraceSrc src, int64_t ntr, int ns, int64_t row, uint16_t *__res
 #pragma unroll
         for (int m = 0; m < KTM_WAVE / 2; ++m) s_in[2 * m + half][sub] = decode_word<SRC>(wv[m]);
         __syncthreads();
-        const int s_end = min(PREP_TS, ns - t0);
-        if (s_end == PREP_TS) {
-            float xk[PREP_TS];
+        const int s_end = min(QUANT_TS, ns - t0);
+        if (s_end == QUANT_TS) {
+            float xk[QUANT_TS];
 #pragma unroll
-            for (int k = 0; k < PREP_TS; ++k) xk[k] = s_in[lane][k];
+            for (int k = 0; k < QUANT_TS; ++k) xk[k] = s_in[lane][k];
 #pragma unroll
-            for (int k = 0; k < PREP_TS; ++k) {
+            for (int k = 0; k < QUANT_TS; ++k) {
                 const float fb = ((((QA1 * e1 + QA2 * e2) + QA3 * e3) + QA4 * e4) + QA5 * e5) + QA6 * e6;
                 const float v = xk[k] * inv + fb;
                 const uint16_t h = DT == KTM_TRACE_BF16 ? f32_to_bf16(v) : f32_to_f16(v);
@@ -1926,7 +2014,7 @@ static int prep_launch(const ktm_plan *p, const TraceSrc src, int64_t ntr, int p
     if (dtype == KTM_TRACE_F32) {
         if (prep_mode == KTM_PREP_REFERENCE) {
             hipLaunchKernelGGL(k_prep_ref<SRC>, dim3((unsigned)((ntr + KTM_WAVE - 1) / KTM_WAVE)),
-                               dim3(KTM_WAVE), 0, s, src, ntr, ns, p->row, p->tb.s.dt, p->d_t2,
+                               dim3(PREP_NT), 0, s, src, ntr, ns, p->row, p->tb.s.dt, p->d_t2,
                                (float *)prepared);
         } else {
             if (ntr > 65535 * 1024LL) return KTM_ERR_UNSUPPORTED;

@@ -181,3 +181,39 @@ def test_image_records_match_host_headers(cuda, ns):
                     tr = img[xs * nx + xc, ys * ny + yc, ih].astype(">f4").view(np.uint8)
                     assert np.array_equal(got[r, 240:], tr)
                     r += 1
+
+
+@pytest.mark.parametrize("fmt", [SEGY_IBM, SEGY_IEEE])
+@pytest.mark.parametrize("ns,ntr", [(4, 1), (29, 3), (30, 64), (31, 65), (32, 63), (33, 1), (61, 130),
+                                    (64, 64), (95, 2), (1501, 67)])
+def test_reference_prep_tiles_bitexact(cuda, fmt, ns, ntr):
+    """The running sums over every tile edge (steps t = 32 i + 2), partial
+    workgroups of 64 traces, and words that are zero of either sign, infinite
+    (an IBM exponent past 2^127) and subnormal, against the oracle."""
+    print(f"case: {ntr} records x {ns} samples, format {fmt}", flush=True)
+    sv = surveys.line2d(nshots=1, nrecv_side=2, ns=max(ns, 4), ncols=4)
+    plan = Plan(sv.cfg, ns, sv.dt, np.ascontiguousarray(sv.vel[:, :, :ns]))
+    rng = np.random.default_rng(ns * 1000 + ntr)
+    words = rng.integers(0, 2 ** 32, (ntr, ns), dtype=np.uint64).astype(np.uint32)
+    if fmt == SEGY_IBM:
+        words = (words & 0x80ffffff) | (rng.integers(58, 70, (ntr, ns)).astype(np.uint32) << 24)
+    else:
+        words = rng.standard_normal((ntr, ns)).astype(np.float32).view(np.uint32)
+    words[0, ::7] = 0x80000000
+    words[0, 1::7] = 0
+    if ntr > 2:                        # one trace each: inf, and tiny values
+        words[1, ns // 2] = 0x7f123456 if fmt == SEGY_IBM else 0x7f800000
+        words[2, ::3] = 0x1c000001 if fmt == SEGY_IBM else 0x00000123
+    raw = np.zeros((ntr, 60 + ns), np.uint32)
+    raw[:, 18:22] = 1000
+    raw[:, 60:] = words
+    d_raw = torch.from_numpy(raw.byteswap().view(np.uint8).reshape(-1).copy()).to(cuda)
+    got = plan.ingest(d_raw, ntr, fmt)[0].cpu().numpy()
+    tr = oracle.ibm_to_float(words.byteswap().view(np.uint8)).reshape(ntr, ns) \
+        if fmt == SEGY_IBM else words.view(np.float32)
+    for j in range(ntr):
+        want = oracle.filtered_trace(oracle.trace_prep(tr[j], sv.dt, 2), 2, ns)
+        nan = np.isnan(want)
+        assert np.array_equal(np.isnan(got[j, :ns]), nan), j
+        assert np.array_equal(got[j, :ns].view(np.uint32)[~nan], want.view(np.uint32)[~nan]), j
+    assert got.shape == (ntr, plan.row) and not got[:, ns:].any()
