@@ -12,8 +12,8 @@
  * hipStream_t passed as void* (NULL = the null stream).  A plan is not
  * thread-safe; distinct plans may be used from distinct threads.  A plan's
  * workspaces (the BF16/FP16 decode buffer and the compensated partial
- * images of ktm_migrate_block, the demigration sort keys and max-|km| word
- * of ktm_demigrate) are reused by
+ * images of ktm_migrate_block, the demigration sort keys, sums of column
+ * parts and max-|km| word of ktm_demigrate) are reused by
  * every call without stream ordering: all calls on one plan must be issued
  * on a single stream (or the caller orders them), or a later call can
  * overwrite a workspace an earlier call's kernels still read.  ktm_prep,

@@ -76,6 +76,8 @@ struct ktm_plan {
     void *d_dm_tmp;
     size_t dm_cap, dm_tmp_bytes;
     uint32_t *d_dm_amax;    /* bits of max |km| of the last demigration */
+    unsigned long long *d_dm_sum; /* sums of a demigration whose columns are in parts */
+    size_t dm_sum_cap;      /* words of d_dm_sum */
     float *d_scratch;       /* this device's copy of `scratch` (ktm_migrate_block_static) */
     /* compensated migration of small images: partial images of parts 1..
      * parts_max-1 of a trace block, [part][km, fold, comp][image or region] */
@@ -788,6 +790,7 @@ __device__ __forceinline__ int reference_T(float dIS2, float dIR2, float rsn, fl
 
 typedef __attribute__((address_space(3))) float lds_float;
 typedef __attribute__((address_space(3))) void lds_void;
+typedef __attribute__((address_space(3))) unsigned long long lds_u64;
 typedef __attribute__((address_space(1))) const void global_void;
 
 /* One workgroup = NW waves = NCOL image columns x W time segments.  Each lane
@@ -1539,19 +1542,65 @@ __global__ void k_pixel_velocity(const float *__restrict__ vel2, const int32_t *
 }
 
 #define DM_TB 8                      /* traces per demigration workgroup, at most */
+#define DM_PAD KTM_WAVE              /* words past g[ns - 1]: one per lane */
 
 struct DemigArgs {
     const float *km;                 /* image [nxp][nyp][nh][ns] */
     const ktm_trace_geom *geom;
-    const int32_t *order;            /* trace order (workgroup b takes order[b*tb ...]) or NULL */
+    const int32_t *order;            /* trace order (workgroup b takes order[b*tb ...]) */
     int64_t ntr;
     float *traces;                   /* out [ntr][ns] */
+    unsigned long long *gsum;        /* columns in parts (gridDim.y > 1): [ntr][ns], zeroed */
     const float *pv2, *prs, *t2, *w, *colx, *coly, *slab_cx, *slab_cy, *slab_x2thr;
     const uint32_t *amax;            /* bits of max |km| (k_absmax) */
     float ap_x2thr, aperture, dt, rdt;
     int ns, nh, nxp, nyp, nx, ny, jobs_y, tb;
     int lg_terms;                    /* 2^lg_terms >= nxp * nyp * ns, terms per g[T] at most */
 };
+
+/* the fixed point of g: km is scaled by 2^E, max |km| < 2^emax; |km 2^E| <
+ * 2^51 in any case (to_fixed) */
+__device__ __forceinline__ int demig_exponent(const DemigArgs &a)
+{
+    const float amax = __uint_as_float(*a.amax);
+    int emax = 0;
+    if (amax > 0.0f) (void)frexpf(amax, &emax);
+    return min(59 - a.lg_terms, 51) - emax;
+}
+
+/* trunc(m 2^E) as an integer, |m 2^E| < 2^51: the double sum with 1.5 * 2^52
+ * holds it in its low bits (the compiler's float to 64-bit conversion takes
+ * twice the instructions) */
+__device__ __forceinline__ unsigned long long to_fixed(float m, int E)
+{
+    constexpr double MAGIC = 6755399441055744.0;
+    const double s = __builtin_trunc(__builtin_amdgcn_ldexp((double)m, E)) + MAGIC;
+    return (unsigned long long)__double_as_longlong(s) -
+           (unsigned long long)__double_as_longlong(MAGIC);
+}
+
+/* sample t of L m from the trace's sums g[0..ns): the transpose of F =
+ * closed_tap(x), x[t] = tr[min(t, ns-1)] * w[t], in double from the
+ * fixed-point sums (q = 2^-E) */
+__device__ __forceinline__ float demig_sample(const long long *gl, int t, int ns, const float *w,
+                                              double q)
+{
+    double acc = 0.0;
+    const int nt_ = t == ns - 1 ? 3 : 1;   /* tr[ns-1] also feeds x[ns], x[ns+1] */
+    for (int u = 0; u < nt_; ++u) {
+        const int tt = t + u;
+        long long xb = 0;                  /* exact: |g| < 2^59, weights summing to <= 6 */
+        if (tt >= 2 && tt < ns) xb += gl[tt];
+        if (tt - 1 >= 2 && tt - 1 < ns) xb += 2 * gl[tt - 1];
+        if (tt - 2 >= 2 && tt - 2 < ns) xb += gl[tt - 2];
+        if (tt == 0) xb += 4 * gl[0] + 2 * gl[1];
+        if (tt == 1) xb += 4 * gl[0] + 2 * gl[1];
+        if (tt == 2) xb += 2 * gl[0] + 2 * gl[1];
+        if (tt == 3) xb += gl[1];
+        acc += (double)w[tt] * ((double)xb * q);
+    }
+    return (float)acc;
+}
 
 /* *out = bits of max |x| over n floats (out zeroed by k_zero_u32 first;
  * non-negative floats order like their bit patterns) */
@@ -1610,6 +1659,27 @@ __global__ void k_demig_keys(const ktm_trace_geom *__restrict__ geom, int64_t nt
     idx[i] = (int32_t)i;
 }
 
+/* add v to the LDS word at byte address ad */
+__device__ __forceinline__ void lds_add(uint32_t ad, unsigned long long v)
+{
+    (void)__hip_atomic_fetch_add((lds_u64 *)(uintptr_t)ad, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+/* the largest of a wave's non-negative floats, in a scalar */
+__device__ __forceinline__ float wave_max(float v)
+{
+    int m = __float_as_int(v);
+#define KTM_DPP_MAX(ctrl, rows) m = max(m, __builtin_amdgcn_update_dpp(m, m, ctrl, rows, 0xf, false))
+    KTM_DPP_MAX(0x111, 0xf);    /* row_shr 1, 2, 4, 8 */
+    KTM_DPP_MAX(0x112, 0xf);
+    KTM_DPP_MAX(0x114, 0xf);
+    KTM_DPP_MAX(0x118, 0xf);
+    KTM_DPP_MAX(0x142, 0xa);    /* row_bcast 15, 31 */
+    KTM_DPP_MAX(0x143, 0xc);
+#undef KTM_DPP_MAX
+    return __int_as_float(__builtin_amdgcn_readlane(m, 63));
+}
+
 /* L, the exact transpose of migration with the CLOSED filter (km = L^T d).
  * A workgroup takes up to DM_TB traces, neighbours in the sort order of
  * k_demig_keys: the waves walk the image columns of the union of their
@@ -1626,35 +1696,50 @@ __global__ void k_demig_keys(const ktm_trace_geom *__restrict__ geom, int64_t nt
  * max |km| * 2^(lg_terms - 59).
  * Each trace is then the transpose of the 3-tap filter and of the sample
  * weights applied to its g.
- * Lane l owns samples l*K + ((k + l) mod K) of its wave's 64K-sample
+ * Lane l owns samples l*K + ((k + l / P) mod K) of its wave's 64K-sample
  * segment, not k*64 + l: far from the CMP, T(t) grows slowly at early
  * times, and 64 consecutive samples land on a few T, whose atomics then
- * serialise; samples ~13 apart land on distinct T in distinct banks.
+ * serialise; samples K apart land on distinct T, and with P = 32 / gcd(K, 32)
+ * the 64 lanes' T spread over all banks where T(t) = t + const.  A sample past
+ * the trace is clamped to ns + lane + 1/2 and adds into its lane's own unread
+ * word (all lanes adding into one word serialised: with offsets up to 4 km
+ * and 751 samples that was most of the time).
  * A sample whose fast-form q lies within the form's error bound of an
  * integer needs the reference arithmetic: each lane defers its first such
  * sample of a column and the wave resolves them after the column's traces,
  * every lane's together (the integer sums do not depend on the order of the
- * additions); a lane's further ones in the column take it inline.
- * FASTIDX: the index floor(min(q, ns + 1/2)) of the fast form alone, the
- * transpose of k_migrate's FASTIDX variant (floor(min(q, ns)) there: both
- * are ns for q >= ns, so they index the same samples). */
+ * additions); a lane's further ones in the column take it inline.  The test is
+ * k_migrate's: one threshold per trace, at the largest q of its samples in
+ * the column, for G slots at a time.
+ * FASTIDX: the index floor(min(q, ns + lane + 1/2)) of the fast form alone,
+ * the transpose of k_migrate's FASTIDX variant (floor(min(q, ns)) there: both
+ * are >= ns for q >= ns, so they index the same samples).
+ * Few traces (fewer than DM_TARGET_WGS workgroups) leave the chip idle:
+ * gridDim.y parts then take every gridDim.y-th column of a group's box each,
+ * add their sums into gsum (integers: in any order) and k_demig_finish forms
+ * the traces.
+ * Bound by VALU issue like k_migrate, the image samples' conversion to fixed
+ * point and the gates shared by the traces of a column.  48,000 traces x 1501
+ * samples, 1600 columns: 23.0 -> 18.9 ms against a test, a branch and a
+ * quarter-rate floor per slot and addresses formed anew for every column;
+ * 3001 traces x 751 of a wide-azimuth patch of 61 x 61 columns, relaxed
+ * index: 25.7 -> 3.0 ms, by the words past the trace and the column parts. */
 template <int K, int W, bool FASTIDX>
 __global__ void __launch_bounds__(8 * KTM_WAVE) __attribute__((amdgpu_waves_per_eu(4, 4)))
 k_demigrate(const DemigArgs a)
 {
     constexpr int NCOL = 8 / W;
-    extern __shared__ unsigned long long sg[];     /* [tb][ns + 4] fixed point */
+    constexpr int G = K % 3 ? 4 : 3;               /* slots side by side */
+    extern __shared__ unsigned long long sg[];     /* [tb][ns + DM_PAD] fixed point */
     __shared__ int32_t sIdx[DM_TB];
-    const int tid = threadIdx.x, lane = tid & (KTM_WAVE - 1), wv = tid / KTM_WAVE;
+    const int tid = threadIdx.x, lane = tid & (KTM_WAVE - 1);
+    const int wv = __builtin_amdgcn_readfirstlane(tid / KTM_WAVE);
     const int cw = wv / W, seg = wv % W;
-    const int ns = a.ns, ldg = ns + 4;
+    const int ns = a.ns, ldg = ns + DM_PAD;
     const int64_t b0 = (int64_t)blockIdx.x * a.tb;
     const int nb = (int)min((int64_t)a.tb, a.ntr - b0);
     for (int e = tid; e < a.tb * ldg; e += 8 * KTM_WAVE) sg[e] = 0ull;
-    const float amax = __uint_as_float(*a.amax);
-    int emax = 0;                          /* max |km| < 2^emax */
-    if (amax > 0.0f) (void)frexpf(amax, &emax);
-    const int E = 59 - emax - a.lg_terms;
+    const int E = demig_exponent(a);
     /* lane j < nb of every wave holds trace j of the workgroup */
     ktm_trace_geom g;
     memset(&g, 0, sizeof g);
@@ -1662,7 +1747,7 @@ k_demigrate(const DemigArgs a)
     int gi = 0;
     int xlo = a.nxp, xhi = -1, ylo = a.nyp, yhi = -1;
     if (lane < nb) {
-        gi = a.order ? a.order[b0 + lane] : (int)(b0 + lane);
+        gi = a.order[b0 + lane];
         g = a.geom[gi];
         valid = g.off >= 0 && g.off < a.nh;
         if (valid) {
@@ -1677,25 +1762,31 @@ k_demigrate(const DemigArgs a)
         ylo = min(ylo, __shfl_xor(ylo, m));
         yhi = max(yhi, __shfl_xor(yhi, m));
     }
+    xlo = __builtin_amdgcn_readfirstlane(xlo); xhi = __builtin_amdgcn_readfirstlane(xhi);
+    ylo = __builtin_amdgcn_readfirstlane(ylo); yhi = __builtin_amdgcn_readfirstlane(yhi);
     __syncthreads();
-    const float nsh = (float)ns + 0.5f;   /* clamp of q */
-    int rot = lane % K;
-    const int tbase = seg * K * KTM_WAVE + lane * K;
+    const float qlim = (float)(ns + lane) + 0.5f;  /* clamp of q */
+    constexpr int P = K == 8 ? 4 : 8;
+    const int rot = lane / P % K, tbase = seg * K * KTM_WAVE + lane * K;
     auto slot_t = [&](int k) __attribute__((always_inline)) {   /* sample of slot k */
         return tbase + (k + rot < K ? k + rot : k + rot - K);
     };
-    /* past the trace, tq puts q at ns + 1: clamped to ns + 0.5, T = ns, no add */
-    const float tq_past = 0.25f * ((float)ns + 1.0f) * ((float)ns + 1.0f);
+    /* past the end, tq puts q beyond every clamp */
+    const float tq_past = 0.25f * (float)(ns + 2 * KTM_WAVE) * (float)(ns + 2 * KTM_WAVE);
     float tq[K];
+    uint32_t to[K];                                /* the slot's sample, at most ns - 1 */
 #pragma unroll
     for (int k = 0; k < K; ++k) {
         const int t = slot_t(k);
         tq[k] = t < ns ? fast_tq(t) : tq_past;
+        to[k] = (uint32_t)min(t, ns - 1);
     }
+    const float tq_max = fast_tq(min(ns, (seg + 1) * K * KTM_WAVE) - 1);
     const int nbx = xhi - xlo + 1, nby = yhi - ylo + 1;
-    const int64_t ncols = nbx > 0 && nby > 0 ? (int64_t)nbx * nby : 0;
-    for (int64_t cidx = cw; cidx < ncols; cidx += NCOL) {
-        const int X = xlo + (int)(cidx / nby), Y = ylo + (int)(cidx % nby);
+    const int ncols = nbx > 0 && nby > 0 ? nbx * nby : 0;
+    const int cstep = NCOL * (int)gridDim.y;
+    for (int cidx = cw + NCOL * (int)blockIdx.y; cidx < ncols; cidx += cstep) {
+        const int X = xlo + cidx / nby, Y = ylo + cidx % nby;
         const float IX = a.colx[X], IY = a.coly[Y];
         const int job = (X / a.nx) * a.jobs_y + (Y / a.ny);
         float g_is = 0.0f, g_ir = 0.0f;
@@ -1710,62 +1801,91 @@ k_demigrate(const DemigArgs a)
         }
         uint64_t pm = __ballot(gp);
         if (!pm) continue;
-        /* the slot samples and their addresses are recomputed where used
-         * rather than held in registers across the loops (an empty asm
-         * hides that rot is loop-invariant) */
-        asm volatile("" : "+v"(rot));
         const int64_t pixc = ((int64_t)X * a.nyp + Y) * ns;
+        const float *rc = a.prs + pixc;
         float rs[K];
-        long long mq[K];                   /* km samples, fixed point */
+        unsigned long long mq[K];          /* km samples, fixed point */
 #pragma unroll
         for (int k = 0; k < K; ++k) {
-            const int t = slot_t(k);
-            rs[k] = t < ns ? a.prs[pixc + t] : 0.0f;
-            mq[k] = 0;
+            rs[k] = rc[to[k]];
+            mq[k] = 0ull;
+        }
+        float g_thr = 0.0f;                /* lane j: trace j's ambiguity threshold */
+        if (!FASTIDX) {
+            float m = rs[0];
+#pragma unroll
+            for (int k = 1; k < K; ++k) m = fmaxf(m, rs[k]);
+            g_thr = ambiguous_from(fminf(fast_qs(g_is, g_ir, wave_max(m), tq_max) * 1.00001f,
+                                         (float)ns + 1.0f));
         }
         int cur = -1;                      /* offset class whose samples mq holds */
         /* one ambiguous sample per lane deferred to the end of the column:
          * its slot | trace << 8 (-1: none) and its fixed-point value */
         int qkj = -1;
-        long long qv = 0;
+        unsigned long long qv = 0;
         while (pm) {
             const int j = __builtin_ctzll(pm);
             pm &= pm - 1ull;
             const float dIS2 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(g_is), j));
             const float dIR2 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(g_ir), j));
             const int offj = __builtin_amdgcn_readlane(g.off, j);
-            asm volatile("" : "+v"(rot));
             if (offj != cur) {
                 cur = offj;
                 const float *mk = a.km + (((int64_t)X * a.nyp + Y) * a.nh + offj) * ns;
+                float m[K];
+#pragma unroll
+                for (int k = 0; k < K; ++k) m[k] = mk[to[k]];
+#pragma unroll
+                for (int k = 0; k < K; ++k) mq[k] = to_fixed(m[k], E);
+            }
+            const uint32_t gl = (uint32_t)(uintptr_t)(lds_u64 *)(sg + j * ldg);
+            if (FASTIDX) {
 #pragma unroll
                 for (int k = 0; k < K; ++k) {
-                    const int t = slot_t(k);
-                    mq[k] = t < ns ? (long long)ldexpf(mk[t], E) : 0;
+                    const float qc = fast_clamp(fast_qs(dIS2, dIR2, rs[k], tq[k]), qlim);
+                    lds_add(((uint32_t)fast_T(qc) << 3) + gl, mq[k]);
                 }
+                continue;
             }
-            unsigned long long *gl = sg + j * ldg;
+            const float thr = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(g_thr), j));
 #pragma unroll
-            for (int k = 0; k < K; ++k) {
-                const float qc = fast_clamp(fast_qs(dIS2, dIR2, rs[k], tq[k]), nsh);
-                int T = fast_T(qc);
-                if (!FASTIDX && fast_ambiguous(qc, KTM_FAST_EPS_S)) {   /* never past the trace */
-                    if (qkj < 0) {
-                        /* deferred: the integer sums do not depend on the
-                         * order of their additions */
-                        qkj = k | (j << 8);
-                        qv = mq[k];
-                        T = ns;
-                    } else {
-                        const int t = slot_t(k);
-                        const float v2 = a.pv2[pixc + t];
-                        T = exact_T(dIS2, dIR2, a.t2[t], v2, 1.0f / v2, a.dt, a.rdt, ns);
+            for (int k = 0; k < K; k += G) {
+                uint32_t ad[G];
+                float dev[G], far = 0.0f;
+#pragma unroll
+                for (int i = 0; i < G; ++i) {
+                    const float qc = fast_clamp(fast_qs(dIS2, dIR2, rs[k + i], tq[k + i]), qlim);
+                    /* floor_p's rounding, on q itself; t = 0 is in slot 0 */
+                    float M = qc + KTM_FLOOR_MAGIC;
+                    if (k + i == 0) M = fmaxf(M, 8388608.0f);
+                    dev[i] = qc - (M - KTM_FLOOR_MAGIC);
+                    ad[i] = (__float_as_uint(M) << 3) + (gl - 8u * KTM_FLOOR_BITS);
+                    far = i ? fmaxf(far, fabsf(dev[i])) : fabsf(dev[i]);
+                }
+                if (far >= thr) {
+#pragma unroll
+                    for (int i = 0; i < G; ++i) {
+                        if (!(fabsf(dev[i]) >= thr)) continue;
+                        int T = ns + lane;
+                        if (qkj < 0) {
+                            /* deferred: the integer sums do not depend on the
+                             * order of their additions */
+                            qkj = (k + i) | (j << 8);
+                            qv = mq[k + i];
+                        } else {
+                            /* (hidden, so that the compiler does not hold
+                             * every slot's addresses in registers) */
+                            uint32_t t = to[k + i];
+                            asm volatile("" : "+v"(t));
+                            const float v2 = a.pv2[pixc + t];
+                            const int Te = exact_T(dIS2, dIR2, a.t2[t], v2, 1.0f / v2, a.dt, a.rdt, ns);
+                            if (Te < ns && tq[k + i] != tq_past) T = Te;
+                        }
+                        ad[i] = ((uint32_t)T << 3) + gl;
                     }
                 }
-                /* T = ns (past the trace, or deferred) adds into the pad
-                 * g[ns], which the transpose below never reads: no compare
-                 * and no branch per slot */
-                atomicAdd(&gl[T], (unsigned long long)mq[k]);
+#pragma unroll
+                for (int i = 0; i < G; ++i) lds_add(ad[i], mq[k + i]);
             }
         }
         if (!FASTIDX && __ballot(qkj >= 0)) {
@@ -1777,35 +1897,46 @@ k_demigrate(const DemigArgs a)
             const float dIS2 = __shfl(g_is, jq), dIR2 = __shfl(g_ir, jq);
             if (qkj >= 0) {
                 const int t = slot_t(qkj & 0xff);
-                const float v2 = a.pv2[pixc + t];
-                const int T = exact_T(dIS2, dIR2, a.t2[t], v2, 1.0f / v2, a.dt, a.rdt, ns);
-                if (T < ns) atomicAdd(&sg[jq * ldg + T], (unsigned long long)qv);
+                if (t < ns) {
+                    const float v2 = a.pv2[pixc + t];
+                    const int T = exact_T(dIS2, dIR2, a.t2[t], v2, 1.0f / v2, a.dt, a.rdt, ns);
+                    if (T < ns) atomicAdd(&sg[jq * ldg + T], qv);
+                }
             }
         }
     }
     __syncthreads();
-    /* transpose of F = closed_tap(x), x[t] = tr[min(t, ns-1)] * w[t], in
-     * double from the fixed-point sums */
+    if (gridDim.y > 1) {
+        for (int e = tid; e < nb * ns; e += 8 * KTM_WAVE) {
+            const int j = e / ns, t = e - j * ns;
+            const unsigned long long v = sg[j * ldg + t];
+            if (v) atomicAdd(a.gsum + (int64_t)sIdx[j] * ns + t, v);
+        }
+        return;
+    }
     const double q = ldexp(1.0, -E);
     for (int e = tid; e < nb * ns; e += 8 * KTM_WAVE) {
         const int j = e / ns, t = e - j * ns;
-        const long long *gl = reinterpret_cast<const long long *>(sg + j * ldg);
-        double acc = 0.0;
-        const int nt_ = t == ns - 1 ? 3 : 1;   /* tr[ns-1] also feeds x[ns], x[ns+1] */
-        for (int u = 0; u < nt_; ++u) {
-            const int tt = t + u;
-            long long xb = 0;                  /* exact: |g| < 2^59, weights summing to <= 6 */
-            if (tt >= 2 && tt < ns) xb += gl[tt];
-            if (tt - 1 >= 2 && tt - 1 < ns) xb += 2 * gl[tt - 1];
-            if (tt - 2 >= 2 && tt - 2 < ns) xb += gl[tt - 2];
-            if (tt == 0) xb += 4 * gl[0] + 2 * gl[1];
-            if (tt == 1) xb += 4 * gl[0] + 2 * gl[1];
-            if (tt == 2) xb += 2 * gl[0] + 2 * gl[1];
-            if (tt == 3) xb += gl[1];
-            acc += (double)a.w[tt] * ((double)xb * q);
-        }
-        a.traces[(int64_t)sIdx[j] * ns + t] = (float)acc;
+        a.traces[(int64_t)sIdx[j] * ns + t] =
+            demig_sample(reinterpret_cast<const long long *>(sg + j * ldg), t, ns, a.w, q);
     }
+}
+
+/* the traces of a demigration whose columns were taken in parts: one
+ * workgroup per trace */
+__global__ void __launch_bounds__(256) k_demig_finish(const DemigArgs a)
+{
+    const double q = ldexp(1.0, -demig_exponent(a));
+    const int64_t o = (int64_t)blockIdx.x * a.ns;
+    for (int t = threadIdx.x; t < a.ns; t += 256)
+        a.traces[o + t] = demig_sample(reinterpret_cast<const long long *>(a.gsum + o), t, a.ns, a.w, q);
+}
+
+__global__ void k_zero_u64(unsigned long long *p, int64_t n)
+{
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+         i += (int64_t)gridDim.x * blockDim.x)
+        p[i] = 0ull;
 }
 
 /* Transpose of the post-stack chain image = P0 H C D km of Kirchhoff.c:
@@ -1885,7 +2016,7 @@ extern "C" void ktm_plan_destroy(ktm_plan *p)
     void *bufs[] = {p->d_t2, p->d_t1, p->d_colx, p->d_coly, p->d_velx, p->d_vely,
                     p->d_slab_cx, p->d_slab_cy, p->d_slab_x2thr, p->d_vel2, p->d_w, p->d_hconv2,
                     p->d_stage, p->d_pix_v2, p->d_pix_rs, p->d_dm_keys, p->d_dm_idx,
-                    p->d_dm_tmp, p->d_dm_amax, p->d_parts, p->d_pf_g, p->d_pf_tw};
+                    p->d_dm_tmp, p->d_dm_amax, p->d_dm_sum, p->d_parts, p->d_pf_g, p->d_pf_tw};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
     ktm_tables_free(&p->tb);
@@ -2782,6 +2913,13 @@ static int demig_order(const ktm_plan *cp, const ktm_trace_geom *geom, int64_t n
     return KTM_OK;
 }
 
+/* Workgroups below which a demigration takes its columns in parts (four rounds
+ * of the 512 that run at once), the parts at most, and the bound of its
+ * workspace (256 MiB) */
+#define DM_TARGET_WGS 2048
+#define DM_MAX_PARTS 16
+#define DM_SUM_MAX_WORDS (32ll << 20)
+
 static int demigrate(const ktm_plan *p, const float *km, const ktm_trace_geom *geom, int64_t ntr,
                      float *traces, bool fast, void *stream);
 
@@ -2833,7 +2971,7 @@ static int demigrate(const ktm_plan *p, const float *km, const ktm_trace_geom *g
     hipLaunchKernelGGL(k_absmax, dim3(1024), dim3(256), 0, hs, km, nimg, p->d_dm_amax);
     /* traces per workgroup: DM_TB, fewer so that two workgroups share a CU
      * (g rows of 8 bytes per sample within 76 KB), or one beyond that */
-    const size_t row = sizeof(unsigned long long) * (size_t)(s->ns + 4);
+    const size_t row = sizeof(unsigned long long) * (size_t)(s->ns + DM_PAD);
     a.tb = (int)((76 * 1024) / row);
     if (a.tb < 2) a.tb = (int)((152 * 1024) / row);
     if (a.tb > DM_TB) a.tb = DM_TB;
@@ -2857,7 +2995,29 @@ static int demigrate(const ktm_plan *p, const float *km, const ktm_trace_geom *g
         b.ntr = n;
         if ((st = demig_order(p, b.geom, n, hs, &b.order)) != KTM_OK) return st;
         const int64_t nblk = (n + a.tb - 1) / a.tb;
-        hipLaunchKernelGGL(fn, dim3((unsigned)nblk), dim3(8 * KTM_WAVE), lds, hs, b);
+        /* few traces: their columns in parts, up to what a bounded workspace
+         * of sums allows */
+        const int64_t words = n * s->ns;
+        int64_t parts = (DM_TARGET_WGS + nblk - 1) / nblk;
+        if (parts > DM_MAX_PARTS) parts = DM_MAX_PARTS;
+        if (words > DM_SUM_MAX_WORDS) parts = 1;
+        if (parts > 1) {
+            ktm_plan *pm = const_cast<ktm_plan *>(p);
+            if ((size_t)words > p->dm_sum_cap) {
+                if (p->d_dm_sum) HIP_TRY(hipFree(p->d_dm_sum));
+                pm->d_dm_sum = nullptr;
+                pm->dm_sum_cap = 0;
+                if (hipMalloc((void **)&pm->d_dm_sum, (size_t)words * sizeof(unsigned long long)) !=
+                    hipSuccess)
+                    return KTM_ERR_NOMEM;
+                pm->dm_sum_cap = (size_t)words;
+            }
+            b.gsum = p->d_dm_sum;
+            hipLaunchKernelGGL(k_zero_u64, dim3(2048), dim3(256), 0, hs, b.gsum, words);
+        }
+        hipLaunchKernelGGL(fn, dim3((unsigned)nblk, (unsigned)parts), dim3(8 * KTM_WAVE), lds, hs, b);
+        if (parts > 1)
+            hipLaunchKernelGGL(k_demig_finish, dim3((unsigned)n), dim3(256), 0, hs, b);
     }
     HIP_TRY(hipGetLastError());
     return KTM_OK;

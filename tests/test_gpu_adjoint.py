@@ -201,3 +201,24 @@ def test_demigration_deterministic_and_scale_exact(cuda):
     assert float(a.abs().max()) > 0.0
     for s in (2.0 ** 40, 2.0 ** -40):
         assert torch.equal(plan.demigrate(m * s, geom), a * s)
+
+
+@pytest.mark.parametrize("fast", [False, True])
+@pytest.mark.parametrize("ns,take", [(4, 1), (301, 9), (700, 130), (1501, 1000), (3001, 65)])
+def test_demigration_of_few_traces_bitexact(cuda, ns, take, fast):
+    """Few traces have their columns taken in parts whose integer sums are
+    added in any order: the same bits as among enough traces to fill the chip
+    undivided, with traces past the classes and far past the image among
+    them."""
+    print(f"case: {take} of 17,000 traces x {ns} samples", flush=True)
+    sv = surveys.line2d(nshots=850, nrecv_side=10, shot_dx=0.5, ns=ns, ncols=30, nscat=2,
+                        x0=130.0, dh=105.0, t0_range=(0.01, 0.02))
+    plan = Plan(sv.cfg, sv.ns, sv.dt, sv.vel)
+    g = torch.Generator(device=cuda).manual_seed(ns)
+    m = torch.randn(plan.image_shape, generator=g, device=cuda)
+    geom = plan.geometry(torch.from_numpy(sv.coords).to(cuda))
+    want = plan.demigrate(m, geom, fast=fast)
+    at = torch.randperm(sv.ntr, generator=g, device=cuda)[:take]
+    got = plan.demigrate(m, geom[at].contiguous(), fast=fast)
+    assert bool(want.any())
+    assert torch.equal(got, want[at])
