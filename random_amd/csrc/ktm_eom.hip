@@ -296,6 +296,40 @@ __global__ void k_eom_geometry(const EomGeoArgs a, const int32_t *__restrict__ c
     geo[i] = make_float4(h2, cmpX, cmpY, (float)ta);   /* talpha: an integer, exact in float */
 }
 
+/* The taper of EOM.c:1290-1292, (float)(0.5 + atan(200 d / 0.080) / EOM_PI) in
+ * double for the float d.  Away from its centre (|z| = 2500 |d| >= 8, i.e.
+ * everywhere but within 3.2 ms of it) atan(z) = +-pi/2 - atan(1/z), the latter
+ * a polynomial in w = 1/z, |w| <= 1/8: terms to w^13 leave w^15/15 <= 1.9e-15.
+ * The sum v is within 6.1e-16 of the exact value (measured over 4e6 d of
+ * either sign), the reference's double expression (atan to one ulp, a division
+ * and a sum) within 6e-16; where v - E and v + E, E = 2e-15, round to the same
+ * float, that float is the reference's.  Otherwise (6e-4 of the samples, the
+ * smallest values) and near the centre the expression itself decides.  16 FP64 instructions
+ * where the full atan and a division by 0.08 took about 100: see
+ * k_eom_accum. */
+__device__ __forceinline__ float eom_taper(float df)
+{
+    constexpr double PI_L = 3.14159265358979323846, HALF = 0.5 * PI_L / EOM_PI;
+    constexpr double E = 2.0e-15, RPI = 1.0 / EOM_PI;
+    const double d = (double)df;
+    double y = __builtin_amdgcn_rcp(d);
+    y = __builtin_fma(__builtin_fma(-d, y, 1.0), y, y);
+    y = __builtin_fma(__builtin_fma(-d, y, 1.0), y, y);
+    const double w = 4.0e-4 * y, x = w * w;                   /* 0.080 / 200 / d */
+    double p = __builtin_fma(x, 1.0 / 13.0, -1.0 / 11.0);
+    p = __builtin_fma(x, p, 1.0 / 9.0);
+    p = __builtin_fma(x, p, -1.0 / 7.0);
+    p = __builtin_fma(x, p, 1.0 / 5.0);
+    p = __builtin_fma(x, p, -1.0 / 3.0);
+    p = __builtin_fma(x, p, 1.0);
+    const double v = __builtin_fma(-(w * RPI), p, df > 0.0f ? 0.5 + HALF : 0.5 - HALF);
+    const float lo = (float)(v - E), hi = (float)(v + E);
+    if (fabsf(df) >= 0.0032f && lo == hi) return lo;
+    constexpr double R008 = 1.0 / 0.080;
+    const double z = div_cr(200.0 * d, 0.080, R008);
+    return (float)(0.5 + div_cr(atan(z), EOM_PI, RPI));
+}
+
 struct EomArgs {
     const float *traces;          /* [ntr][ns] */
     const float4 *geo;            /* [ntr] h2, cmpX, cmpY, talpha */
@@ -311,7 +345,8 @@ struct EomArgs {
     int cx0, cy0, nyl;            /* gather array: CSP (cx0, cy0) first, nyl per X */
 };
 
-__global__ void __launch_bounds__(EOM_NT) k_eom_accum(const EomArgs a)
+__global__ void __launch_bounds__(EOM_NT) __attribute__((amdgpu_waves_per_eu(5)))
+k_eom_accum(const EomArgs a)
 {
     /* per passing trace: 4 x2 h2 (exact in double) and RN(x2 + h2), the
      * trace-only terms of EOM.c:1285-1286 */
@@ -342,7 +377,6 @@ __global__ void __launch_bounds__(EOM_NT) k_eom_accum(const EomArgs a)
      * quotients are those of the reference's double divisions */
     const double rden0 = 1.0 / (double)den0;   /* +inf at t = 0: NaN offset, as 0-divides */
     const double rsvt = 1.0 / svt, rdh = 1.0 / a.dh;
-    constexpr double R008 = 1.0 / 0.080, RPI = 1.0 / EOM_PI;
     const float t2dt = a.t2d[tc];
     const float rt2d = 1.0f / t2dt;   /* t = 0 never bins: its offset is NaN */
     const int64_t col_base = ((int64_t)(X - a.cx0) * a.nyl + (Y - a.cy0)) * a.nh;
@@ -400,8 +434,7 @@ __global__ void __launch_bounds__(EOM_NT) k_eom_accum(const EomArgs a)
             if (!(fl >= 0.0 && fl < (double)(a.nh - 1))) continue;
             const int off = (int)fl;
             const float tcv = (float)div_cr(2.25 * (double)eq, svt, rsvt);
-            const double z = div_cr(200.0 * (double)(tdt - tcv), 0.080, R008);
-            const float s3 = (float)(0.5 + div_cr(atan(z), EOM_PI, RPI));
+            const float s3 = eom_taper(tdt - tcv);
             const float s2 = (float)(qo - (double)off);
             const float s1 = (float)(1.0 - (double)s2);
             const float x = a.traces[(c0 + sIdx[j]) * a.ns + t];
