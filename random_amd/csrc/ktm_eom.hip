@@ -14,12 +14,12 @@
  *
  * k_eom_geometry: per trace h2, CMP and talpha with the reference's float and
  *   double promotions (EOM.c:1245-1272).
- * k_eom_accum: one workgroup = one CSP x one segment of 256 samples, one lane
+ * k_eom_accum: one workgroup = one CSP x one segment of 64 samples, one lane
  *   per sample.  The lane owns its sample of every offset bin of its CSP for
  *   the whole launch, so it adds into the gather without atomics and in trace
  *   order (the reference's order of additions per bin); the two bins of the
  *   latest trace stay in registers until another trace needs their slot.
- *   Traces stream in chunks of 256: the aperture gate of each is evaluated
+ *   Traces stream in chunks of 64: the aperture gate of each is evaluated
  *   lane-parallel, the passing ones are compacted in order through LDS.
  * k_postfft<PostEom> (ktm_postfft.h; k_postmx<PostEom> of ktm_postmx.h on
  *   the matrix cores beyond 4096 samples): the post filter as a real
@@ -44,8 +44,8 @@
 #include "ktm_postmx.h"
 #include "ktm_postfft.h"
 
-#define EOM_NT 256
-#define EOM_RUN 16     /* consecutive tiles per XCD run */
+#define EOM_NT 64      /* samples (and lanes) of a workgroup: one wave */
+#define EOM_RUN 64     /* consecutive tiles per XCD run */
 #define EOM_WAVE 64
 #define EOM_PI 3.14159265359 /* EOM.c:124 */
 
@@ -300,20 +300,20 @@ __global__ void k_eom_geometry(const EomGeoArgs a, const int32_t *__restrict__ c
  * double for the float d.  Away from its centre (|z| = 2500 |d| >= 8, i.e.
  * everywhere but within 3.2 ms of it) atan(z) = +-pi/2 - atan(1/z), the latter
  * a polynomial in w = 1/z, |w| <= 1/8: terms to w^13 leave w^15/15 <= 1.9e-15.
- * The sum v is within 6.1e-16 of the exact value (measured over 4e6 d of
- * either sign), the reference's double expression (atan to one ulp, a division
- * and a sum) within 6e-16; where v - E and v + E, E = 2e-15, round to the same
- * float, that float is the reference's.  Otherwise (6e-4 of the samples, the
- * smallest values) and near the centre the expression itself decides.  16 FP64 instructions
+ * The sum v is within 1.2e-15 of the exact value (1.4e-14 / (8 pi) from the
+ * reciprocal, 6.1e-16 measured over 4e6 d of either sign from the rest), the
+ * reference's double expression (atan to one ulp, a division and a sum) within
+ * 6e-16; where v - E and v + E, E = 2.5e-15, round to the same float, that
+ * float is the reference's.  Otherwise (8e-4 of the samples, the smallest
+ * values) and near the centre the expression itself decides.  16 FP64 instructions
  * where the full atan and a division by 0.08 took about 100: see
  * k_eom_accum. */
 __device__ __forceinline__ float eom_taper(float df)
 {
     constexpr double PI_L = 3.14159265358979323846, HALF = 0.5 * PI_L / EOM_PI;
-    constexpr double E = 2.0e-15, RPI = 1.0 / EOM_PI;
+    constexpr double E = 2.5e-15, RPI = 1.0 / EOM_PI;
     const double d = (double)df;
-    double y = __builtin_amdgcn_rcp(d);
-    y = __builtin_fma(__builtin_fma(-d, y, 1.0), y, y);
+    double y = (double)__builtin_amdgcn_rcpf(df);             /* one Newton step: 1.4e-14 */
     y = __builtin_fma(__builtin_fma(-d, y, 1.0), y, y);
     const double w = 4.0e-4 * y, x = w * w;                   /* 0.080 / 200 / d */
     double p = __builtin_fma(x, 1.0 / 13.0, -1.0 / 11.0);
@@ -328,6 +328,19 @@ __device__ __forceinline__ float eom_taper(float df)
     constexpr double R008 = 1.0 / 0.080;
     const double z = div_cr(200.0 * d, 0.080, R008);
     return (float)(0.5 + div_cr(atan(z), EOM_PI, RPI));
+}
+
+/* RN(sqrt(x)), x >= 0: v_sqrt_f32 to one ulp and the two tests of its
+ * neighbours, without the scaling of subnormal radicands unless a lane has
+ * one below 2^-96 */
+__device__ __forceinline__ float sqrt_rn(float x)
+{
+    if (__ballot(x < 0x1p-96f && x > 0.0f)) return __builtin_sqrtf(x);
+    const float s = __builtin_amdgcn_sqrtf(x);
+    const float dn = __uint_as_float(__float_as_uint(s) - 1u);
+    const float up = __uint_as_float(__float_as_uint(s) + 1u);
+    const float r = __builtin_fmaf(-dn, s, x) <= 0.0f ? dn : s;
+    return __builtin_fmaf(-up, s, x) > 0.0f ? up : r;
 }
 
 struct EomArgs {
@@ -345,7 +358,18 @@ struct EomArgs {
     int cx0, cy0, nyl;            /* gather array: CSP (cx0, cy0) first, nyl per X */
 };
 
-__global__ void __launch_bounds__(EOM_NT) __attribute__((amdgpu_waves_per_eu(5)))
+/* WIDE: a CSP's gathers have 2^30 samples or more (or 2^24 bins, or 2^22
+ * samples a bin), whose bins need 64-bit offsets.
+ * Bound by the gathers' traffic: a lane moves to the next bin every other
+ * trace (a store and a load of both arrays, 51 GB on the 40-shot line, 4 TB/s;
+ * the bins a wave returns to with the next shot, 82 KB, do not fit the L2 at
+ * any useful occupancy).  Four waves per SIMD measured faster than five or
+ * six (fewer gathers in flight to evict each other), and workgroups of one
+ * wave than of four (no barrier, and the segments' unequal counts even out):
+ * 14.8 -> 12.2 ms with 7.5e9 -> 5.1e9 VALU instructions, the sample of the
+ * next trace loaded ahead and the bins before the taper. */
+template <bool WIDE>
+__global__ void __launch_bounds__(EOM_NT) __attribute__((amdgpu_waves_per_eu(4)))
 k_eom_accum(const EomArgs a)
 {
     /* per passing trace: 4 x2 h2 (exact in double) and RN(x2 + h2), the
@@ -379,13 +403,22 @@ k_eom_accum(const EomArgs a)
     const double rsvt = 1.0 / svt, rdh = 1.0 / a.dh;
     const float t2dt = a.t2d[tc];
     const float rt2d = 1.0f / t2dt;   /* t = 0 never bins: its offset is NaN */
-    const int64_t col_base = ((int64_t)(X - a.cx0) * a.nyl + (Y - a.cy0)) * a.nh;
+    /* the CSP's gathers, and the byte offset of the lane's sample of bin b */
+    const int64_t col_base = ((int64_t)(X - a.cx0) * a.nyl + (Y - a.cy0)) * a.nh * a.ns;
+    char *csp = reinterpret_cast<char *>(a.csp + col_base);
+    char *fold = reinterpret_cast<char *>(a.fold + col_base);
+    const uint32_t ns4 = 4u * (uint32_t)a.ns, t4 = 4u * (uint32_t)t;
+    auto bin_at = [&](int b) __attribute__((always_inline)) {
+        if constexpr (WIDE) return (uint64_t)ns4 * (uint64_t)b + t4;
+        else return __umul24((uint32_t)b, ns4) + t4;
+    };
+    auto at = [](char *p, auto o) __attribute__((always_inline)) { return reinterpret_cast<float *>(p + o); };
     uint64_t nev = 0;
     /* the lane's sample of two offset bins, held in registers between traces */
     int tagE = -1, tagO = -1;
     float cE = 0.0f, fE = 0.0f, cO = 0.0f, fO = 0.0f;
     for (int64_t c0 = 0; c0 < a.ntr; c0 += EOM_NT) {
-        /* ---- aperture gate of EOM.c:1268-1270 for 256 traces, in order ---- */
+        /* ---- aperture gate of EOM.c:1268-1270 for 64 traces, in order ---- */
         const int64_t i = c0 + tid;
         bool pass = false;
         float x2 = 0.0f, h2 = 0.0f;
@@ -415,7 +448,16 @@ k_eom_accum(const EomArgs a)
             sIdx[base + pre] = tid;
         }
         __syncthreads();
+        /* the lane's sample of trace j + 1 is loaded while trace j is binned */
+        const int tc32 = tin ? t : 0;
+        auto sample = [&](int j) __attribute__((always_inline)) {
+            const float *row = a.traces + (c0 + __builtin_amdgcn_readfirstlane(sIdx[j])) * a.ns;
+            return row[(uint32_t)tc32];
+        };
+        float xnext = total ? sample(0) : 0.0f;
         for (int j = 0; j < total; ++j) {
+            const float x = xnext;
+            xnext = sample(j + 1 < total ? j + 1 : j);
             const int taj = sTa[j];
             const bool live = tin && t >= taj;
             nev += __popcll(__ballot(live));
@@ -427,18 +469,12 @@ k_eom_accum(const EomArgs a)
             /* (float)sqrt((double)arg) of the reference: the double square
              * root of a float, rounded to float, is the correctly rounded
              * float square root (double rounding is innocuous for sqrt when
-             * 53 >= 2 x 24 + 2), which __builtin_sqrtf is without fast-math */
-            const float eq = __builtin_sqrtf(arg);
+             * 53 >= 2 x 24 + 2) */
+            const float eq = sqrt_rn(arg);
             const double qo = div_cr((double)(eq - (float)a.oh), a.dh, rdh);
             const double fl = floor(qo);
             if (!(fl >= 0.0 && fl < (double)(a.nh - 1))) continue;
             const int off = (int)fl;
-            const float tcv = (float)div_cr(2.25 * (double)eq, svt, rsvt);
-            const float s3 = eom_taper(tdt - tcv);
-            const float s2 = (float)(qo - (double)off);
-            const float s1 = (float)(1.0 - (double)s2);
-            const float x = a.traces[(c0 + sIdx[j]) * a.ns + t];
-            const float v1 = div_cr(s1 * s3 * x, t2dt, rt2d), v2 = div_cr(s2 * s3 * x, t2dt, rt2d);
             /* bins off and off+1 have opposite parity: the even one goes to
              * slot E, the odd one to slot O; a slot that holds another bin
              * is written back and refilled, so every bin lives in exactly
@@ -447,26 +483,31 @@ k_eom_accum(const EomArgs a)
             const int be = ev ? off : off + 1, bo = ev ? off + 1 : off;
             if (tagE != be) {
                 if (tagE >= 0) {
-                    const int64_t w = (col_base + tagE) * a.ns + t;
-                    a.csp[w] = cE;
-                    a.fold[w] = fE;
+                    const auto w = bin_at(tagE);
+                    *at(csp, w) = cE;
+                    *at(fold, w) = fE;
                 }
-                const int64_t r = (col_base + be) * a.ns + t;
-                cE = a.csp[r];
-                fE = a.fold[r];
+                const auto r = bin_at(be);
+                cE = *at(csp, r);
+                fE = *at(fold, r);
                 tagE = be;
             }
             if (tagO != bo) {
                 if (tagO >= 0) {
-                    const int64_t w = (col_base + tagO) * a.ns + t;
-                    a.csp[w] = cO;
-                    a.fold[w] = fO;
+                    const auto w = bin_at(tagO);
+                    *at(csp, w) = cO;
+                    *at(fold, w) = fO;
                 }
-                const int64_t r = (col_base + bo) * a.ns + t;
-                cO = a.csp[r];
-                fO = a.fold[r];
+                const auto r = bin_at(bo);
+                cO = *at(csp, r);
+                fO = *at(fold, r);
                 tagO = bo;
             }
+            const float tcv = (float)div_cr(2.25 * (double)eq, svt, rsvt);
+            const float s3 = eom_taper(tdt - tcv);
+            const float s2 = (float)(qo - fl);
+            const float s1 = (float)(1.0 - (double)s2);
+            const float v1 = div_cr(s1 * s3 * x, t2dt, rt2d), v2 = div_cr(s2 * s3 * x, t2dt, rt2d);
             cE = cE + (ev ? v1 : v2);
             fE = fE + 1.0f;
             cO = cO + (ev ? v2 : v1);
@@ -475,14 +516,12 @@ k_eom_accum(const EomArgs a)
         __syncthreads();
     }
     if (tagE >= 0) {
-        const int64_t w = (col_base + tagE) * a.ns + t;
-        a.csp[w] = cE;
-        a.fold[w] = fE;
+        *at(csp, bin_at(tagE)) = cE;
+        *at(fold, bin_at(tagE)) = fE;
     }
     if (tagO >= 0) {
-        const int64_t w = (col_base + tagO) * a.ns + t;
-        a.csp[w] = cO;
-        a.fold[w] = fO;
+        *at(csp, bin_at(tagO)) = cO;
+        *at(fold, bin_at(tagO)) = fO;
     }
     if (lane == 0 && a.counter) atomicAdd(a.counter, (unsigned long long)nev);
 }
@@ -565,7 +604,10 @@ static int eom_block(const ktm_eom_plan *cp, const float *traces, const int32_t 
     if (ntiles > 0x7fffff00LL) return KTM_ERR_UNSUPPORTED;
     const int64_t span = 8 * EOM_RUN;   /* tiles per round of runs over the 8 XCDs */
     const int64_t nblk = (ntiles + span - 1) / span * span;
-    hipLaunchKernelGGL(k_eom_accum, dim3((unsigned)nblk), dim3(EOM_NT), 0, st, a);
+    if ((int64_t)a.nh * a.ns >= (1 << 30) || a.nh >= (1 << 24) || a.ns >= (1 << 22))
+        hipLaunchKernelGGL(k_eom_accum<true>, dim3((unsigned)nblk), dim3(EOM_NT), 0, st, a);
+    else
+        hipLaunchKernelGGL(k_eom_accum<false>, dim3((unsigned)nblk), dim3(EOM_NT), 0, st, a);
     EOM_TRY(hipGetLastError());
     return KTM_OK;
 }
