@@ -2086,8 +2086,8 @@ extern "C" int ktm_plan_create(ktm_plan **out, const ktm_config *cfg, int ns, fl
         double *g = (double *)malloc(sizeof(double) * 4 * n);
         if (!g) st = KTM_ERR_NOMEM;
         if (st == KTM_OK) {
-            postfft_host_tables(tb->hconv, ns, p->pf_n, g, g + 2 * n);
-            st = upload(&p->d_pf_g, reinterpret_cast<const double2 *>(g), n);
+            if (postfft_host_tables(tb->hconv, ns, p->pf_n, g, g + 2 * n)) st = KTM_ERR_NOMEM;
+            if (st == KTM_OK) st = upload(&p->d_pf_g, reinterpret_cast<const double2 *>(g), n);
             if (st == KTM_OK) st = upload(&p->d_pf_tw, reinterpret_cast<const double2 *>(g + 2 * n), n);
         }
         free(g);

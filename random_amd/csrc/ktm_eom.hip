@@ -200,17 +200,8 @@ extern "C" int ktm_eom_plan_create(ktm_eom_plan **out, const ktm_eom_config *c, 
         /* g[m] = (1/ns) sum_k lowpass[k] rootrho[k] cos(2 pi k m / ns): the
          * spectrum is even (both factors are mirrored), so the filtered trace
          * is the circular convolution with g */
-        const long double two_pi = 2.0L * acosl(-1.0L);
-        for (int m = 0; m < ns; ++m) {
-            long double acc = 0.0L;
-            long long km = 0;
-            for (int k = 0; k < ns; ++k) {
-                acc += (long double)lp[k] * (long double)rr[k] * cosl(two_pi * km / ns);
-                km += m;
-                if (km >= ns) km -= ns;
-            }
-            g[m] = g[m + ns] = (double)(acc / ns);
-        }
+        st = ktm_even_kernel(lp, rr, ns, g) == KTM_OK ? st : KTM_ERR_NOMEM;
+        for (int m = 0; st != KTM_ERR_NOMEM && m < ns; ++m) g[m + ns] = g[m];
     }
     if (st == KTM_OK && hipGetDevice(&p->device) != hipSuccess) st = KTM_ERR_DEVICE;
     if (st == KTM_OK &&
@@ -234,8 +225,9 @@ extern "C" int ktm_eom_plan_create(ktm_eom_plan **out, const ktm_eom_config *c, 
         double *t = (double *)malloc(sizeof(double) * 4 * n);
         if (!t) st = KTM_ERR_NOMEM;
         if (st == KTM_OK) {
-            postfft_host_tables(g, ns, p->pf_n, t, t + 2 * n);
-            if (hipMalloc(&p->d_pf_g, sizeof(double2) * n) != hipSuccess ||
+            if (postfft_host_tables(g, ns, p->pf_n, t, t + 2 * n))
+                st = KTM_ERR_NOMEM;
+            else if (hipMalloc(&p->d_pf_g, sizeof(double2) * n) != hipSuccess ||
                 hipMalloc(&p->d_pf_tw, sizeof(double2) * n) != hipSuccess)
                 st = KTM_ERR_NOMEM;
             else if (hipMemcpy(p->d_pf_g, t, sizeof(double2) * n, hipMemcpyHostToDevice) != hipSuccess ||

@@ -295,7 +295,7 @@ static void free_bufs(dev_bufs *b)
  * the caller's arrays) while the DMA out of the other is in flight; each
  * chunk's event marks its copy done before the chunk is refilled.  For raw
  * SEG-Y records a chunk holds whole records, so the coordinate words of
- * each record are checked as it arrives. */
+ * each record are checked as it arrives.  Chunks are at most this large. */
 #define KTM_STAGE_BYTES ((size_t)64 << 20)
 
 typedef struct stage_ring {
@@ -314,6 +314,18 @@ static void ring_free(stage_ring *r)
         ktm_rt_pinned_free(r->buf[k]);
     }
     memset(r, 0, sizeof *r);
+}
+
+/* the chunk size for total bytes of units of rec: half of them, so that one
+ * chunk's copy runs while the other is filled, between 1 MiB and
+ * KTM_STAGE_BYTES, and a unit at least (pinning two 64 MiB chunks took longer
+ * than a small survey's migration) */
+static size_t stage_bytes(size_t total, size_t rec)
+{
+    size_t cap = total / 2 + rec;
+    if (cap < ((size_t)1 << 20)) cap = (size_t)1 << 20;
+    if (cap > KTM_STAGE_BYTES) cap = KTM_STAGE_BYTES;
+    return cap < rec ? rec : cap;
 }
 
 static int ring_init(stage_ring *r, size_t cap)
@@ -397,7 +409,7 @@ static int write_device_file(const char *name, const void *src, size_t bytes)
     if (!f) return KTM_ERR_IO;
     stage_ring ring;
     void *s = NULL;
-    int st = ring_init(&ring, KTM_STAGE_BYTES);
+    int st = ring_init(&ring, stage_bytes(bytes, 1));
     if (st == KTM_OK) st = ktm_rt_stream_create(&s);
     if (st == KTM_OK && bytes) st = ring_write(&ring, f, src, bytes, s);
     if (s && ktm_rt_stream_sync(s) != KTM_OK && st == KTM_OK) st = KTM_ERR_DEVICE;
@@ -443,7 +455,8 @@ static int run_survey(const ktm_plan *plan, const ktm_config *cfg, const char *p
     int st = KTM_OK;
     if (path && !(f = fopen(path, "rb"))) st = KTM_ERR_IO;
     if (st == KTM_OK)
-        st = ring_init(&ring, path && (size_t)rec > KTM_STAGE_BYTES ? (size_t)rec : KTM_STAGE_BYTES);
+        st = ring_init(&ring, path ? stage_bytes((size_t)(nb * rec), (size_t)rec)
+                                   : stage_bytes(sizeof(float) * (size_t)(nb * s.ns), 1));
     if (st == KTM_OK) st = ktm_rt_stream_create(&s_in);
     if (st == KTM_OK) st = ktm_rt_stream_create(&s_mig);
     if (st == KTM_OK && !(tev = (void **)calloc((size_t)(2 * nblocks + 1), sizeof(void *))))
@@ -814,7 +827,7 @@ static int eom_csp_job(int job_id)
     if (st == KTM_OK && nblocks > 0) {
         if (!(f = fopen(E.input_data, "rb"))) st = KTM_ERR_IO;
         if (st == KTM_OK)
-            st = ring_init(&ring, (size_t)rec > KTM_STAGE_BYTES ? (size_t)rec : KTM_STAGE_BYTES);
+            st = ring_init(&ring, stage_bytes((size_t)(nb * rec), (size_t)rec));
         if (st == KTM_OK) st = ktm_rt_stream_create(&s_in);
         if (st == KTM_OK) st = ktm_rt_stream_create(&s_bin);
         for (int k = 0; k < 2 && k < nblocks && st == KTM_OK; ++k) {

@@ -304,41 +304,10 @@ static inline int postfft_size(int ns)
     return 0;
 }
 
-/* Host tables of the FFT form for the kernel h[0..ns): G = DFT_N(g) and the
- * twiddles exp(-2 pi i m / N), m < N, each N double2 ({re, im}) into
- * caller arrays.  G in double: by an iterative radix-2 transform for a
- * power of two, directly (the sum over g's 2 ns - 1 nonzero points, angles
- * from the twiddle table) otherwise; twiddles from cos/sin of the exact
- * angle. */
-static inline void postfft_host_tables(const double *h, int ns, int n, double *G, double *tw)
+/* in-place DFT of n (a power of two) complex doubles, twiddles
+ * exp(-2 pi i q / n) = tw[q step]: bit reversal, then log2 n butterfly stages */
+static inline void postfft_host_fft(double *G, int n, const double *tw, int step)
 {
-    const double two_pi = 6.283185307179586476925286766559;
-    for (int m = 0; m < n; ++m) {
-        tw[2 * m] = cos(two_pi * m / n);
-        tw[2 * m + 1] = -sin(two_pi * m / n);
-    }
-    if (n & (n - 1)) {
-        for (int k = 0; k < n; ++k) {
-            double re = 0.0, im = 0.0;
-            /* g[d] = h[d]: angle index d k mod n, stepped by k */
-            for (int d = 0, m = 0; d < ns; ++d, m = m + k >= n ? m + k - n : m + k) {
-                re += h[d] * tw[2 * m];
-                im += h[d] * tw[2 * m + 1];
-            }
-            /* g[n - d] = h[ns - d]: angle index (n - d) k mod n = -d k mod n */
-            for (int d = 1, m = k ? n - k : 0; d < ns; ++d, m = m >= k ? m - k : m - k + n) {
-                re += h[ns - d] * tw[2 * m];
-                im += h[ns - d] * tw[2 * m + 1];
-            }
-            G[2 * k] = re;
-            G[2 * k + 1] = im;
-        }
-        return;
-    }
-    for (int j = 0; j < n; ++j) G[2 * j] = G[2 * j + 1] = 0.0;
-    for (int d = 0; d < ns; ++d) G[2 * d] = h[d];
-    for (int d = 1; d < ns; ++d) G[2 * (n - d)] = h[ns - d];
-    /* bit-reversal permutation, then log2 N butterfly stages */
     for (int i = 1, j = 0; i < n; ++i) {
         int bit = n >> 1;
         for (; j & bit; bit >>= 1) j ^= bit;
@@ -350,7 +319,7 @@ static inline void postfft_host_tables(const double *h, int ns, int n, double *G
         }
     }
     for (int len = 2; len <= n; len <<= 1) {
-        const int half = len >> 1, stride = n / len;
+        const int half = len >> 1, stride = n / len * step;
         for (int s = 0; s < n; s += len)
             for (int k = 0; k < half; ++k) {
                 const double wr = tw[2 * k * stride], wi = tw[2 * k * stride + 1];
@@ -360,6 +329,51 @@ static inline void postfft_host_tables(const double *h, int ns, int n, double *G
                 a[0] += br; a[1] += bi;
             }
     }
+}
+
+/* Host tables of the FFT form for the kernel h[0..ns): G = DFT_N(g) and the
+ * twiddles exp(-2 pi i m / N), m < N, each N double2 ({re, im}) into
+ * caller arrays.  G in double, by radix-2 transforms (of the three decimated
+ * sequences for 3072 points); twiddles from cos/sin of the exact angle.
+ * Returns nonzero if out of memory. */
+static inline int postfft_host_tables(const double *h, int ns, int n, double *G, double *tw)
+{
+    const double two_pi = 6.283185307179586476925286766559;
+    for (int m = 0; m < n; ++m) {
+        tw[2 * m] = cos(two_pi * m / n);
+        tw[2 * m + 1] = -sin(two_pi * m / n);
+    }
+    if (n & (n - 1)) {
+        /* n = 3 m, m a power of two: the transforms F_r of the three sequences
+         * g[3 j + r] in G's thirds, then G[k] = sum_r W^(r k) F_r[k mod m] */
+        const int m = n / 3;
+        double *F = (double *)malloc(sizeof(double) * 2 * (size_t)n);
+        if (!F) return 1;
+        for (int j = 0; j < n; ++j) {
+            const int d = j < ns ? j : j > n - ns ? ns - (n - j) : -1;   /* g[n - e] = h[ns - e] */
+            double *f = F + 2 * (j % 3 * m + j / 3);
+            f[0] = d >= 0 ? h[d] : 0.0;
+            f[1] = 0.0;
+        }
+        for (int r = 0; r < 3; ++r) postfft_host_fft(F + 2 * r * m, m, tw, 3);
+        for (int k = 0; k < n; ++k) {
+            double re = 0.0, im = 0.0;
+            for (int r = 0; r < 3; ++r) {
+                const double *f = F + 2 * (r * m + k % m), *w = tw + 2 * ((long long)r * k % n);
+                re += f[0] * w[0] - f[1] * w[1];
+                im += f[0] * w[1] + f[1] * w[0];
+            }
+            G[2 * k] = re;
+            G[2 * k + 1] = im;
+        }
+        free(F);
+        return 0;
+    }
+    for (int j = 0; j < n; ++j) G[2 * j] = G[2 * j + 1] = 0.0;
+    for (int d = 0; d < ns; ++d) G[2 * d] = h[d];
+    for (int d = 1; d < ns; ++d) G[2 * (n - d)] = h[ns - d];
+    postfft_host_fft(G, n, tw, 1);
+    return 0;
 }
 
 /* Launch k_postfft<Pro> over ntraces traces of ns samples; G and tw are the

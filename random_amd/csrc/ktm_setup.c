@@ -140,6 +140,32 @@ static float image_coord(const ktm_config *c, double col, int axis)
     return (float)((start + col * inc) * d);
 }
 
+int ktm_even_kernel(const float *a, const float *b, int ns, double *g)
+{
+    /* the ns cosines once: each sum takes them in steps of m around the
+     * circle, so the ns^2 calls of cosl gave these ns values (1001 samples:
+     * 60 ms of a plan's set-up, now 2) */
+    const long double two_pi = 2.0L * acosl(-1.0L);
+    long double *c = (long double *)malloc(sizeof(long double) * 2 * (size_t)ns);
+    if (!c) return KTM_ERR_NOMEM;
+    long double *s = c + ns;
+    for (int k = 0; k < ns; ++k) {
+        c[k] = cosl(two_pi * k / ns);
+        s[k] = b ? (long double)a[k] * (long double)b[k] : (long double)a[k];
+    }
+    for (int m = 0; m < ns; ++m) {
+        long double acc = 0.0L;
+        for (int k = 0, km = 0; k < ns; ++k) {
+            acc += s[k] * c[km];
+            km += m;
+            if (km >= ns) km -= ns;
+        }
+        g[m] = (double)(acc / ns);
+    }
+    free(c);
+    return KTM_OK;
+}
+
 void ktm_tables_free(ktm_tables *tb)
 {
     free(tb->anti_alias); free(tb->t2); free(tb->t1); free(tb->colx); free(tb->coly);
@@ -217,16 +243,9 @@ int ktm_tables_build(const ktm_config *c, int ns, float dt, int nsm, float dtm,
     /* post-stack kernel: h[m] = (1/ns) sum_k aa[k] cos(2 pi k m / ns); the
      * spectrum is even (aa[k] == aa[ns-k], odd-ns zero bins included), so the
      * filter of Kirchhoff.c:1465-1478 is this real circular convolution */
-    const long double two_pi = 2.0L * acosl(-1.0L);
-    for (int m = 0; m < ns; ++m) {
-        long double acc = 0.0L;
-        long long km = 0;
-        for (int k = 0; k < ns; ++k) {
-            acc += (long double)tb->anti_alias[k] * cosl(two_pi * km / ns);
-            km += m;
-            if (km >= ns) km -= ns;
-        }
-        tb->hconv[m] = (double)(acc / ns);
+    if (ktm_even_kernel(tb->anti_alias, NULL, ns, tb->hconv) != KTM_OK) {
+        ktm_tables_free(tb);
+        return KTM_ERR_NOMEM;
     }
     if (bad) {
         ktm_tables_free(tb);
