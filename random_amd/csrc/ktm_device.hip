@@ -36,6 +36,8 @@
 
 #include <mutex>
 
+#include <math.h>
+
 #include <stdint.h>
 #include <stdlib.h>
 #include <string.h>
@@ -788,6 +790,9 @@ __device__ __forceinline__ int reference_T(float dIS2, float dIR2, float rsn, fl
     return exact_T(dIS2, dIR2, t2, v2, 1.0f / v2, dt, rdt, ns);
 }
 
+/* slots whose traveltime chains run side by side under one test */
+constexpr int mig_group(int K) { return K % 3 == 0 ? 3 : K % 4 == 0 ? 4 : K % 5 == 0 ? 5 : 2; }
+
 typedef __attribute__((address_space(3))) float lds_float;
 typedef __attribute__((address_space(3))) void lds_void;
 typedef __attribute__((address_space(3))) unsigned long long lds_u64;
@@ -802,11 +807,11 @@ typedef __attribute__((address_space(1))) const void global_void;
  * to those whose CMP can reach the tile (ordered compaction into a list);
  * the aperture and slab gates of the next 64 of the list are evaluated
  * lane-parallel (lane j = trace j), and the passing ones are walked in order.
- * Rows are staged C at a time into a ring of three such chunks by loads that
+ * Rows are staged C at a time into a ring of WN + 1 such chunks by loads that
  * write LDS directly: chunk q + 1 is in flight while chunk q is used, so the
  * loads' latency is hidden, no register holds a staged row, and one barrier
- * per chunk separates the two (the third slot keeps the previous chunk for
- * the re-summation below).
+ * per chunk separates the two (the other slots keep the window's earlier
+ * chunks for the re-summation below).
  *
  * Traveltime index, two variants:
  * - exact (the FP32 reference path, and the Kahan modes unless FASTIDX): the
@@ -814,7 +819,7 @@ typedef __attribute__((address_space(1))) const void global_void;
  *   used at once; a sample whose p ns lies within the form's error bound of an
  *   integer (and is not past the trace for certain) is added with that index
  *   and remembered with the running sum before the add (one per lane and
- *   window of two chunks; a lane's further ambiguous samples take the inline
+ *   window of WN chunks; a lane's further ambiguous samples take the inline
  *   exact path).  At the end of the window one wave-wide pass computes the
  *   reference index of every lane's remembered sample together; where it
  *   differs from the fast one (a few percent of them) the sample's running sum
@@ -844,22 +849,24 @@ typedef __attribute__((address_space(1))) const void global_void;
  * 6.75 ms.  12 waves of K = 8 (six per SIMD) measured the same as 8 of K = 12
  * with 1500 samples, 16 waves in one workgroup 15 % slower (all of a CU's waves
  * at one barrier); slot groups of 2, 4 and 6 within 3 % of 3. */
-template <int K, int W, int NW, int C, int EU, bool KAHAN, bool FASTIDX>
+template <int K, int W, int NW, int C, int WN, int EU, bool KAHAN, bool FASTIDX>
 __global__ void __launch_bounds__(NW * KTM_WAVE) __attribute__((amdgpu_waves_per_eu(EU, EU)))
 k_migrate(const MigArgs a)
 {
-    constexpr int NCOL = NW / W;            /* image columns per workgroup */
     constexpr int NT = NW * KTM_WAVE;
     constexpr int WPR = NW / C;             /* waves that stage one row of a chunk */
     constexpr bool SPEC = !FASTIDX;
-    constexpr int G = K % 3 ? 4 : 3;        /* slots side by side */
-    static_assert(NW % C == 0 && 2 * C <= 16 && K < 16 && K % G == 0 && KTM_WAVE % (2 * C) == 0,
+    constexpr int G = mig_group(K);         /* slots side by side */
+    constexpr int WT = WN * C;              /* traces of a window */
+    constexpr int SB = KTM_WAVE / WT * WT;  /* traces whose gates are evaluated at once */
+    constexpr int RING = WN + 1;            /* chunks in LDS: a window's and the next */
+    static_assert(NW % C == 0 && WT <= 16 && K < 16 && K % G == 0,
                   "remembered samples pack the slot and the trace in 4 bits each");
     extern __shared__ float4 lds4[];
     const int ldl = (int)a.row;             /* LDS row = prepared row (floats) */
-    float *sF = reinterpret_cast<float *>(lds4);            /* [3][C][ldl]  */
-    float2 *sMax = reinterpret_cast<float2 *>(sF + 3 * C * ldl);   /* [NW][K] largest rs, tq */
-    int *sSel = reinterpret_cast<int *>(sMax + NW * K);     /* [64 + C + NT] */
+    float *sF = reinterpret_cast<float *>(lds4);            /* [RING][C][ldl] */
+    float2 *sMax = reinterpret_cast<float2 *>(sF + RING * C * ldl);   /* [NW][K] largest rs, tq */
+    int *sSel = reinterpret_cast<int *>(sMax + NW * K);     /* [64 + C + NT], SB + C - 1 + NT used */
     int *sCnt = sSel + KTM_WAVE + C + NT;                   /* [NW]     */
 
     const int tid = threadIdx.x, lane = tid & (KTM_WAVE - 1);
@@ -932,7 +939,7 @@ k_migrate(const MigArgs a)
     }
 
     /* Kahan variants: the taps are summed onto y = -c in plain FP32 over
-     * KTM_KAHAN_FOLD windows (at most KTM_KAHAN_FOLD * 2C terms, error
+     * 2 KTM_KAHAN_FOLD chunks (at most 2 KTM_KAHAN_FOLD C terms, error
      * <= (terms - 1) u times their magnitudes) and added to the image with one
      * compensated step, which keeps the compensated error bound of order
      * u * sum |f| at a fraction of the per-tap cost.  Plain variants add
@@ -957,9 +964,9 @@ k_migrate(const MigArgs a)
     /* the list of traces that can reach the tile, in order: sSel[head, n) */
     int head = 0, n = 0;
     auto refill = [&]() __attribute__((always_inline)) {
-        while (n - head < KTM_WAVE + C && c0 < a.ntr) {
+        while (n - head < SB + C && c0 < a.ntr) {
             if (head) {                          /* the rest to the front */
-                const int left = n - head;       /* < 64 + C <= NT */
+                const int left = n - head;       /* < SB + C <= NT */
                 const int v = tid < left ? sSel[head + tid] : 0;
                 __syncthreads();
                 if (tid < left) sSel[tid] = v;
@@ -1021,7 +1028,7 @@ k_migrate(const MigArgs a)
         /* gates and distances of Kirchhoff.c:1334-1354 for the next 64 traces
          * at once (lane j = trace j), on squared distances with the exact
          * thresholds of ktm_gate_threshold */
-        const int nb = min(KTM_WAVE, n - head);
+        const int nb = min(SB, n - head);
         float g_is = 0.0f, g_ir = 0.0f;
         int g_ti = 0;
         bool gp = false;
@@ -1059,15 +1066,18 @@ k_migrate(const MigArgs a)
          * index << 8 (-1: none) and the sum before it */
         int qi = -1;
         float qs = 0.0f;
+        int wnext = 0;
         for (int q = 0; q * C < nb; ++q) {
+            /* chunk q's place in its window */
+            const int wq = (WN & (WN - 1)) ? wnext : (q & (WN - 1));
             /* chunk q has arrived and every wave is done with chunk q - 1,
              * so with the slot that chunk q + 1 goes to */
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             __syncthreads();
-            const int nslot = slot == 2 ? 0 : slot + 1;
+            const int nslot = slot == RING - 1 ? 0 : slot + 1;
             const int jn = (q + 1) * C + jrow;      /* this wave's row of chunk q + 1 */
             if (head + jn < n)
-                issue(jn < KTM_WAVE ? __builtin_amdgcn_readlane(g_ti, jn)
+                issue(jn < SB ? __builtin_amdgcn_readlane(g_ti, jn)
                                     : __builtin_amdgcn_readfirstlane(sSel[head + jn]), nslot);
 
             uint32_t pmc = (uint32_t)(pm >> (q * C)) & ((1u << C) - 1u);
@@ -1118,7 +1128,7 @@ k_migrate(const MigArgs a)
                         }
                         const float thr = __uint_as_float(lim);
                         if (far >= thr) {
-                            const int jw = (q & 1) * C + j;
+                            const int jw = wq * C + j;
 #pragma unroll
                             for (int i = 0; i < G; ++i) {
                                 if (!(fabsf(fg[i].dev) >= thr)) continue;
@@ -1147,16 +1157,15 @@ k_migrate(const MigArgs a)
                     }
                 }
             }
-            const bool wend = (q & 1) || (q + 1) * C >= nb;     /* end of the window */
+            const bool wend = wq == WN - 1 || (q + 1) * C >= nb;    /* end of the window */
             if (SPEC && wend && __ballot(qi >= 0)) {
                 /* ---- the reference index of every lane's remembered sample ---- */
-                const int w0 = (q & ~1) * C;         /* the window's first trace */
-                /* row of the window's trace jw: the previous slot holds the
-                 * first chunk when the current one is the second */
-                const int pslot = slot == 0 ? 2 : slot - 1;
+                const int w0 = (q - wq) * C;         /* the window's first trace */
+                /* row of the window's trace jw: its chunk lies wq - jw / C
+                 * slots before the current one */
                 auto row_of = [&](int jw) __attribute__((always_inline)) {
-                    const int s = (q & 1) && jw < C ? pslot : slot;
-                    return sF + (s * C + (jw & (C - 1))) * ldl;
+                    const int s = slot - wq + jw / C;
+                    return sF + ((s < 0 ? s + RING : s) * C + jw % C) * ldl;
                 };
                 const int jw = (qi >> 4) & 15, k = qi & 15;
                 const float dIS2 = __shfl(g_is, w0 + (qi >= 0 ? jw : 0));
@@ -1180,7 +1189,7 @@ k_migrate(const MigArgs a)
 #pragma unroll
                     for (int kk = 0; kk < K; ++kk)
                         if (kk == k) rsk = rs[kk];
-                    uint32_t later = (uint32_t)(pm >> w0) & ((1u << (2 * C)) - 1u);
+                    uint32_t later = (uint32_t)(pm >> w0) & ((1u << WT) - 1u);
                     while (later) {
                         const int jj = __builtin_ctz(later);
                         later &= later - 1u;
@@ -1202,10 +1211,11 @@ k_migrate(const MigArgs a)
                 }
                 qi = -1;
             }
-            if (KAHAN && wend && ++nfold == KTM_KAHAN_FOLD) {
+            if (KAHAN && wend && (nfold += WN) >= 2 * KTM_KAHAN_FOLD) {
                 nfold = 0;
                 fold_y();
             }
+            wnext = wq == WN - 1 ? 0 : wq + 1;
             slot = nslot;
         }
         head += nb;
@@ -1729,7 +1739,7 @@ __global__ void __launch_bounds__(8 * KTM_WAVE) __attribute__((amdgpu_waves_per_
 k_demigrate(const DemigArgs a)
 {
     constexpr int NCOL = 8 / W;
-    constexpr int G = K % 3 ? 4 : 3;               /* slots side by side */
+    constexpr int G = mig_group(K);                /* slots side by side */
     extern __shared__ unsigned long long sg[];     /* [tb][ns + DM_PAD] fixed point */
     __shared__ int32_t sIdx[DM_TB];
     const int tid = threadIdx.x, lane = tid & (KTM_WAVE - 1);
@@ -1766,7 +1776,8 @@ k_demigrate(const DemigArgs a)
     ylo = __builtin_amdgcn_readfirstlane(ylo); yhi = __builtin_amdgcn_readfirstlane(yhi);
     __syncthreads();
     const float qlim = (float)(ns + lane) + 0.5f;  /* clamp of q */
-    constexpr int P = K == 8 ? 4 : 8;
+    constexpr int P = K % 8 == 0 ? 4 : K % 4 == 0 ? 8 : 16;
+    static_assert(K % 2 == 0 && K <= 12, "P = 32 / gcd(K, 32)");
     const int rot = lane / P % K, tbase = seg * K * KTM_WAVE + lane * K;
     auto slot_t = [&](int k) __attribute__((always_inline)) {   /* sample of slot k */
         return tbase + (k + rot < K ? k + rot : k + rot - K);
@@ -2467,39 +2478,72 @@ extern "C" int ktm_image_reset(const ktm_plan *p, float *km, float *fold, float 
 typedef void (*mig_fn)(const MigArgs);
 struct MigShape {
     mig_fn fn;
-    int K, W, NW, C;    /* samples per lane, waves per column, waves, rows per chunk */
+    int K, W, NW, C, RING;   /* samples per lane, waves per column, waves, rows per chunk, chunks */
 };
 
 /* accum is KTM_ACCUM_PLAIN or KTM_ACCUM_KAHAN, optionally with KTM_INDEX_FAST */
-template <int K, int W, int NW, int C, int EU = 4>
-static MigShape pick_accum(int accum)
+template <int K, int W, int NW, int C, int WN>
+static MigShape mig_shape(int accum)
 {
     const bool kahan = (accum & ~KTM_INDEX_FAST) == KTM_ACCUM_KAHAN;
-    MigShape m = {nullptr, K, W, NW, C};
-    if (accum & KTM_INDEX_FAST)
-        m.fn = kahan ? k_migrate<K, W, NW, C, EU, true, true> : k_migrate<K, W, NW, C, EU, false, true>;
-    else
-        m.fn = kahan ? k_migrate<K, W, NW, C, EU, true, false> : k_migrate<K, W, NW, C, EU, false, false>;
-    return m;
+    if (accum & KTM_INDEX_FAST)         /* no window to keep */
+        return {kahan ? k_migrate<K, W, NW, C, 1, 4, true, true> : k_migrate<K, W, NW, C, 1, 4, false, true>,
+                K, W, NW, C, 2};
+    return {kahan ? k_migrate<K, W, NW, C, WN, 4, true, false> : k_migrate<K, W, NW, C, WN, 4, false, false>,
+            K, W, NW, C, WN + 1};
+}
+
+/* Relative time of a shape on ncol columns (x offset classes).  A trace costs
+ * a wave about MIG_SLOT instructions per slot and MIG_TRACE besides (k_migrate);
+ * a SIMD runs its waves' sum, ncol columns in workgroups of NW / W over 256
+ * CUs (whole workgroups while there are few), and issues at full rate from
+ * four waves.  Against 8 or 12 slots with 2 or 4 waves by length alone: 751
+ * samples take 12 x 1 instead of 8 x 2 (a 61 x 61 patch with the relaxed index
+ * 5.0 -> 3.3 ms), 1251 10 x 2 instead of 12 x 2 (150 x 150 columns 187 -> 171),
+ * 2503 10 x 4 instead of 12 x 4 (12 classes of 500 columns 6.75 -> 5.9), and 32
+ * columns of 501 samples 2 x 4 instead of 4 x 2 (60 -> 45 us).  The 800-column,
+ * 1001-sample line: 4 x 4 2.96 ms, 8 x 2 3.92, 2 x 8 3.22. */
+static double mig_cost(int K, int W, int NW, int64_t ncol, bool fast)
+{
+    static const double rate[5] = {0.0, 0.40, 0.65, 0.85, 1.0};
+    const double per_cu = (double)((ncol * W + NW - 1) / NW) / 256.0;
+    const double whole = per_cu < 8.0 ? ceil(per_cu) : per_cu;
+    const double waves = whole * NW / 4.0;
+    const double r = waves >= 4.0 ? 1.0 : rate[(int)waves] + (waves - (int)waves) *
+                                                                  (rate[(int)waves + 1] - rate[(int)waves]);
+    return waves * (fast ? 8.0 * K + 25.0 : 10.7 * K + 40.0) / r;
 }
 
 /* W waves share one image column (each owns K*64 consecutive samples); a
  * workgroup of NW waves covers NW/W columns. */
-static MigShape pick_migrate(int ns, int accum, int64_t wgs8)
+static MigShape pick_migrate(int ns, int accum, int64_t ncol)
 {
-    /* wgs8: workgroups of 8 columns (x offset classes) in the region.  An
-     * image too small to give every CU two workgroups at the default layout
-     * takes twice the waves per column with half the samples per lane: on
-     * the 800-column, 1001-sample line 3.77 ms against 4.79 ms (the 1536-
-     * sample layout gained nothing from 6 x 4 on a 1600-column line). */
-    if (ns <= 512) return wgs8 < 512 ? pick_accum<4, 2, 8, 4>(accum) : pick_accum<8, 1, 8, 4>(accum);
-    if (ns <= 1024) return 2 * wgs8 < 512 ? pick_accum<4, 4, 8, 4>(accum) : pick_accum<8, 2, 8, 4>(accum);
-    if (ns <= 1536) return pick_accum<12, 2, 8, 4>(accum);
-    if (ns <= 2048) return pick_accum<8, 4, 16, 4>(accum);
-    if (ns <= 3072) return pick_accum<12, 4, 16, 4>(accum);
-    /* fewer rows per chunk for long traces, so that the ring fits the LDS */
-    if (ns <= 4096) return pick_accum<8, 8, 16, 2>(accum);
-    return pick_accum<12, 8, 16, 2>(accum);
+    /* every shape, by samples per column; the ring of rows within half of a
+     * CU's LDS (two workgroups of 8 waves) or all of it (one of 16) */
+    static const struct { int cap, K, W, NW; MigShape (*make)(int); } S[] = {
+        {256, 2, 2, 8, mig_shape<2, 2, 8, 4, 4>},    {384, 6, 1, 8, mig_shape<6, 1, 8, 4, 4>},
+        {512, 2, 4, 8, mig_shape<2, 4, 8, 4, 4>},    {512, 4, 2, 8, mig_shape<4, 2, 8, 4, 4>},
+        {512, 8, 1, 8, mig_shape<8, 1, 8, 4, 4>},    {640, 10, 1, 8, mig_shape<10, 1, 8, 4, 4>},
+        {768, 6, 2, 8, mig_shape<6, 2, 8, 4, 3>},    {768, 12, 1, 8, mig_shape<12, 1, 8, 4, 3>},
+        {1024, 2, 8, 8, mig_shape<2, 8, 8, 4, 3>},   {1024, 4, 4, 8, mig_shape<4, 4, 8, 4, 3>},
+        {1024, 8, 2, 8, mig_shape<8, 2, 8, 4, 3>},   {1280, 10, 2, 8, mig_shape<10, 2, 8, 4, 2>},
+        {1536, 6, 4, 8, mig_shape<6, 4, 8, 4, 2>},   {1536, 12, 2, 8, mig_shape<12, 2, 8, 4, 2>},
+        {2048, 8, 4, 16, mig_shape<8, 4, 16, 4, 3>}, {2560, 10, 4, 16, mig_shape<10, 4, 16, 4, 2>},
+        {3072, 12, 4, 16, mig_shape<12, 4, 16, 4, 2>}, {4096, 8, 8, 16, mig_shape<8, 8, 16, 2, 2>},
+        {5120, 10, 8, 16, mig_shape<10, 8, 16, 2, 2>}, {6144, 12, 8, 16, mig_shape<12, 8, 16, 2, 2>}};
+    /* compensated sums of a small image are split along the traces instead */
+    if ((accum & ~KTM_INDEX_FAST) == KTM_ACCUM_KAHAN && ncol < (1 << 20)) ncol = 1 << 20;
+    int best = -1;
+    double tbest = 0.0;
+    for (int i = 0; i < (int)(sizeof S / sizeof S[0]); ++i) {
+        if (S[i].cap < ns) continue;
+        const double t = mig_cost(S[i].K, S[i].W, S[i].NW, ncol, (accum & KTM_INDEX_FAST) != 0);
+        if (best < 0 || t < tbest) {
+            best = i;
+            tbest = t;
+        }
+    }
+    return S[best].make(accum);
 }
 
 /* Tiles of the region [rx0,rx1) x [ry0,ry1): ncol columns, a row on a 2-D
@@ -2540,7 +2584,7 @@ static int parts_workspace(ktm_plan *p)
     memset(&a, 0, sizeof a);
     a.rx1 = s->nxp; a.ry1 = s->nyp;
     const MigShape m = pick_migrate(s->ns, KTM_ACCUM_KAHAN,
-                                    ((int64_t)s->nxp * s->nyp + 7) / 8 * s->nh);
+                                    (int64_t)s->nxp * s->nyp * s->nh);
     tile_layout(s, m.NW / m.W, &a);
     int n = parts_for((int64_t)a.ntiles * s->nh);
     const uint64_t per = 3ull * sizeof(float) * (uint64_t)s->nxp * s->nyp * s->nh * s->ns;
@@ -2692,7 +2736,7 @@ static int migrate_block(const ktm_plan *p, const void *prepared, int dtype, int
         a.ry0 = (job % p->cfg.jobs_y) * s->ny; a.ry1 = a.ry0 + s->ny;
     }
     const int64_t ncols_region = (int64_t)(a.rx1 - a.rx0) * (a.ry1 - a.ry0);
-    const MigShape m = pick_migrate(s->ns, accum, (ncols_region + 7) / 8 * s->nh);
+    const MigShape m = pick_migrate(s->ns, accum, ncols_region * s->nh);
     const mig_fn fn = m.fn;
     tile_layout(s, m.NW / m.W, &a);
     const int nthreads = m.NW * KTM_WAVE;
@@ -2708,7 +2752,7 @@ static int migrate_block(const ktm_plan *p, const void *prepared, int dtype, int
     }
     a.nparts = nparts;
     /* the ring of rows, the slots' largest constants, the trace list, counts */
-    const size_t lds = sizeof(float) * (size_t)(3 * m.C * p->row + 2 * m.NW * m.K) +
+    const size_t lds = sizeof(float) * (size_t)(m.RING * m.C * p->row + 2 * m.NW * m.K) +
                        sizeof(int) * (size_t)(KTM_WAVE + m.C + nthreads + m.NW);
     if (lds > 160 * 1024) return KTM_ERR_UNSUPPORTED;
     /* runs of a row of tiles, but at least 8 runs per XCD */
@@ -2978,13 +3022,23 @@ static int demigrate(const ktm_plan *p, const float *km, const ktm_trace_geom *g
     if (a.tb < 1) return KTM_ERR_UNSUPPORTED;
     typedef void (*fn_t)(const DemigArgs);
     fn_t fn;
-    if (s->ns <= 512) fn = fast ? k_demigrate<8, 1, true> : k_demigrate<8, 1, false>;
-    else if (s->ns <= 1024) fn = fast ? k_demigrate<8, 2, true> : k_demigrate<8, 2, false>;
-    else if (s->ns <= 1536) fn = fast ? k_demigrate<12, 2, true> : k_demigrate<12, 2, false>;
-    else if (s->ns <= 2048) fn = fast ? k_demigrate<8, 4, true> : k_demigrate<8, 4, false>;
-    else if (s->ns <= 3072) fn = fast ? k_demigrate<12, 4, true> : k_demigrate<12, 4, false>;
-    else if (s->ns <= 4096) fn = fast ? k_demigrate<8, 8, true> : k_demigrate<8, 8, false>;
-    else fn = fast ? k_demigrate<12, 8, true> : k_demigrate<12, 8, false>;
+    static const struct { int cap; fn_t f[2]; } shapes[] = {
+        {384, {k_demigrate<6, 1, false>, k_demigrate<6, 1, true>}},
+        {512, {k_demigrate<8, 1, false>, k_demigrate<8, 1, true>}},
+        {640, {k_demigrate<10, 1, false>, k_demigrate<10, 1, true>}},
+        {768, {k_demigrate<12, 1, false>, k_demigrate<12, 1, true>}},
+        {1024, {k_demigrate<8, 2, false>, k_demigrate<8, 2, true>}},
+        {1280, {k_demigrate<10, 2, false>, k_demigrate<10, 2, true>}},
+        {1536, {k_demigrate<12, 2, false>, k_demigrate<12, 2, true>}},
+        {2048, {k_demigrate<8, 4, false>, k_demigrate<8, 4, true>}},
+        {2560, {k_demigrate<10, 4, false>, k_demigrate<10, 4, true>}},
+        {3072, {k_demigrate<12, 4, false>, k_demigrate<12, 4, true>}},
+        {4096, {k_demigrate<8, 8, false>, k_demigrate<8, 8, true>}},
+        {5120, {k_demigrate<10, 8, false>, k_demigrate<10, 8, true>}},
+        {KTM_MAX_NS, {k_demigrate<12, 8, false>, k_demigrate<12, 8, true>}}};
+    int sh = 0;
+    while (shapes[sh].cap < s->ns) ++sh;    /* ns <= KTM_MAX_NS by ktm_plan_create */
+    fn = shapes[sh].f[fast ? 1 : 0];
     const size_t lds = row * (size_t)a.tb;
     HIP_TRY(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     for (int64_t i0 = 0; i0 < ntr; i0 += 1 << 30) {

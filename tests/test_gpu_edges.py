@@ -228,3 +228,34 @@ def test_prepared_rows_at_any_float(cuda):
     km2, fold2, _ = plan.new_image(device=cuda)
     plan.migrate_block(odd, geom, km2, fold2)
     assert bool(km.any()) and torch.equal(km, km2) and torch.equal(fold, fold2)
+
+
+# both sides of every boundary of the lane layouts by samples per lane and
+# waves per column (2, 4, 6, 8, 10 or 12 x 64 x 1, 2, 4 or 8); the 4104-column
+# image takes the widest lanes of its length, the 40-column one the narrowest
+LAYOUT_NS = [256, 257, 384, 385, 640, 641, 768, 769, 1280, 1281, 2560, 2561, 5120, 5121]
+
+
+@pytest.mark.parametrize("ncols", [40, 4104])
+@pytest.mark.parametrize("ns", LAYOUT_NS)
+def test_lane_layout_boundaries_bitexact(cuda, ns, ncols):
+    print(f"case: ns={ns}, 60 traces, {ncols} columns", flush=True)
+    sv = small_line(ns, ncols=ncols)
+    tr = surveys.traces_numpy(sv)
+    _, km, _, n = bitexact_case(sv, tr, cuda, block=43)
+    assert n > 0 and np.abs(km).max() > 0
+
+
+@pytest.mark.parametrize("fast", [False, True])
+@pytest.mark.parametrize("ns", LAYOUT_NS)
+def test_adjoint_at_lane_layout_boundaries(cuda, ns, fast):
+    print(f"case: dot test at ns={ns}, fast={fast}", flush=True)
+    sv = small_line(ns)
+    plan = Plan(sv.cfg, sv.ns, sv.dt, sv.vel)
+    op = Operator(plan, torch.from_numpy(sv.coords).to(cuda), fast=fast)
+    g = torch.Generator(device=cuda).manual_seed(ns)
+    d = torch.randn((sv.ntr, sv.ns), generator=g, device=cuda)
+    m = torch.randn(plan.image_shape, generator=g, device=cuda)
+    lhs, rhs, rel = dot_test(op, d, m)
+    print(f"  rel {rel:.2e}", flush=True)
+    assert rel <= 1e-5
