@@ -21,7 +21,7 @@
  *                   an FP64 FFT convolution (ktm_postfft.h; beyond 4096
  *                   samples the FP64 matrix product of ktm_postmx.h); its
  *                   transpose k_postfft<PostImg> + k_poststack_adjoint_tail
- *   k_image_*       image<job>.su trace records (headers + big-endian
+ *   k_image_records image<job>.su trace records (headers + big-endian
  *                   samples), Kirchhoff.c:1437-1598
  *   k_demigrate     exact transpose of k_migrate (CLOSED prep)
  *   k_synth_*       seeded synthetic surveys
@@ -66,7 +66,8 @@ struct ktm_plan {
     float *d_vel2;          /* [nvel_il][nvel_xl][nsm], squared like Kirchhoff.c:617 */
     float *d_w;             /* [ns+2] CLOSED weights */
     double *d_hconv2;       /* [2 ns] post-stack kernel, h2[m] = h[m mod ns] */
-    double2 *d_pf_g, *d_pf_tw; /* [N] FFT form of the post-stack kernel and twiddles */
+    double *d_pf_g;         /* [N] FFT form of the post-stack kernel */
+    double2 *d_pf_tw;       /* [N] twiddles */
     int pf_n;                /* points of the FFT form, 0: the direct product */
     float *d_stage;         /* FP32 filtered traces of a BF16/FP16 block */
     size_t stage_cap;       /* elements of d_stage */
@@ -1352,9 +1353,13 @@ __global__ void k_image_reset(float *km, float *fold, float *comp, int64_t n)
 /* x of the post-stack filter, Kirchhoff.c:1460: a float expression stored
  * into a double */
 struct PostKtm {
-    static __device__ __forceinline__ double x(const float *k, const float *f, int u, float dt)
+    static __device__ __forceinline__ float3 load(const float *k, const float *f, int u)
     {
-        return (double)(-dt * (float)u * (k[u] - k[u - 1]) * dt / f[u]);
+        return make_float3(k[u], k[u - 1], f[u]);
+    }
+    static __device__ __forceinline__ double value(float3 l, int u, float dt)
+    {
+        return (double)(-dt * (float)u * (l.x - l.y) * dt / l.z);
     }
 };
 
@@ -1998,10 +2003,11 @@ __global__ void k_zero_u64(unsigned long long *p, int64_t n)
  * trace per workgroup in place: uu[t] = C[t] w[t] (FP64, uu[0] = uu[ns] = 0),
  * out[t] = uu[t] - uu[t + 1]. */
 struct PostImg {
-    static __device__ __forceinline__ double x(const float *im, const float *, int u, float)
+    static __device__ __forceinline__ float3 load(const float *im, const float *, int u)
     {
-        return (double)im[u];
+        return make_float3(im[u], 0.0f, 0.0f);
     }
+    static __device__ __forceinline__ double value(float3 l, int, float) { return (double)l.x; }
 };
 
 __global__ void __launch_bounds__(PS_NT) k_poststack_adjoint_tail(const float *__restrict__ fold,
@@ -2133,12 +2139,12 @@ extern "C" int ktm_plan_create(ktm_plan **out, const ktm_config *cfg, int ns, fl
     }
     if (st == KTM_OK && (p->pf_n = postfft_size(ns)) != 0) {
         const size_t n = (size_t)p->pf_n;
-        double *g = (double *)malloc(sizeof(double) * 4 * n);
+        double *g = (double *)malloc(sizeof(double) * 5 * n);
         if (!g) st = KTM_ERR_NOMEM;
         if (st == KTM_OK) {
-            if (postfft_host_tables(tb->hconv, ns, p->pf_n, g, g + 2 * n)) st = KTM_ERR_NOMEM;
-            if (st == KTM_OK) st = upload(&p->d_pf_g, reinterpret_cast<const double2 *>(g), n);
-            if (st == KTM_OK) st = upload(&p->d_pf_tw, reinterpret_cast<const double2 *>(g + 2 * n), n);
+            postfft_host_tables(tb->hconv, ns, p->pf_n, g, g + n, g + 3 * n);
+            st = upload(&p->d_pf_g, g, n);
+            if (st == KTM_OK) st = upload(&p->d_pf_tw, reinterpret_cast<const double2 *>(g + n), n);
         }
         free(g);
     }
@@ -2371,14 +2377,11 @@ struct ImgHdrArgs {
     uint32_t dt_us;                 /* (unsigned short)(dt * 1e6), Kirchhoff.c:1447 */
 };
 
-/* image<job>.su, Kirchhoff.c:1437-1598: record r = (xc ny + yc) nh + ih of
- * the job's slab; one lane per record writes its 240-byte header (the
- * fields the reference sets, big-endian, the rest zero) */
-__global__ void k_image_headers(const ImgHdrArgs a, uint32_t *__restrict__ rec)
+/* word w of the 240-byte header of image<job>.su's record r = (xc ny + yc) nh +
+ * ih of the job's slab, Kirchhoff.c:1437-1598: the fields the reference sets,
+ * big-endian, the rest zero */
+__device__ __forceinline__ uint32_t image_header_word(const ImgHdrArgs &a, int64_t r, int w)
 {
-    const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t nrec = (int64_t)a.nx * a.ny * a.nh;
-    if (r >= nrec) return;
     const int ih = (int)(r % a.nh);
     const int64_t c = r / a.nh;
     const int xc = (int)(c / a.ny), yc = (int)(c % a.ny);
@@ -2391,36 +2394,31 @@ __global__ void k_image_headers(const ImgHdrArgs a, uint32_t *__restrict__ rec)
     const float cx = (float)a.ox_i + a.cosA * (float)xm - a.sinA * (float)ym;
     const float cy = (float)a.oy_i + a.sinA * (float)xm + a.cosA * (float)ym;
     const int tracl = a.nx * a.ny * a.nh * a.job + 1 + (xc * a.ny + yc) * a.nh + ih;
-    uint32_t *h = rec + r * (60 + (int64_t)a.ns);
-    for (int w = 0; w < 60; ++w) {
-        uint32_t v = 0u;
-        switch (w) {
-        case 0: v = __builtin_bswap32((uint32_t)tracl); break;                  /* tracl */
-        case 5: v = __builtin_bswap32((uint32_t)(X + a.Nx * Y + 1)); break;     /* cdp */
-        case 9: v = __builtin_bswap32((uint32_t)(int)ceil(a.oh + ih * a.dh)); break;  /* offset */
-        case 18: case 19: case 20: case 21: v = __builtin_bswap32(1u); break;   /* sx..gy */
-        case 28: v = __builtin_bswap32((uint32_t)(a.ns & 0xffff)); break;       /* ns, 114 */
-        case 29: v = __builtin_bswap32(a.dt_us << 16); break;                   /* dt, 116 */
-        case 45: v = __builtin_bswap32((uint32_t)(int)cx); break;               /* cdpx */
-        case 46: v = __builtin_bswap32((uint32_t)(int)cy); break;               /* cdpy */
-        case 47: v = __builtin_bswap32((uint32_t)(int)il); break;               /* iline */
-        case 48: v = __builtin_bswap32((uint32_t)(int)xl); break;               /* xline */
-        case 51: case 55: case 56: case 58:     /* mess: 0 in the first record, */
-            v = r > 0 ? __builtin_bswap32(9999u) : 0u; break;   /* then 9999 (:1224, 1589) */
-        case 59: v = __builtin_bswap32(9999u); break;                           /* :1589-1590 */
-        default: break;
-        }
-        h[w] = v;
+    switch (w) {
+    case 0: return __builtin_bswap32((uint32_t)tracl);                      /* tracl */
+    case 5: return __builtin_bswap32((uint32_t)(X + a.Nx * Y + 1));         /* cdp */
+    case 9: return __builtin_bswap32((uint32_t)(int)ceil(a.oh + ih * a.dh));    /* offset */
+    case 18: case 19: case 20: case 21: return __builtin_bswap32(1u);       /* sx..gy */
+    case 28: return __builtin_bswap32((uint32_t)(a.ns & 0xffff));           /* ns, 114 */
+    case 29: return __builtin_bswap32(a.dt_us << 16);                       /* dt, 116 */
+    case 45: return __builtin_bswap32((uint32_t)(int)cx);                   /* cdpx */
+    case 46: return __builtin_bswap32((uint32_t)(int)cy);                   /* cdpy */
+    case 47: return __builtin_bswap32((uint32_t)(int)il);                   /* iline */
+    case 48: return __builtin_bswap32((uint32_t)(int)xl);                   /* xline */
+    case 51: case 55: case 56: case 58:         /* mess: 0 in the first record, */
+        return r > 0 ? __builtin_bswap32(9999u) : 0u;       /* then 9999 (:1224, 1589) */
+    case 59: return __builtin_bswap32(9999u);                               /* :1589-1590 */
+    default: return 0u;
     }
 }
 
-/* samples of image<job>.su: record r of the slab <- image[X][Y][ih][t] */
-/* the samples of image<job>.su: one workgroup per record r, its image row
- * byte-swapped into place; 16-byte vectors when ns % 4 == 0 (image rows and
- * records then start 16-byte aligned: 240-byte header, 4 (60 + ns)-byte
- * records) */
+/* image<job>.su: one workgroup per record r, its header by the first 60 lanes
+ * (a kernel of its own with one lane per record took 53 us of 160,000 records'
+ * 410) and its image row [X][Y][ih][t] byte-swapped into place; 16-byte
+ * vectors when ns % 4 == 0 (image rows and records then start 16-byte aligned:
+ * 240-byte header, 4 (60 + ns)-byte records) */
 template <bool V4>
-__global__ void __launch_bounds__(128) k_image_samples(const float *__restrict__ image,
+__global__ void __launch_bounds__(128) k_image_records(const float *__restrict__ image,
                                                         const ImgHdrArgs a,
                                                         uint32_t *__restrict__ rec)
 {
@@ -2431,6 +2429,7 @@ __global__ void __launch_bounds__(128) k_image_samples(const float *__restrict__
     const int64_t Y = c % a.ny + (int64_t)(a.job % a.jobs_y) * a.ny;
     const float *src = image + ((X * a.nyp + Y) * a.nh + ih) * a.ns;
     uint32_t *dst = rec + r * (60 + (int64_t)a.ns) + 60;
+    if (threadIdx.x < 60) dst[(int)threadIdx.x - 60] = image_header_word(a, r, (int)threadIdx.x);
     if (V4) {
         const int n4 = a.ns / 4;
         for (int i = threadIdx.x; i < n4; i += blockDim.x) {
@@ -2488,17 +2487,14 @@ extern "C" int ktm_image_records(const ktm_plan *p, const float *image, int job,
     a.job = job; a.jobs_y = c->jobs_y;
     a.dt_us = (uint32_t)(uint16_t)(st->dt * 1000000);
     const int64_t nrec = (int64_t)a.nx * a.ny * a.nh;
-    const int nt = 256;
     if (nrec > 0x7fffffffLL) return KTM_ERR_UNSUPPORTED;
     hipStream_t s = (hipStream_t)stream;
-    hipLaunchKernelGGL(k_image_headers, dim3((unsigned)((nrec + nt - 1) / nt)), dim3(nt), 0, s, a,
-                       (uint32_t *)records);
     const bool v4 = a.ns % 4 == 0 && ((uintptr_t)records & 15u) == 0 && ((uintptr_t)image & 15u) == 0;
     if (v4)
-        hipLaunchKernelGGL(k_image_samples<true>, dim3((unsigned)nrec), dim3(128), 0, s, image, a,
+        hipLaunchKernelGGL(k_image_records<true>, dim3((unsigned)nrec), dim3(128), 0, s, image, a,
                            (uint32_t *)records);
     else
-        hipLaunchKernelGGL(k_image_samples<false>, dim3((unsigned)nrec), dim3(128), 0, s, image, a,
+        hipLaunchKernelGGL(k_image_records<false>, dim3((unsigned)nrec), dim3(128), 0, s, image, a,
                            (uint32_t *)records);
     HIP_TRY(hipGetLastError());
     return KTM_OK;

@@ -144,7 +144,8 @@ struct ktm_eom_plan {
     float *d_v2, *d_t2d;      /* [ns] v^2 (EOM.c:877), sqrt(t dt) t dt (EOM.c:1196) */
     double *d_sv;             /* [ns] sqrt(v^2) in double (EOM.c:1290) */
     double *d_g2;             /* [2 ns] post-filter kernel, g2[m] = g[m mod ns] */
-    double2 *d_pf_g, *d_pf_tw; /* [N] FFT form of the post-filter kernel and twiddles */
+    double *d_pf_g;            /* [N] FFT form of the post-filter kernel */
+    double2 *d_pf_tw;          /* [N] twiddles */
     int pf_n;                  /* points of the FFT form, 0: the direct product */
     float4 *d_geo;            /* [cap] per-trace h2, cmpX, cmpY, talpha */
     int64_t geo_cap;
@@ -222,16 +223,15 @@ extern "C" int ktm_eom_plan_create(ktm_eom_plan **out, const ktm_eom_config *c, 
         st = KTM_ERR_DEVICE;
     if (st == KTM_OK && (p->pf_n = postfft_size(ns)) != 0) {
         const size_t n = (size_t)p->pf_n;
-        double *t = (double *)malloc(sizeof(double) * 4 * n);
+        double *t = (double *)malloc(sizeof(double) * 5 * n);
         if (!t) st = KTM_ERR_NOMEM;
         if (st == KTM_OK) {
-            if (postfft_host_tables(g, ns, p->pf_n, t, t + 2 * n))
-                st = KTM_ERR_NOMEM;
-            else if (hipMalloc(&p->d_pf_g, sizeof(double2) * n) != hipSuccess ||
+            postfft_host_tables(g, ns, p->pf_n, t, t + n, t + 3 * n);
+            if (hipMalloc(&p->d_pf_g, sizeof(double) * n) != hipSuccess ||
                 hipMalloc(&p->d_pf_tw, sizeof(double2) * n) != hipSuccess)
                 st = KTM_ERR_NOMEM;
-            else if (hipMemcpy(p->d_pf_g, t, sizeof(double2) * n, hipMemcpyHostToDevice) != hipSuccess ||
-                     hipMemcpy(p->d_pf_tw, t + 2 * n, sizeof(double2) * n, hipMemcpyHostToDevice) !=
+            else if (hipMemcpy(p->d_pf_g, t, sizeof(double) * n, hipMemcpyHostToDevice) != hipSuccess ||
+                     hipMemcpy(p->d_pf_tw, t + n, sizeof(double2) * n, hipMemcpyHostToDevice) !=
                          hipSuccess)
                 st = KTM_ERR_DEVICE;
         }
@@ -530,9 +530,13 @@ __global__ void k_eom_reset(float *csp, float *fold, int64_t n)
 /* x of the post filter, EOM.c:1391: the float (csp / fold) dt t, stored into
  * a double; out = g (*) x in FP64 (k_postfft or k_postmx), out[0] = 0 */
 struct PostEom {
-    static __device__ __forceinline__ double x(const float *c, const float *f, int u, float dt)
+    static __device__ __forceinline__ float3 load(const float *c, const float *f, int u)
     {
-        return (double)((c[u] / f[u]) * dt * (float)u);
+        return make_float3(c[u], f[u], 0.0f);
+    }
+    static __device__ __forceinline__ double value(float3 l, int u, float dt)
+    {
+        return (double)((l.x / l.y) * dt * (float)u);
     }
 };
 

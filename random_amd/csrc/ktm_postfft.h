@@ -6,26 +6,35 @@
  * wrapped into N points, g[d] = h[d] (0 <= d < ns) and g[N - d] = h[ns - d]
  * (0 < d < ns), zero between, makes the length-N circular convolution of the
  * zero-padded trace equal the length-ns one on t < ns:
- *   out = IDFT_N(G . DFT_N(x)) / N,   G = DFT_N(g),
+ *   out = IDFT_N(G . DFT_N(x)) / N,   G = DFT_N(g)  (h is even, so is g, and
+ * G is real),
  * the O(ns log ns) form of Kirchhoff.c:1465-1478 (FFTW forward, filter,
  * backward, / ns: here the 1/ns is in h) and EOM.c:1386-1413.  g is real,
  * so two traces go through one complex transform, x_a + i x_b, and come
  * out as its real and imaginary parts.
  *
- * k_postfft: radix-16 Stockham passes (the last one radix 2, 4, 8 or 12
- * when N is not a power of 16), in place in LDS: every thread loads the
- * points of its butterflies (at most 16) into registers, the workgroup
- * synchronises, and the results go to their Stockham positions.  N / 16
- * threads per transform; a workgroup of 256 threads holds 4096 / N
- * transforms (N <= 4096) or one transform of 512 threads (N = 8192); N =
- * 3072 = 16 x 16 x 12 (traces of 1025 to 1536 samples) takes 256 threads,
- * 192 of them busy in the radix-16 passes, and 52 KB of LDS, so three
- * workgroups share a CU where two of 4096 points would.  The first forward pass
- * reads the traces (the prologue Pro of ktm_postmx.h), the first inverse
- * pass multiplies by G, the last inverse pass writes the output (both with
- * consecutive threads on consecutive samples).  LDS rows are padded by one
- * double2 per 16 so the stride-16 stores of the first pass spread over the
- * banks.
+ * k_postfft, in place in LDS without any reordering: the forward transform
+ * leaves X[k] where its decimation does and the inverse takes it from there,
+ * so the filter table lies in that order.  A pass over blocks of L points
+ * combines, in registers, the R points L / R apart that a lane holds (at most
+ * 16) and multiplies them by powers of a twiddle; the next works on blocks of
+ * L / R:
+ *   N -> N / 16 -> 16 -> done, the middle step of radix N / 256 = 2, 4, 8 or
+ *   12 (512 to 3072 points), 16 (4096) or 2 and 16 (8192), none for 256.
+ * N / 16 blocks of 16 are transformed, filtered and transformed back without
+ * leaving the registers.  Between the first and the last pass a wave works on
+ * 1024 points of its own (768 of 3072): whole blocks of N / 16, so these
+ * passes need no barrier, and a workgroup has two in all (none up to 1024
+ * points, where a wave holds 1024 / N transforms).  The first pass reads the
+ * traces (the prologue Pro of ktm_postmx.h), whose second half is padding, the
+ * last one writes t < ns <= N / 2; both with consecutive lanes on consecutive
+ * samples.  LDS rows are padded by one double2 per 16 so that lanes 16 points
+ * apart spread over the banks.
+ * 160,000 traces of 1500 samples: 1.3 ms (2.1 before, with a Stockham
+ * reordering and two barriers in every pass), 2.2 TB/s of traces and fold in
+ * and image out.  It is bound by FP64 instructions (about 1500 per lane, 0.9
+ * ms at one per four cycles) and by LDS latency at the three waves per SIMD
+ * that 52 KB per workgroup leave: without its input loads it takes 1.2 ms.
  */
 #ifndef KTM_POSTFFT_H
 #define KTM_POSTFFT_H
@@ -122,7 +131,8 @@ template <int R> __device__ __forceinline__ constexpr int pf_slot(int k)
            : R == 8 ? 4 * (k & 1) + (k >> 1) : k;
 }
 
-template <int R, bool INV> __device__ __forceinline__ void pf_dft(double2 *v)
+/* HALF: the inputs of the second half are zero (R = 16) */
+template <int R, bool INV, bool HALF = false> __device__ __forceinline__ void pf_dft(double2 *v)
 {
     if (R == 2) {
         pf_dft2<INV>(v[0], v[1]);
@@ -150,7 +160,17 @@ template <int R, bool INV> __device__ __forceinline__ void pf_dft(double2 *v)
     } else {
         /* n = 4 n1 + n2: 4-point DFTs over n1, twiddle W16^(n2 k1), 4-point over n2 */
 #pragma unroll
-        for (int n2 = 0; n2 < 4; ++n2) pf_dft4<INV>(v[n2], v[4 + n2], v[8 + n2], v[12 + n2]);
+        for (int n2 = 0; n2 < 4; ++n2) {
+            if (HALF) {
+                const double2 a = v[n2], b = v[4 + n2], ib = pf_rot<INV>(b);
+                v[n2] = pf_add(a, b);
+                v[4 + n2] = pf_add(a, ib);
+                v[8 + n2] = pf_sub(a, b);
+                v[12 + n2] = pf_sub(a, ib);
+            } else {
+                pf_dft4<INV>(v[n2], v[4 + n2], v[8 + n2], v[12 + n2]);
+            }
+        }
 #pragma unroll
         for (int k1 = 1; k1 < 4; ++k1)
 #pragma unroll
@@ -163,134 +183,190 @@ template <int R, bool INV> __device__ __forceinline__ void pf_dft(double2 *v)
 
 __device__ __forceinline__ int pf_pad(int i) { return i + (i >> 4); }
 
-/* One Stockham pass of radix R, stride NS (points already combined), on the
- * transform of N points whose TPF threads include this one (index tj): the
- * N / R butterflies go round-robin over the threads.  MODE 0: LDS -> LDS;
- * 1: the first forward pass, input from Pro; 2: the first inverse pass,
- * input times G; 3: the last inverse pass, output to out. */
-template <class Pro, int N, int R, int NS, int TPF, bool INV, int MODE>
-__device__ __forceinline__ void pf_pass(double2 *buf, int tj, const double2 *__restrict__ tw,
-                                        const double2 *__restrict__ G, const float *in,
-                                        const float *fold, int64_t tra, int64_t ntraces, int ns,
-                                        float dt, float *out)
-{
-    constexpr int NBF = N / R, NB = (NBF + TPF - 1) / TPF, STEP = N / R;
-    static_assert(NB * R <= 16, "at most 16 points per thread");
-    constexpr bool GUARD = NBF % TPF != 0;  /* some threads idle in this pass */
-    double2 v[16];
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-        const int j = tj + b * TPF;
-        if (GUARD && j >= NBF) continue;
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const int u = j + r * STEP;
-            if (MODE == 1) {
-                double xa = 0.0, xb = 0.0;
-                if (u >= 1 && u < ns) {
-                    if (tra < ntraces) xa = Pro::x(in + tra * ns, fold + tra * ns, u, dt);
-                    if (tra + 1 < ntraces) xb = Pro::x(in + (tra + 1) * ns, fold + (tra + 1) * ns, u, dt);
-                }
-                v[b * R + r] = make_double2(xa, xb);
-            } else {
-                v[b * R + r] = buf[pf_pad(u)];
-                if (MODE == 2) v[b * R + r] = pf_mul(v[b * R + r], G[u]);
-            }
-        }
-        if (NS > 1) {
-            /* twiddle W_N^(r * (j mod NS) * N / (NS R)) of element r: the
-             * powers 1, 2, 4, 8 from the table, the others their products */
-            const int c = (j % NS) * (N / (NS * R));
-            double2 w[16];
-            w[1] = tw[c];
-            if (R > 2) w[2] = tw[2 * c];
-            if (R > 4) w[4] = tw[4 * c];
-            if (R > 8) w[8] = tw[8 * c];
-#pragma unroll
-            for (int r = 3; r < R; ++r) {
-                const int hi = r & (r - 1) ? (r & 8 ? 8 : r & 4 ? 4 : 2) : 0;
-                if (hi) w[r] = pf_mul(w[hi], w[r - hi]);
-            }
-#pragma unroll
-            for (int r = 1; r < R; ++r) v[b * R + r] = pf_mul(v[b * R + r], pf_conj<INV>(w[r]));
-        }
-        pf_dft<R, INV>(v + b * R);
-    }
-    if (MODE != 3) {
-        __syncthreads();                    /* every load of the pass done */
-#pragma unroll
-        for (int b = 0; b < NB; ++b) {
-            const int j = tj + b * TPF;
-            if (GUARD && j >= NBF) continue;
-            const int d0 = (j / NS) * NS * R + j % NS;
-#pragma unroll
-            for (int r = 0; r < R; ++r) buf[pf_pad(d0 + r * NS)] = v[b * R + pf_slot<R>(r)];
-        }
-        __syncthreads();                    /* every store of the pass done */
-    } else {
-        /* last pass: NS R = N, so the destination is j + r N / R */
-        constexpr double inv_n = 1.0 / (double)N;
-#pragma unroll
-        for (int b = 0; b < NB; ++b) {
-            const int j = tj + b * TPF;
-            if (GUARD && j >= NBF) continue;
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                const int t = j + r * STEP;
-                if (t < ns) {
-                    const double2 y = v[b * R + pf_slot<R>(r)];
-                    if (tra < ntraces) out[tra * ns + t] = t == 0 ? 0.0f : (float)(y.x * inv_n);
-                    if (tra + 1 < ntraces) out[(tra + 1) * ns + t] = t == 0 ? 0.0f : (float)(y.y * inv_n);
-                }
-            }
-        }
-    }
-}
-
-/* the passes of one direction: radix 16 with strides 1, 16, 256, ... and a
- * last pass of radix N / 16^k (2, 4, 8 or 12) when N is not a power of 16 */
-template <class Pro, int N, int NS, int TPF, bool INV, int FIRST, bool LAST_OUT>
-__device__ __forceinline__ void pf_passes(double2 *buf, int tj, const double2 *tw,
-                                          const double2 *G, const float *in, const float *fold,
-                                          int64_t tra, int64_t ntraces, int ns, float dt,
-                                          float *out)
-{
-    constexpr int REM = N / NS;             /* points left to combine */
-    constexpr int R = REM >= 16 ? 16 : REM;
-    constexpr bool LAST = NS * R == N;
-    constexpr int MODE = (LAST && LAST_OUT) ? 3 : FIRST;
-    pf_pass<Pro, N, R, NS, TPF, INV, MODE>(buf, tj, tw, G, in, fold, tra, ntraces, ns, dt, out);
-    if constexpr (!LAST)
-        pf_passes<Pro, N, NS * R, TPF, INV, 0, LAST_OUT>(buf, tj, tw, G, in, fold, tra, ntraces,
-                                                         ns, dt, out);
-}
-
-/* threads per workgroup and per transform for an N-point transform */
+/* points per wave, threads per transform and per workgroup, transforms per
+ * workgroup for an N-point transform */
 template <int N> struct PfShape {
-    static constexpr int NT = N == 8192 ? 512 : 256;
+    static constexpr int E = N == 3072 ? 768 : 1024;
     static constexpr int TPF = N == 3072 ? 256 : N / 16;
-    static constexpr int FPW = NT / TPF;   /* transforms per workgroup */
+    static constexpr int NT = TPF < 64 ? 64 : TPF;
+    static constexpr int FPW = NT / TPF;
     static constexpr int ROW = N + N / 16; /* padded LDS row (double2) */
     static constexpr int WAVES_PER_EU = N == 3072 ? 3 : 2;
 };
 
+struct PfArgs {
+    const float *in, *fold;
+    int64_t ntraces;
+    int ns;
+    float dt;
+    const double *G;
+    const double2 *tw;
+    float *out;
+};
+
+/* powers 1, 2, 4, 8 (as far as R needs them) of W_L^q, L points of N */
+template <int N, int L, int R>
+__device__ __forceinline__ void pf_twiddle(double2 *w, const double2 *__restrict__ tw, int q)
+{
+    w[1] = tw[q * (N / L)];
+    if (R > 2) w[2] = tw[2 * q * (N / L)];
+    if (R > 4) w[4] = tw[4 * q * (N / L)];
+    if (R > 8) w[8] = tw[8 * q * (N / L)];
+}
+
+/* element r of v times the power r of the twiddle, those not in w being
+ * products of them; SLOT: element r lies where pf_dft left it */
+template <int R, bool INV, bool SLOT> __device__ __forceinline__ void pf_turn(double2 *v, double2 *w)
+{
+#pragma unroll
+    for (int r = 3; r < R; ++r) {
+        const int hi = r & (r - 1) ? (r & 8 ? 8 : r & 4 ? 4 : 2) : 0;
+        if (hi) w[r] = pf_mul(w[hi], w[r - hi]);
+    }
+#pragma unroll
+    for (int r = 1; r < R; ++r) {
+        const int o = SLOT ? pf_slot<R>(r) : r;
+        v[o] = pf_mul(v[o], pf_conj<INV>(w[r]));
+    }
+}
+
+/* LDS accesses of a wave are done in order: the compiler has to keep it */
+__device__ __forceinline__ void pf_wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+/* The passes over blocks of L < N points, forward, filter and inverse, of the
+ * E points of one wave from buf on; e0: the wave's first point in its
+ * transform. */
+template <int N, int L>
+__device__ __forceinline__ void pf_inner(double2 *buf, int lane, int e0, const PfArgs &a)
+{
+    constexpr int E = PfShape<N>::E;
+    if constexpr (L == 16) {
+        constexpr int NBF = E / 16;
+        static_assert(NBF <= 64, "one block of 16 per lane");
+        if (NBF == 64 || lane < NBF) {
+            double g[16];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) g[r] = a.G[r * (N / 16) + ((e0 / 16 + lane) & (N >= 1024 ? -1 : N / 16 - 1))];
+            double2 v[16], x[16], *b = buf + 17 * lane;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) v[r] = b[r];
+            pf_dft<16, false>(v);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const double2 y = v[pf_slot<16>(r)];
+                x[r] = make_double2(y.x * g[r], y.y * g[r]);
+            }
+            pf_dft<16, true>(x);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) b[r] = x[pf_slot<16>(r)];
+        }
+    } else {
+        constexpr int R = L / 16 <= 16 ? L / 16 : L / 256;
+        constexpr int S = L / R, SP = S + S / 16, NB = E / R / 64;
+        static_assert(NB * R <= 16 && NB * R * 64 == E, "16 points per lane, all lanes busy");
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            const int j = lane + 64 * b, q = j % S;
+            double2 v[R], w[16], *p = buf + pf_pad(j / S * L + q);
+            pf_twiddle<N, L, R>(w, a.tw, q);
+#pragma unroll
+            for (int r = 0; r < R; ++r) v[r] = p[r * SP];
+            pf_dft<R, false>(v);
+            pf_turn<R, false, true>(v, w);
+#pragma unroll
+            for (int r = 0; r < R; ++r) p[r * SP] = v[pf_slot<R>(r)];
+        }
+        pf_wave_sync();
+        pf_inner<N, S>(buf, lane, e0, a);
+        pf_wave_sync();
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            const int j = lane + 64 * b, q = j % S;
+            double2 v[R], w[16], *p = buf + pf_pad(j / S * L + q);
+            pf_twiddle<N, L, R>(w, a.tw, q);
+#pragma unroll
+            for (int r = 0; r < R; ++r) v[r] = p[r * SP];
+            pf_turn<R, true, false>(v, w);
+            pf_dft<R, true>(v);
+#pragma unroll
+            for (int r = 0; r < R; ++r) p[r * SP] = v[pf_slot<R>(r)];
+        }
+    }
+}
+
 template <class Pro, int N>
 __global__ void __launch_bounds__(PfShape<N>::NT)
     __attribute__((amdgpu_waves_per_eu(PfShape<N>::WAVES_PER_EU)))
-k_postfft(const float *__restrict__ in, const float *__restrict__ fold, int64_t ntraces, int ns,
-          float dt, const double2 *__restrict__ G, const double2 *__restrict__ tw,
-          float *__restrict__ out)
+k_postfft(const PfArgs a)
 {
     typedef PfShape<N> S;
+    constexpr int M = N / 16, MP = M + M / 16;
     extern __shared__ double2 pf_lds[];
     const int tid = threadIdx.x;
-    const int f = tid / S::TPF, tj = tid % S::TPF;
-    double2 *buf = pf_lds + f * S::ROW;
+    /* 3072 points: 192 of the 256 threads work in the first and the last pass;
+     * which wave idles differs from workgroup to workgroup, since a wave's
+     * index in its workgroup fixes the SIMD it runs on */
+    const int rot = N == 3072 ? 64 * ((blockIdx.x >> 3) + (blockIdx.x >> 8)) : 0;
+    const int f = tid / S::TPF, tj = (tid + rot) % S::TPF;
+    const bool busy = S::TPF == M || tj < M;
+    double2 *p = pf_lds + f * S::ROW + pf_pad(tj);
     const int64_t tra = ((int64_t)blockIdx.x * S::FPW + f) * 2;
-    pf_passes<Pro, N, 1, S::TPF, false, 1, false>(buf, tj, tw, G, in, fold, tra, ntraces, ns, dt,
-                                                  out);
-    pf_passes<Pro, N, 1, S::TPF, true, 2, true>(buf, tj, tw, G, in, fold, tra, ntraces, ns, dt,
-                                                out);
+    double2 v[16], w[16];
+    if (busy) {
+        /* Inputs u >= N / 2 >= ns are zeros.  All samples are asked for at once,
+         * where there is none at an index that has one: behind a branch each,
+         * their 16 latencies in a row took 0.4 ms of 160,000 traces' 1.9. */
+        const int64_t last = a.ntraces - 1;
+        const int64_t ta = (tra < last ? tra : last) * a.ns, tb = (tra + 1 < last ? tra + 1 : last) * a.ns;
+        float3 ka[8] = {}, kb[8] = {};
+        if (a.ns > 1) {
+#pragma unroll
+            for (int r = 0; r < 8; ++r) {
+                const int u = min(max(tj + r * M, 1), a.ns - 1);
+                ka[r] = Pro::load(a.in + ta, a.fold + ta, u);
+                kb[r] = Pro::load(a.in + tb, a.fold + tb, u);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        pf_twiddle<N, N, 16>(w, a.tw, tj);
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+            const int u = tj + r * M;
+            const bool in = u >= 1 && u < a.ns;
+            v[r] = make_double2(in && tra <= last ? Pro::value(ka[r], u, a.dt) : 0.0,
+                                in && tra < last ? Pro::value(kb[r], u, a.dt) : 0.0);
+        }
+        pf_dft<16, false, true>(v);
+        pf_turn<16, false, true>(v, w);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) p[r * MP] = v[pf_slot<16>(r)];
+    }
+    if (N > S::E) __syncthreads(); else pf_wave_sync();
+    const int wave = tid / 64, e0 = wave * S::E;
+    pf_inner<N, M>(pf_lds + pf_pad(e0), tid % 64, N > S::E ? e0 : 0, a);
+    if (N > S::E) __syncthreads(); else pf_wave_sync();
+    if (!busy) return;
+    pf_twiddle<N, N, 16>(w, a.tw, tj);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) v[r] = p[r * MP];
+    pf_turn<16, true, false>(v, w);
+    pf_dft<16, true>(v);
+    constexpr double inv_n = 1.0 / (double)N;
+    float *o = a.out + tra * a.ns;
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {           /* t >= N / 2 >= ns is not stored */
+        const int t = tj + r * M;
+        if (t < a.ns) {
+            const double2 y = v[pf_slot<16>(r)];
+            if (tra < a.ntraces) o[t] = t == 0 ? 0.0f : (float)(y.x * inv_n);
+            if (tra + 1 < a.ntraces) o[a.ns + t] = t == 0 ? 0.0f : (float)(y.y * inv_n);
+        }
+    }
 }
 
 /* The transform length for ns samples: the smallest of 256, 512, 1024, 2048,
@@ -331,81 +407,79 @@ static inline void postfft_host_fft(double *G, int n, const double *tw, int step
     }
 }
 
-/* Host tables of the FFT form for the kernel h[0..ns): G = DFT_N(g) and the
- * twiddles exp(-2 pi i m / N), m < N, each N double2 ({re, im}) into
- * caller arrays.  G in double, by radix-2 transforms (of the three decimated
- * sequences for 3072 points); twiddles from cos/sin of the exact angle.
- * Returns nonzero if out of memory. */
-static inline int postfft_host_tables(const double *h, int ns, int n, double *G, double *tw)
+/* Host tables of the FFT form for the even kernel h[0..ns): G = DFT_N(g), N
+ * doubles in the order in which k_postfft reads it, and the twiddles exp(-2 pi i m / N), m < N, N double2 ({re, im}),
+ * into caller arrays; work: 2 N doubles.  G in double, by radix-2 transforms
+ * (of the three decimated sequences for 3072 points); twiddles from cos/sin
+ * of the exact angle. */
+static inline void postfft_host_tables(const double *h, int ns, int n, double *Gr, double *tw,
+                                       double *G)
 {
     const double two_pi = 6.283185307179586476925286766559;
     for (int m = 0; m < n; ++m) {
         tw[2 * m] = cos(two_pi * m / n);
         tw[2 * m + 1] = -sin(two_pi * m / n);
     }
-    if (n & (n - 1)) {
-        /* n = 3 m, m a power of two: the transforms F_r of the three sequences
-         * g[3 j + r] in G's thirds, then G[k] = sum_r W^(r k) F_r[k mod m] */
-        const int m = n / 3;
-        double *F = (double *)malloc(sizeof(double) * 2 * (size_t)n);
-        if (!F) return 1;
-        for (int j = 0; j < n; ++j) {
-            const int d = j < ns ? j : j > n - ns ? ns - (n - j) : -1;   /* g[n - e] = h[ns - e] */
-            double *f = F + 2 * (j % 3 * m + j / 3);
-            f[0] = d >= 0 ? h[d] : 0.0;
-            f[1] = 0.0;
-        }
-        for (int r = 0; r < 3; ++r) postfft_host_fft(F + 2 * r * m, m, tw, 3);
-        for (int k = 0; k < n; ++k) {
-            double re = 0.0, im = 0.0;
-            for (int r = 0; r < 3; ++r) {
-                const double *f = F + 2 * (r * m + k % m), *w = tw + 2 * ((long long)r * k % n);
-                re += f[0] * w[0] - f[1] * w[1];
-                im += f[0] * w[1] + f[1] * w[0];
-            }
-            G[2 * k] = re;
-            G[2 * k + 1] = im;
-        }
-        free(F);
-        return 0;
+    const int r = n & (n - 1) ? 3 : 1, l = n / r;
+    /* the transforms F_q of the r sequences g[r j + q] in G's r parts, then
+     * G[k] = sum_q W^(q k) F_q[k mod l] */
+    for (int j = 0; j < n; ++j) {
+        const int d = j < ns ? j : j > n - ns ? ns - (n - j) : -1;   /* g[n - e] = h[ns - e] */
+        double *f = G + 2 * (j % r * l + j / r);
+        f[0] = d >= 0 ? h[d] : 0.0;
+        f[1] = 0.0;
     }
-    for (int j = 0; j < n; ++j) G[2 * j] = G[2 * j + 1] = 0.0;
-    for (int d = 0; d < ns; ++d) G[2 * d] = h[d];
-    for (int d = 1; d < ns; ++d) G[2 * (n - d)] = h[ns - d];
-    postfft_host_fft(G, n, tw, 1);
-    return 0;
+    for (int q = 0; q < r; ++q) postfft_host_fft(G + 2 * q * l, l, tw, r);
+    /* position m = 16 b + t of block b: digits of radix 16, then n / 256 (of 512
+     * for 8192: 2, then 16), then 16, the first digit of k the lowest */
+    for (int m = 0; m < n; ++m) {
+        int k = 0, one = 1;
+        for (int len = n, p = m; len > 1;) {
+            const int rad = len == n || len <= 16 ? 16 : len / 16 <= 16 ? len / 16 : len / 256;
+            len /= rad;
+            k += one * (p / len);
+            one *= rad;
+            p %= len;
+        }
+        double re = 0.0;
+        for (int q = 0; q < r; ++q) {
+            const double *f = G + 2 * (q * l + k % l), *w = tw + 2 * ((long long)q * k % n);
+            re += f[0] * w[0] - f[1] * w[1];
+        }
+        Gr[m % 16 * (n / 16) + m / 16] = re;
+    }
 }
 
 /* Launch k_postfft<Pro> over ntraces traces of ns samples; G and tw are the
  * device copies of postfft_host_tables for n = postfft_size(ns). */
 template <class Pro>
 static hipError_t postfft_launch(const float *in, const float *fold, int64_t ntraces, int ns,
-                                 float dt, const double2 *G, const double2 *tw, float *out,
+                                 float dt, const double *G, const double2 *tw, float *out,
                                  hipStream_t stream)
 {
-    typedef void (*fn_t)(const float *, const float *, int64_t, int, float, const double2 *,
-                         const double2 *, float *);
+    void (*fn)(const PfArgs) = nullptr;
     const int n = postfft_size(ns);
-    fn_t fn = nullptr;
-    int nt = 256, fpw = 1;
+    int nt = 0, fpw = 0;
+#define PF_CASE(n) case n: fn = k_postfft<Pro, n>; nt = PfShape<n>::NT; fpw = PfShape<n>::FPW; break
     switch (n) {
-    case 256: fn = k_postfft<Pro, 256>; fpw = PfShape<256>::FPW; break;
-    case 512: fn = k_postfft<Pro, 512>; fpw = PfShape<512>::FPW; break;
-    case 1024: fn = k_postfft<Pro, 1024>; fpw = PfShape<1024>::FPW; break;
-    case 2048: fn = k_postfft<Pro, 2048>; fpw = PfShape<2048>::FPW; break;
-    case 3072: fn = k_postfft<Pro, 3072>; fpw = PfShape<3072>::FPW; break;
-    case 4096: fn = k_postfft<Pro, 4096>; fpw = PfShape<4096>::FPW; break;
-    case 8192: fn = k_postfft<Pro, 8192>; fpw = PfShape<8192>::FPW; nt = 512; break;
+    PF_CASE(256);
+    PF_CASE(512);
+    PF_CASE(1024);
+    PF_CASE(2048);
+    PF_CASE(3072);
+    PF_CASE(4096);
+    PF_CASE(8192);
     default: return hipErrorInvalidValue;
     }
+#undef PF_CASE
+    const PfArgs a = {in, fold, ntraces, ns, dt, G, tw, out};
     const size_t lds = sizeof(double2) * (size_t)fpw * (size_t)(n + n / 16);
     const int64_t nblk = (ntraces + 2 * fpw - 1) / (2 * fpw);
     if (nblk > 0x7fffffffLL) return hipErrorInvalidValue;
     hipError_t e = hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize,
                                        (int)lds);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(fn, dim3((unsigned)nblk), dim3(nt), lds, stream, in, fold, ntraces, ns, dt,
-                       G, tw, out);
+    hipLaunchKernelGGL(fn, dim3((unsigned)nblk), dim3(nt), lds, stream, a);
     return hipGetLastError();
 }
 

@@ -63,7 +63,7 @@ k_postmx(const float *__restrict__ in, const float *__restrict__ fold, int64_t n
             const int j = e / PM_UC, ul = e - j * PM_UC, u = c0 + ul;
             const int64_t tr = tr0 + j;
             double v = 0.0;
-            if (tr < ntraces && u >= 1 && u < ns) v = Pro::x(in + tr * ns, fold + tr * ns, u, dt);
+            if (tr < ntraces && u >= 1 && u < ns) v = Pro::value(Pro::load(in + tr * ns, fold + tr * ns, u), u, dt);
             xs[ul * PM_LD + j] = v;
         }
         __syncthreads();

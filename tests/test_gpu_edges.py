@@ -140,6 +140,33 @@ def test_plan_size_limits(cuda):
         assert e.value.status == _lib.KTM_ERR_UNSUPPORTED
 
 
+@pytest.mark.parametrize("ns", [37, 128, 200, 300, 512, 700, 1500, 2000])
+def test_poststack_many_traces(cuda, ns):
+    """Several transforms per wave (N = 256 to 1024), several waves per transform
+    and several workgroups, the last one partly filled: 61 traces of one image
+    against an FFT in double of the same single-precision differences.  The
+    result is rounded to float once, so its distance is at most 2^-24 of its
+    norm, plus the double transforms' own error (below 1e-13)."""
+    print(f"case: post-stack of 61 traces at ns={ns}", flush=True)
+    sv = small_line(ns, ncols=61, jobs_x=1)
+    plan = Plan(sv.cfg, sv.ns, sv.dt, sv.vel)
+    g = torch.Generator(device=cuda).manual_seed(ns)
+    km = torch.randn(plan.image_shape, generator=g, device=cuda)
+    fold = torch.randint(1, 40, plan.image_shape, generator=g, device=cuda).float()
+    out = plan.poststack(km, fold).cpu().numpy().reshape(-1, ns)
+    _, aa = oracle.alias_filter(sv.cfg, sv.ns, sv.dt)
+    k, f = km.cpu().numpy().reshape(-1, ns), fold.cpu().numpy().reshape(-1, ns)
+    dt = np.float32(sv.dt)
+    d = np.zeros((k.shape[0], ns))
+    d[:, 1:] = -dt * np.arange(1, ns, dtype=np.float32) * (k[:, 1:] - k[:, :-1]) * dt / f[:, 1:]
+    ref = np.fft.ifft(np.fft.fft(d, axis=-1) * aa.astype(np.float64), axis=-1).real
+    ref[:, 0] = 0.0
+    assert k.shape[0] == 61
+    r = float(np.linalg.norm(out - ref) / np.linalg.norm(ref))
+    print(f"  relL2 {r:.2e}", flush=True)
+    assert r <= 2.0 ** -24 + 1e-13
+
+
 @pytest.mark.parametrize("ns", [4, 128, 129, 512, 1024, 1025, 1536, 1537, 2048, 2049, 4096, 4097,
                                 6144])
 def test_poststack_long_traces(cuda, ns):
