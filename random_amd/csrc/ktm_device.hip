@@ -2950,10 +2950,21 @@ static int pixel_tables(const ktm_plan *cp, hipStream_t hs)
     return KTM_OK;
 }
 
+/* Workgroups below which a demigration takes its columns in parts (four rounds
+ * of the 512 that run at once), the parts at most, and the bound of its
+ * workspace (256 MiB) */
+#define DM_TARGET_WGS 2048
+#define DM_MAX_PARTS 16
+#define DM_SUM_MAX_WORDS (32ll << 20)
+
 /* the demigration trace order of n traces (sorted by k_demig_keys) into
- * plan-owned buffers; *order points at the sorted indices */
-static int demig_order(const ktm_plan *cp, const ktm_trace_geom *geom, int64_t n, hipStream_t hs,
-                       const int32_t **order)
+ * plan-owned buffers; *order points at the sorted indices.  The buffers grow
+ * with n, and with them the sums of column parts, up to the most traces that
+ * take parts (tb a workgroup): a call of no more traces than an earlier one
+ * allocates and frees nothing.  Without memory for the sums a call is not
+ * divided. */
+static int demig_order(const ktm_plan *cp, const ktm_trace_geom *geom, int64_t n, int tb,
+                       hipStream_t hs, const int32_t **order)
 {
     ktm_plan *p = const_cast<ktm_plan *>(cp);
     const ktm_setup *s = &p->tb.s;
@@ -2968,6 +2979,20 @@ static int demig_order(const ktm_plan *cp, const ktm_trace_geom *geom, int64_t n
             return KTM_ERR_NOMEM;
         if (hipMalloc((void **)&p->d_dm_idx, 2 * (size_t)n * sizeof(int32_t)) != hipSuccess)
             return KTM_ERR_NOMEM;
+        int64_t words = (n < (int64_t)DM_TARGET_WGS * tb ? n : (int64_t)DM_TARGET_WGS * tb) * s->ns;
+        if (words > DM_SUM_MAX_WORDS) words = DM_SUM_MAX_WORDS;
+        if ((size_t)words > p->dm_sum_cap) {
+            if (p->d_dm_sum) HIP_TRY(hipFree(p->d_dm_sum));
+            p->d_dm_sum = nullptr;
+            p->dm_sum_cap = 0;
+            if (hipMalloc((void **)&p->d_dm_sum, (size_t)words * sizeof(unsigned long long)) ==
+                hipSuccess) {
+                p->dm_sum_cap = (size_t)words;
+            } else {                        /* no memory for parts: undivided */
+                p->d_dm_sum = nullptr;
+                (void)hipGetLastError();
+            }
+        }
         p->dm_cap = (size_t)n;
     }
     uint64_t *k_in = p->d_dm_keys, *k_out = p->d_dm_keys + n;
@@ -2991,13 +3016,6 @@ static int demig_order(const ktm_plan *cp, const ktm_trace_geom *geom, int64_t n
     *order = i_out;
     return KTM_OK;
 }
-
-/* Workgroups below which a demigration takes its columns in parts (four rounds
- * of the 512 that run at once), the parts at most, and the bound of its
- * workspace (256 MiB) */
-#define DM_TARGET_WGS 2048
-#define DM_MAX_PARTS 16
-#define DM_SUM_MAX_WORDS (32ll << 20)
 
 static int demigrate(const ktm_plan *p, const float *km, const ktm_trace_geom *geom, int64_t ntr,
                      float *traces, bool fast, void *stream);
@@ -3082,27 +3100,16 @@ static int demigrate(const ktm_plan *p, const float *km, const ktm_trace_geom *g
         b.geom = geom + i0;
         b.traces = traces + i0 * s->ns;
         b.ntr = n;
-        if ((st = demig_order(p, b.geom, n, hs, &b.order)) != KTM_OK) return st;
+        if ((st = demig_order(p, b.geom, n, a.tb, hs, &b.order)) != KTM_OK) return st;
         const int64_t nblk = (n + a.tb - 1) / a.tb;
-        /* few traces: their columns in parts, up to what a bounded workspace
-         * of sums allows */
-        const int64_t words = n * s->ns;
+        /* few traces: their columns in parts, where the workspace of sums
+         * holds them */
         int64_t parts = (DM_TARGET_WGS + nblk - 1) / nblk;
         if (parts > DM_MAX_PARTS) parts = DM_MAX_PARTS;
-        if (words > DM_SUM_MAX_WORDS) parts = 1;
+        if ((size_t)(n * s->ns) > p->dm_sum_cap) parts = 1;
         if (parts > 1) {
-            ktm_plan *pm = const_cast<ktm_plan *>(p);
-            if ((size_t)words > p->dm_sum_cap) {
-                if (p->d_dm_sum) HIP_TRY(hipFree(p->d_dm_sum));
-                pm->d_dm_sum = nullptr;
-                pm->dm_sum_cap = 0;
-                if (hipMalloc((void **)&pm->d_dm_sum, (size_t)words * sizeof(unsigned long long)) !=
-                    hipSuccess)
-                    return KTM_ERR_NOMEM;
-                pm->dm_sum_cap = (size_t)words;
-            }
             b.gsum = p->d_dm_sum;
-            hipLaunchKernelGGL(k_zero_u64, dim3(2048), dim3(256), 0, hs, b.gsum, words);
+            hipLaunchKernelGGL(k_zero_u64, dim3(2048), dim3(256), 0, hs, b.gsum, n * s->ns);
         }
         hipLaunchKernelGGL(fn, dim3((unsigned)nblk, (unsigned)parts), dim3(8 * KTM_WAVE), lds, hs, b);
         if (parts > 1)

@@ -56,11 +56,11 @@ int  ktm_rt_event_elapsed_ms(void *e0, void *e1, float *ms);
 int  ktm_rt_copy_h2d_async(void *dst, const void *src, size_t bytes, void *s);
 int  ktm_rt_copy_d2h_async(void *dst, const void *src, size_t bytes, void *s);
 
-/* Shared by the C host code: big-endian helpers. */
 /* g[m] = (1/ns) sum_k a[k] b[k] cos(2 pi k m / ns), m < ns (b NULL: 1), in long
  * double: the circular kernel of an even spectrum */
 int ktm_even_kernel(const float *a, const float *b, int ns, double *g);
 
+/* Shared by the C host code: big-endian helpers. */
 static inline void ktm_put_be32(uint8_t *o, uint32_t u)
 {
     o[0] = (uint8_t)(u >> 24); o[1] = (uint8_t)(u >> 16);

@@ -6,6 +6,7 @@ import pytest
 import torch
 
 from random_amd import surveys
+from random_amd._lib import check, lib
 from random_amd.ktm import Plan
 from random_amd.lsm import Operator, cgls, dot64, dot_test, migrate_op, time_gain
 
@@ -222,3 +223,27 @@ def test_demigration_of_few_traces_bitexact(cuda, ns, take, fast):
     got = plan.demigrate(m, geom[at].contiguous(), fast=fast)
     assert bool(want.any())
     assert torch.equal(got, want[at])
+
+
+def test_demigration_of_few_traces_allocates_nothing_after_many(cuda):
+    """After one call on many traces, calls on fewer (their columns in parts)
+    take no further device memory, and fresh plans give the same bits."""
+    print("case: 17,000, 130, 1000 of 17,000 traces x 301 samples", flush=True)
+    sv = surveys.line2d(nshots=850, nrecv_side=10, shot_dx=0.5, ns=301, ncols=30, nscat=2,
+                        x0=130.0, t0_range=(0.01, 0.02))
+    plan = Plan(sv.cfg, sv.ns, sv.dt, sv.vel)
+    m = torch.randn(plan.image_shape, device=cuda)
+    geom = plan.geometry(torch.from_numpy(sv.coords).to(cuda))
+    parts = [geom[:n].contiguous() for n in (130, 1000)]
+    want = [Plan(sv.cfg, sv.ns, sv.dt, sv.vel).demigrate(m, g) for g in parts]
+    plan.demigrate(m, geom)
+    got = [torch.empty_like(w) for w in want]
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    for g, o in zip(parts, got):
+        check(lib().ktm_demigrate(plan._h, m.data_ptr(), g.data_ptr(), g.shape[0], o.data_ptr(),
+                                  torch.cuda.current_stream().cuda_stream), "ktm_demigrate")
+    torch.cuda.synchronize()
+    assert torch.cuda.mem_get_info()[0] == free
+    for w, o in zip(want, got):
+        assert bool(w.any()) and torch.equal(o, w)
