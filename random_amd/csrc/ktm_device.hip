@@ -945,8 +945,8 @@ k_migrate(const MigArgs a)
     }
 
     /* Kahan variants: the taps are summed onto y = -c in plain FP32 over
-     * 2 KTM_KAHAN_FOLD chunks (at most 2 KTM_KAHAN_FOLD C terms, error
-     * <= (terms - 1) u times their magnitudes) and added to the image with one
+     * 2 KTM_KAHAN_FOLD chunks of at most 4 rows or half as many of 8 (error
+     * <= (terms - 1) u times the terms' magnitudes) and added to the image with one
      * compensated step, which keeps the compensated error bound of order
      * u * sum |f| at a fraction of the per-tap cost.  Plain variants add
      * every tap into the image in trace order, as the reference does. */
@@ -1232,7 +1232,7 @@ k_migrate(const MigArgs a)
                 }
                 qi = -1;
             }
-            if (KAHAN && wend && (nfold += WN) >= 2 * KTM_KAHAN_FOLD) {
+            if (KAHAN && wend && (nfold += C > 4 ? WN * (C / 4) : WN) >= 2 * KTM_KAHAN_FOLD) {
                 nfold = 0;
                 fold_y();
             }
@@ -2554,16 +2554,24 @@ static double mig_cost(int K, int W, int NW, int64_t ncol, bool fast)
 static MigShape pick_migrate(int ns, int accum, int64_t ncol)
 {
     /* every shape, by samples per column; the ring of rows within half of a
-     * CU's LDS (two workgroups of 8 waves) or all of it (one of 16) */
+     * CU's LDS (two workgroups of 8 waves) or all of it (one of 16).  Chunks
+     * of 8 rows wherever that ring holds two of them, with windows of up to 16
+     * traces as it allows: half the barriers of chunks of 4 and twice the rows
+     * in flight.  The 800-column, 1001-sample line (4 x 4) 2.80 -> 2.41 ms,
+     * 12,000 traces into 1600 columns x 4 classes of 640 samples (10 x 1) 3.31
+     * -> 3.13 and of 2001 (8 x 4) 8.90 -> 8.21, 500 samples into 60 columns (2 x
+     * 4) 0.78 -> 0.70; compensated sums and the relaxed index 2 to 13 % as
+     * well.  1280 and 1536 samples and beyond 2048 keep 4 (two chunks of 8 do
+     * not fit). */
     static const struct { int cap, K, W, NW; MigShape (*make)(int); } S[] = {
-        {256, 2, 2, 8, mig_shape<2, 2, 8, 4, 4>},    {384, 6, 1, 8, mig_shape<6, 1, 8, 4, 4>},
-        {512, 2, 4, 8, mig_shape<2, 4, 8, 4, 4>},    {512, 4, 2, 8, mig_shape<4, 2, 8, 4, 4>},
-        {512, 8, 1, 8, mig_shape<8, 1, 8, 4, 4>},    {640, 10, 1, 8, mig_shape<10, 1, 8, 4, 4>},
-        {768, 6, 2, 8, mig_shape<6, 2, 8, 4, 3>},    {768, 12, 1, 8, mig_shape<12, 1, 8, 4, 3>},
-        {1024, 2, 8, 8, mig_shape<2, 8, 8, 4, 3>},   {1024, 4, 4, 8, mig_shape<4, 4, 8, 4, 3>},
-        {1024, 8, 2, 8, mig_shape<8, 2, 8, 4, 3>},   {1280, 10, 2, 8, mig_shape<10, 2, 8, 4, 2>},
+        {256, 2, 2, 8, mig_shape<2, 2, 8, 8, 2>},    {384, 6, 1, 8, mig_shape<6, 1, 8, 8, 2>},
+        {512, 2, 4, 8, mig_shape<2, 4, 8, 8, 2>},    {512, 4, 2, 8, mig_shape<4, 2, 8, 8, 2>},
+        {512, 8, 1, 8, mig_shape<8, 1, 8, 8, 2>},    {640, 10, 1, 8, mig_shape<10, 1, 8, 8, 2>},
+        {768, 6, 2, 8, mig_shape<6, 2, 8, 8, 2>},    {768, 12, 1, 8, mig_shape<12, 1, 8, 8, 2>},
+        {1024, 2, 8, 8, mig_shape<2, 8, 8, 8, 1>},   {1024, 4, 4, 8, mig_shape<4, 4, 8, 8, 1>},
+        {1024, 8, 2, 8, mig_shape<8, 2, 8, 8, 1>},   {1280, 10, 2, 8, mig_shape<10, 2, 8, 4, 2>},
         {1536, 6, 4, 8, mig_shape<6, 4, 8, 4, 2>},   {1536, 12, 2, 8, mig_shape<12, 2, 8, 4, 2>},
-        {2048, 8, 4, 16, mig_shape<8, 4, 16, 4, 3>}, {2560, 10, 4, 16, mig_shape<10, 4, 16, 4, 2>},
+        {2048, 8, 4, 16, mig_shape<8, 4, 16, 8, 1>}, {2560, 10, 4, 16, mig_shape<10, 4, 16, 4, 2>},
         {3072, 12, 4, 16, mig_shape<12, 4, 16, 4, 2>}, {4096, 8, 8, 16, mig_shape<8, 8, 16, 2, 2>},
         {5120, 10, 8, 16, mig_shape<10, 8, 16, 2, 2>}, {6144, 12, 8, 16, mig_shape<12, 8, 16, 2, 2>}};
     /* compensated sums of a small image are split along the traces instead */

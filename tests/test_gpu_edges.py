@@ -286,3 +286,17 @@ def test_adjoint_at_lane_layout_boundaries(cuda, ns, fast):
     lhs, rhs, rel = dot_test(op, d, m)
     print(f"  rel {rel:.2e}", flush=True)
     assert rel <= 1e-5
+
+
+@pytest.mark.parametrize("ns", [200, 380, 500, 630, 700, 1000, 2000])
+@pytest.mark.parametrize("ntr", [7, 8, 9, 63, 71, 72, 73])
+def test_chunks_of_eight_rows_bitexact(cuda, ns, ntr):
+    """Trace counts around chunks of eight staged rows and the 64 traces whose
+    gates are evaluated at once, the last chunk short, for small images and for
+    offset classes that fill the widest lanes."""
+    for nh, ncols in ((1, 9), (600, 9)):
+        print(f"case: {ntr} traces x {ns} samples, {ncols} columns x {nh} classes", flush=True)
+        sv = small_line(ns, nshots=8, nrecv_side=10, ncols=ncols, jobs_x=1, nh=nh, dh=900.0 if nh == 1 else 100.0)
+        sv.coords = sv.coords[np.random.default_rng(ntr).permutation(sv.ntr)[:ntr]].copy()
+        tr = np.random.default_rng(ns).standard_normal((ntr, ns)).astype(np.float32)
+        bitexact_case(sv, tr, cuda)
