@@ -34,10 +34,10 @@ BYTES_FP32 = 12.0   # three FP32 trace taps per contribution
 BYTES_HALF = 6.0    # three 16-bit taps
 METRIC = "G trace×image-pt contributions/s, %HBM roofline; BF16-trace vs FP32 at err"
 # HBM bytes per launch of k_migrate on this workload, from rocprofv3 --pmc
-# FETCH_SIZE (465,868,004 KiB, scaled x2.0) + WRITE_SIZE (1,882,132 KiB, x1.0),
+# FETCH_SIZE (778,777,929 KiB, scaled x2.0) + WRITE_SIZE (1,895,596 KiB, x1.0),
 # the scale factors being what the same counters read for a 1 GiB device copy
 # (profiles/k_migrate_area3d_1e6.md)
-TRAFFIC = 956_024_975_360
+TRAFFIC = 1_596_878_288_896
 
 
 def log(*a):
@@ -176,19 +176,21 @@ def valu_probe(dev, modes=tuple(VALU_MODES), waves_per_simd=(8,), target_ms=40.0
 # v_sqrt_f32, CVT = conversions, INT32 = v_add_u32 and v_lshl_add_u32;
 # v_min/v_med3, v_rndne, v_cmp, v_cndmask, v_readlane are in no class.
 KMIG_COUNTS = {
-    "exact": {"kernel": "k_migrate<12, 2, 8, false, false>", "contributions": 1806379368000,
-              "launch_ms": 942.06, "clock_ghz": 2.381, "valu": 488628380575,
-              "fma_f32": 94969484010, "add_f32": 97736566828, "mul_f32": 5946021325,
-              "trans_f32": 58496827853, "cvt": 30618638965, "int32": 61308780164,
-              "fma_f64": 5207598064, "add_f64": 370325576, "mul_f64": 1532187535,
-              "trans_f64": 744491152, "int64": 6386285760, "salu": 128120225353,
-              "lds": 36591172744},
-    "fast_kahan": {"kernel": "k_migrate<12, 2, 8, true, true>", "contributions": 1806379368000,
-                   "launch_ms": 748.03, "clock_ghz": 2.377, "valu": 371632398974,
-                   "fma_f32": 57804779776, "add_f32": 93506701952, "mul_f32": 2618300416,
-                   "trans_f32": 57806059776, "cvt": 28921269888, "int32": 81815267442,
+    "exact": {"kernel": "k_migrate<12, 2, 8, 4, 2, 4, false, false>",
+              "contributions": 1806379368000,
+              "launch_ms": 830.31, "clock_ghz": 2.382, "valu": 399382949703,
+              "fma_f32": 123061932252, "add_f32": 98669530749, "mul_f32": 3665208252,
+              "trans_f32": 59800466173, "cvt": 1804856454, "int32": 40646009684,
+              "fma_f64": 6214502668, "add_f64": 407006653, "mul_f64": 1808376454,
+              "trans_f64": 900188227, "int64": 3643298780, "salu": 144148207394,
+              "lds": 30424527558},
+    "fast_kahan": {"kernel": "k_migrate<12, 2, 8, 4, 1, 4, true, true>",
+                   "contributions": 1806379368000,
+                   "launch_ms": 555.53, "clock_ghz": 2.381, "valu": 270874098032,
+                   "fma_f32": 58724046808, "add_f32": 65307199744, "mul_f32": 910043424,
+                   "trans_f32": 58725326808, "cvt": 28921589888, "int32": 33421042194,
                    "fma_f64": 23040000, "add_f64": 0, "mul_f64": 15360000, "trans_f64": 3840000,
-                   "int64": 5722754464, "salu": 44813163964, "lds": 62309817190},
+                   "int64": 2629883638, "salu": 82696206820, "lds": 29442340168},
 }
 # the probe mode whose measured rate prices each class (SIMD cycles per
 # wave-instruction); INT32 at the v_add_u32 rate and the unclassified rest

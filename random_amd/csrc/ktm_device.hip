@@ -851,7 +851,7 @@ typedef __attribute__((address_space(1))) const void global_void;
  * through registers between two barriers and every sample past the trace on
  * the rare path: 16,000 traces x 1500 samples into 400 x 400 columns 295 ->
  * 253 ms, 20,000 BF16-stored x 1251 into 150 x 150 222 -> 187 ms, the
- * 40-shot line 3.75 -> 2.85 ms, 12 classes x 2503 samples x 500 columns 10.9 ->
+ * 40-shot line 3.75 -> 2.85 ms (2.40 with chunks of 8 rows), 12 classes x 2503 samples x 500 columns 10.9 ->
  * 6.75 ms.  12 waves of K = 8 (six per SIMD) measured the same as 8 of K = 12
  * with 1500 samples, 16 waves in one workgroup 15 % slower (all of a CU's waves
  * at one barrier); slot groups of 2, 4 and 6 within 3 % of 3. */
@@ -2537,7 +2537,7 @@ static MigShape mig_shape(int accum)
  * 5.0 -> 3.3 ms), 1251 10 x 2 instead of 12 x 2 (150 x 150 columns 187 -> 171),
  * 2503 10 x 4 instead of 12 x 4 (12 classes of 500 columns 6.75 -> 5.9), and 32
  * columns of 501 samples 2 x 4 instead of 4 x 2 (60 -> 45 us).  The 800-column,
- * 1001-sample line: 4 x 4 2.96 ms, 8 x 2 3.92, 2 x 8 3.22. */
+ * 1001-sample line, chunks of 4 rows: 4 x 4 2.96 ms, 8 x 2 3.92, 2 x 8 3.22. */
 static double mig_cost(int K, int W, int NW, int64_t ncol, bool fast)
 {
     static const double rate[5] = {0.0, 0.40, 0.65, 0.85, 1.0};
