@@ -723,6 +723,10 @@ __device__ __forceinline__ float clamp_ns(float q, float hi)
     return __builtin_amdgcn_fmed3f(q, 0.0f, hi);
 }
 
+/* a non-negative float without infinity and NaN, the largest finite one in
+ * their place */
+__device__ __forceinline__ float finite(float x) { return fminf(x, 3.402823466e38f); }
+
 /* The exact variants' form of q, in units of nsh = ns + 1/2: with
  * rsn = RN(1/(v2 dt^2 nsh^2)) and tqn = RN(t^2/(4 nsh^2)) (double, rounded
  * once)
@@ -732,10 +736,17 @@ __device__ __forceinline__ float clamp_ns(float q, float hi)
  * as above (rs and the FMA), so |p nsh - Q| <= 7u Q holds unchanged.  p is
  * limited to 1 by the clamp modifier of its sum, at no cost (a v_med3 is a
  * quarter-rate instruction): a limited sample has Q > ns for certain, its
- * index is ns, and half a sample from an integer it is never ambiguous. */
+ * index is ns, and half a sample from an integer it is never ambiguous.
+ * A trace without a position (NaN or infinite in the caller's geometry), or a
+ * velocity whose square underflows, has no traveltime: the reference arithmetic
+ * gives NaN or infinity, index ns.  So that p is never NaN (which the limit turns
+ * into 0, and floor_p into an index of -1), rsn and the squared distances are
+ * kept finite: such a sample is past the trace by the limit, or ambiguous (both
+ * distances 0). */
 __device__ __forceinline__ float fast_rsn(float v2, float dt, float nsh)
 {
-    return (float)(1.0 / ((double)v2 * (double)dt * (double)dt * ((double)nsh * (double)nsh)));
+    return finite(
+        (float)(1.0 / ((double)v2 * (double)dt * (double)dt * ((double)nsh * (double)nsh))));
 }
 __device__ __forceinline__ float fast_tqn(int t, float nsh)
 {
@@ -1048,6 +1059,10 @@ k_migrate(const MigArgs a)
             const float ax = IX - g0.x, ay = IY - g0.y, bx = IX - g0.z, by = IY - g0.w;
             g_is = ax * ax + ay * ay;
             g_ir = bx * bx + by * by;
+            if (SPEC) {
+                g_is = finite(g_is);
+                g_ir = finite(g_ir);
+            }
             const float cx = IX - g1.x, cy = IY - g1.y;
             const float ex = scx - g1.x, ey = scy - g1.y;
             gp = ex * ex + ey * ey < sthr && cx * cx + cy * cy < a.ap_x2thr;

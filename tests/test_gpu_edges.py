@@ -300,3 +300,33 @@ def test_chunks_of_eight_rows_bitexact(cuda, ns, ntr):
         sv.coords = sv.coords[np.random.default_rng(ntr).permutation(sv.ntr)[:ntr]].copy()
         tr = np.random.default_rng(ns).standard_normal((ntr, ns)).astype(np.float32)
         bitexact_case(sv, tr, cuda)
+
+
+@pytest.mark.parametrize("kahan", [False, True])
+@pytest.mark.parametrize("ns", [63, 301, 700, 1100, 1500, 2000, 2600, 5000])
+def test_traces_without_a_position_add_nothing(cuda, ns, kahan):
+    """A trace whose source or receiver position is NaN or infinite (in a
+    geometry that the caller made, with a CMP in reach) has no traveltime: the
+    reference arithmetic gives NaN or infinity, never an index below ns.  Image
+    and fold are those of the other traces."""
+    print(f"case: traces without a position, ns={ns}, kahan={kahan}", flush=True)
+    sv = small_line(ns, jobs_x=1)
+    plan = Plan(sv.cfg, sv.ns, sv.dt, sv.vel)
+    tr = torch.from_numpy(surveys.traces_numpy(sv)).to(cuda)
+    kw = dict(mode=_lib.PREP_CLOSED, accum=_lib.ACCUM_KAHAN) if kahan else {}
+    prepared, geom = plan.prep(tr, torch.from_numpy(sv.coords).to(cuda), kw.get("mode", 0))
+    without = torch.arange(sv.ntr, device=cuda) % 4 == 1
+    bad = geom.clone()
+    for i in torch.nonzero(without).flatten().tolist():
+        bad[i, i // 4 % 4] = float("nan") if i % 8 == 1 else float("inf")
+    out = []
+    for p, g in ((prepared, bad), (prepared[~without].contiguous(), geom[~without].contiguous())):
+        km, fold, comp = plan.new_image(kahan=kahan, device=cuda)
+        plan.migrate_block(p, g, km, fold, comp, **kw)
+        out.append((km, fold))
+    assert bool(out[1][0].any())
+    assert torch.equal(out[0][1], out[1][1])
+    if kahan:      # other sets of traces between the compensated steps
+        assert float((out[0][0] - out[1][0]).norm() / out[1][0].norm()) <= 1e-6
+    else:
+        assert torch.equal(out[0][0], out[1][0])
