@@ -1608,21 +1608,22 @@ struct DemigArgs {
     int lg_terms;                    /* 2^lg_terms >= nxp * nyp * ns, terms per g[T] at most */
 };
 
-/* the fixed point of g: km is scaled by 2^E, max |km| < 2^emax; |km 2^E| <
- * 2^51 in any case (to_fixed) */
+/* the fixed point of g: km is scaled by 2^E, max |km| < 2^emax, so that a sum
+ * of 2^lg_terms terms stays below 2^59 */
 __device__ __forceinline__ int demig_exponent(const DemigArgs &a)
 {
     const float amax = __uint_as_float(*a.amax);
     int emax = 0;
     if (amax > 0.0f) (void)frexpf(amax, &emax);
-    return min(59 - a.lg_terms, 51) - emax;
+    return 59 - emax - a.lg_terms;
 }
 
-/* trunc(m 2^E) as an integer, |m 2^E| < 2^51: the double sum with 1.5 * 2^52
- * holds it in its low bits (the compiler's float to 64-bit conversion takes
- * twice the instructions) */
-__device__ __forceinline__ unsigned long long to_fixed(float m, int E)
+/* trunc(m 2^E) as an integer.  NARROW (|m 2^E| < 2^51: a finite image of more
+ * than 128 samples): the double sum with 1.5 * 2^52 holds it in its low bits;
+ * the compiler's float to 64-bit conversion takes twice the instructions. */
+template <bool NARROW> __device__ __forceinline__ unsigned long long to_fixed(float m, int E)
 {
+    if (!NARROW) return (unsigned long long)(long long)ldexpf(m, E);
     constexpr double MAGIC = 6755399441055744.0;
     const double s = __builtin_trunc(__builtin_amdgcn_ldexp((double)m, E)) + MAGIC;
     return (unsigned long long)__double_as_longlong(s) -
@@ -1796,6 +1797,7 @@ k_demigrate(const DemigArgs a)
     const int nb = (int)min((int64_t)a.tb, a.ntr - b0);
     for (int e = tid; e < a.tb * ldg; e += 8 * KTM_WAVE) sg[e] = 0ull;
     const int E = demig_exponent(a);
+    const bool narrow = a.lg_terms >= 8 && __builtin_amdgcn_readfirstlane((int)*a.amax) < 0x7f800000;
     /* lane j < nb of every wave holds trace j of the workgroup */
     ktm_trace_geom g;
     memset(&g, 0, sizeof g);
@@ -1896,8 +1898,13 @@ k_demigrate(const DemigArgs a)
                 float m[K];
 #pragma unroll
                 for (int k = 0; k < K; ++k) m[k] = mk[to[k]];
+                if (narrow) {
 #pragma unroll
-                for (int k = 0; k < K; ++k) mq[k] = to_fixed(m[k], E);
+                    for (int k = 0; k < K; ++k) mq[k] = to_fixed<true>(m[k], E);
+                } else {
+#pragma unroll
+                    for (int k = 0; k < K; ++k) mq[k] = to_fixed<false>(m[k], E);
+                }
             }
             /* the source's roots, kept for the column's traces of one source */
             if (__float_as_uint(dIS2) != lastd) {

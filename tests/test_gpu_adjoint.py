@@ -247,3 +247,51 @@ def test_demigration_of_few_traces_allocates_nothing_after_many(cuda):
     assert torch.cuda.mem_get_info()[0] == free
     for w, o in zip(want, got):
         assert bool(w.any()) and torch.equal(o, w)
+
+
+def _near_line(ns, ncols):
+    """64 traces between the columns of a short line, a few samples away."""
+    sv = surveys.line2d(nshots=4, nrecv_side=8, ns=ns, ncols=ncols, nscat=1)
+    sv.coords[:, 0::2] = np.random.default_rng(ns).integers(0, 625 * ncols, (sv.ntr, 2))
+    plan = Plan(sv.cfg, sv.ns, sv.dt, sv.vel)
+    return plan, plan.geometry(torch.from_numpy(sv.coords).cuda())
+
+
+@pytest.mark.parametrize("fast", [False, True])
+@pytest.mark.parametrize("ns,ncols,bits", [(4, 1, 56), (16, 2, 53), (16, 4, 52), (16, 8, 51), (64, 2, 51),
+                                           (33, 4, 50), (128, 2, 50), (300, 9, 46)])
+def test_demigration_keeps_the_bits_its_terms_leave(cuda, ns, ncols, bits, fast):
+    """The sums are exact in units of 2^(emax + lg_terms - 59), 2^emax > max |km|
+    and 2^lg_terms >= the image's samples of one offset class: ones and values
+    of that size side by side give each other's traces exactly wherever they
+    do not meet."""
+    print(f"case: image of {ncols} x {ns} samples, values 1 and 2^-{bits}", flush=True)
+    plan, geom = _near_line(ns, ncols)
+    g = torch.Generator(device=cuda).manual_seed(ns)
+    small = torch.randint(-1, 2, plan.image_shape, generator=g, device=cuda).float()
+    one = torch.zeros_like(small)
+    one[0, 0, 0, ns // 2] = 1.0
+    small[0, 0, 0, ns // 2] = 0.0
+    a = plan.demigrate(one, geom, fast=fast)
+    b = plan.demigrate(small * 2.0 ** -bits, geom, fast=fast)
+    both = plan.demigrate(one + small * 2.0 ** -bits, geom, fast=fast)
+    apart = (a == 0) & (b != 0)
+    assert bool(a.any()) and bool(apart.any())
+    assert torch.equal(both[apart], b[apart])
+
+
+def test_demigration_of_an_image_with_nan(cuda):
+    """A NaN image sample adds nothing: the traces are those of the image with
+    a zero in its place (values up to 1, so the fixed point leaves them their
+    bits; it is then 2^-49 for 32 x 31 samples)."""
+    plan, geom = _near_line(31, 32)
+    g = torch.Generator(device=cuda).manual_seed(1)
+    m = 2.0 * torch.rand(plan.image_shape, generator=g, device=cuda) - 1.0
+    at = torch.rand(plan.image_shape, generator=g, device=cuda) < 0.1
+    m[at] = 0.0
+    want = plan.demigrate(m, geom)
+    m[at] = float("nan")
+    got = plan.demigrate(m, geom)
+    assert bool(want.any())
+    w = float(want.abs().max())
+    assert float((got - want).abs().max()) <= 2.0 ** -23 * w
