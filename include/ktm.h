@@ -269,7 +269,11 @@ int ktm_poststack(const ktm_plan *plan, const float *km, const float *fold,
  * km by powers of two; its quantum is max |km| * 2^(lg - 59), 2^lg >=
  * columns x ns.  It sorts the traces by (offset class, CMP cell) into
  * plan-owned buffers that grow on demand (a first call, or a larger ntr,
- * allocates). */
+ * allocates), and takes the columns of few traces in parts whose sums
+ * (at most 256 MiB, allocated with the sort buffers) a later call finds in
+ * place.  The sums are optional: without memory for them a call is not divided
+ * (same bits), and they are given back when another buffer of the plan needs
+ * the memory. */
 int ktm_demigrate(const ktm_plan *plan, const float *km, const ktm_trace_geom *geom,
                   int64_t ntr, float *traces, void *stream);
 /* ktm_demigrate with the traveltime index of KTM_INDEX_FAST (index =

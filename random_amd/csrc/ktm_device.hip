@@ -81,6 +81,7 @@ struct ktm_plan {
     uint32_t *d_dm_amax;    /* bits of max |km| of the last demigration */
     unsigned long long *d_dm_sum; /* sums of a demigration whose columns are in parts */
     size_t dm_sum_cap;      /* words of d_dm_sum */
+    int64_t dm_sum_ntr;     /* most traces of a call that asked for them */
     float *d_scratch;       /* this device's copy of `scratch` (ktm_migrate_block_static) */
     /* compensated migration of small images: partial images of parts 1..
      * parts_max-1 of a trace block, [part][km, fold, comp][image or region] */
@@ -2664,6 +2665,23 @@ static int parts_workspace(ktm_plan *p)
     return KTM_OK;
 }
 
+/* n elements that a call cannot do without.  The sums of column parts, which a
+ * demigration can do without, are given back for them (hipFree waits for the
+ * kernels that use them). */
+template <class T> static int plan_alloc(ktm_plan *p, T **dst, size_t n)
+{
+    for (;;) {
+        const hipError_t e = hipMalloc((void **)dst, n * sizeof(T));
+        if (e == hipSuccess) return KTM_OK;
+        *dst = nullptr;
+        (void)hipGetLastError();
+        if (e != hipErrorOutOfMemory || !p->d_dm_sum) return KTM_ERR_NOMEM;
+        (void)hipFree(p->d_dm_sum);
+        p->d_dm_sum = nullptr;
+        p->dm_sum_cap = 0;
+    }
+}
+
 /* FP32 filtered traces of a BF16/FP16 block, into stage (ntr * row floats)
  * or, when stage is NULL, into a workspace the plan owns and grows on demand
  * (the only allocation on the migration path) */
@@ -2679,8 +2697,7 @@ static int decode_block(const ktm_plan *cp, const void *prepared, int dtype,
             if (p->d_stage) HIP_TRY(hipFree(p->d_stage));
             p->d_stage = nullptr;
             p->stage_cap = 0;
-            if (hipMalloc((void **)&p->d_stage, need * sizeof(float)) != hipSuccess)
-                return KTM_ERR_NOMEM;
+            if (plan_alloc(p, &p->d_stage, need) != KTM_OK) return KTM_ERR_NOMEM;
             p->stage_cap = need;
         }
         dst = p->d_stage;
@@ -2967,8 +2984,8 @@ static int pixel_tables(const ktm_plan *cp, hipStream_t hs)
     if (p->d_pix_v2) return KTM_OK;
     const ktm_setup *s = &p->tb.s;
     const size_t n = (size_t)s->nxp * s->nyp * s->ns;
-    if (hipMalloc((void **)&p->d_pix_v2, n * sizeof(float)) != hipSuccess) return KTM_ERR_NOMEM;
-    if (hipMalloc((void **)&p->d_pix_rs, n * sizeof(float)) != hipSuccess) {
+    if (plan_alloc(p, &p->d_pix_v2, n) != KTM_OK) return KTM_ERR_NOMEM;
+    if (plan_alloc(p, &p->d_pix_rs, n) != KTM_OK) {
         (void)hipFree(p->d_pix_v2);
         p->d_pix_v2 = nullptr;
         return KTM_ERR_NOMEM;
@@ -2988,12 +3005,8 @@ static int pixel_tables(const ktm_plan *cp, hipStream_t hs)
 #define DM_SUM_MAX_WORDS (32ll << 20)
 
 /* the demigration trace order of n traces (sorted by k_demig_keys) into
- * plan-owned buffers; *order points at the sorted indices.  The buffers grow
- * with n, and with them the sums of column parts, up to the most traces that
- * take parts (tb a workgroup): a call of no more traces than an earlier one
- * allocates and frees nothing.  Without memory for the sums a call is not
- * divided. */
-static int demig_order(const ktm_plan *cp, const ktm_trace_geom *geom, int64_t n, int tb,
+ * plan-owned buffers that grow with n; *order points at the sorted indices */
+static int demig_order(const ktm_plan *cp, const ktm_trace_geom *geom, int64_t n,
                        hipStream_t hs, const int32_t **order)
 {
     ktm_plan *p = const_cast<ktm_plan *>(cp);
@@ -3005,24 +3018,8 @@ static int demig_order(const ktm_plan *cp, const ktm_trace_geom *geom, int64_t n
         p->d_dm_keys = nullptr;
         p->d_dm_idx = nullptr;
         p->dm_cap = 0;
-        if (hipMalloc((void **)&p->d_dm_keys, 2 * (size_t)n * sizeof(uint64_t)) != hipSuccess)
-            return KTM_ERR_NOMEM;
-        if (hipMalloc((void **)&p->d_dm_idx, 2 * (size_t)n * sizeof(int32_t)) != hipSuccess)
-            return KTM_ERR_NOMEM;
-        int64_t words = (n < (int64_t)DM_TARGET_WGS * tb ? n : (int64_t)DM_TARGET_WGS * tb) * s->ns;
-        if (words > DM_SUM_MAX_WORDS) words = DM_SUM_MAX_WORDS;
-        if ((size_t)words > p->dm_sum_cap) {
-            if (p->d_dm_sum) HIP_TRY(hipFree(p->d_dm_sum));
-            p->d_dm_sum = nullptr;
-            p->dm_sum_cap = 0;
-            if (hipMalloc((void **)&p->d_dm_sum, (size_t)words * sizeof(unsigned long long)) ==
-                hipSuccess) {
-                p->dm_sum_cap = (size_t)words;
-            } else {                        /* no memory for parts: undivided */
-                p->d_dm_sum = nullptr;
-                (void)hipGetLastError();
-            }
-        }
+        if (plan_alloc(p, &p->d_dm_keys, 2 * (size_t)n) != KTM_OK) return KTM_ERR_NOMEM;
+        if (plan_alloc(p, &p->d_dm_idx, 2 * (size_t)n) != KTM_OK) return KTM_ERR_NOMEM;
         p->dm_cap = (size_t)n;
     }
     uint64_t *k_in = p->d_dm_keys, *k_out = p->d_dm_keys + n;
@@ -3034,7 +3031,7 @@ static int demig_order(const ktm_plan *cp, const ktm_trace_geom *geom, int64_t n
         if (p->d_dm_tmp) HIP_TRY(hipFree(p->d_dm_tmp));
         p->d_dm_tmp = nullptr;
         p->dm_tmp_bytes = 0;
-        if (hipMalloc(&p->d_dm_tmp, need) != hipSuccess) return KTM_ERR_NOMEM;
+        if (plan_alloc(p, (char **)&p->d_dm_tmp, need) != KTM_OK) return KTM_ERR_NOMEM;
         p->dm_tmp_bytes = need;
     }
     hipLaunchKernelGGL(k_demig_keys, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, hs, geom, n,
@@ -3045,6 +3042,30 @@ static int demig_order(const ktm_plan *cp, const ktm_trace_geom *geom, int64_t n
                                       64u, hs));
     *order = i_out;
     return KTM_OK;
+}
+
+/* The sums of column parts for calls of up to n traces (tb a workgroup), after
+ * everything that a call cannot do without.  They grow with n up to the most
+ * traces that take parts, whether or not this call does: a call of no more
+ * traces than an earlier one allocates and frees nothing.  Without memory for
+ * them calls are not divided until one of more traces asks again. */
+static void demig_sums(ktm_plan *p, int64_t n, int tb)
+{
+    if (n <= p->dm_sum_ntr) return;
+    p->dm_sum_ntr = n;
+    const int64_t most = (int64_t)DM_TARGET_WGS * tb;
+    int64_t words = (n < most ? n : most) * p->tb.s.ns;
+    if (words > DM_SUM_MAX_WORDS) words = DM_SUM_MAX_WORDS;
+    if ((size_t)words <= p->dm_sum_cap) return;
+    if (p->d_dm_sum) (void)hipFree(p->d_dm_sum);
+    p->d_dm_sum = nullptr;
+    p->dm_sum_cap = 0;
+    if (hipMalloc((void **)&p->d_dm_sum, (size_t)words * sizeof(unsigned long long)) == hipSuccess) {
+        p->dm_sum_cap = (size_t)words;
+    } else {
+        p->d_dm_sum = nullptr;
+        (void)hipGetLastError();
+    }
 }
 
 static int demigrate(const ktm_plan *p, const float *km, const ktm_trace_geom *geom, int64_t ntr,
@@ -3090,7 +3111,7 @@ static int demigrate(const ktm_plan *p, const float *km, const ktm_trace_geom *g
     while ((1ull << a.lg_terms) < (unsigned long long)s->nxp * s->nyp * s->ns) ++a.lg_terms;
     if (!p->d_dm_amax) {
         ktm_plan *pm = const_cast<ktm_plan *>(p);
-        if (hipMalloc((void **)&pm->d_dm_amax, sizeof(uint32_t)) != hipSuccess) return KTM_ERR_NOMEM;
+        if (plan_alloc(pm, &pm->d_dm_amax, 1) != KTM_OK) return KTM_ERR_NOMEM;
     }
     a.amax = p->d_dm_amax;
     const int64_t nimg = (int64_t)s->nxp * s->nyp * s->nh * s->ns;
@@ -3130,7 +3151,8 @@ static int demigrate(const ktm_plan *p, const float *km, const ktm_trace_geom *g
         b.geom = geom + i0;
         b.traces = traces + i0 * s->ns;
         b.ntr = n;
-        if ((st = demig_order(p, b.geom, n, a.tb, hs, &b.order)) != KTM_OK) return st;
+        if ((st = demig_order(p, b.geom, n, hs, &b.order)) != KTM_OK) return st;
+        demig_sums(const_cast<ktm_plan *>(p), n, a.tb);
         const int64_t nblk = (n + a.tb - 1) / a.tb;
         /* few traces: their columns in parts, where the workspace of sums
          * holds them */
