@@ -48,6 +48,7 @@
 #include "ktm_postfft.h"
 
 #define KTM_WAVE 64
+#define KTM_CUS 256         /* compute units of the chip */
 
 /* ------------------------------------------------------------------------ */
 /* plan                                                                      */
@@ -1772,10 +1773,9 @@ __device__ __forceinline__ float wave_max(float v)
  * FASTIDX: the index floor(min(q, ns + lane + 1/2)) of the fast form alone,
  * the transpose of k_migrate's FASTIDX variant (floor(min(q, ns)) there: both
  * are >= ns for q >= ns, so they index the same samples).
- * Few traces (fewer than DM_TARGET_WGS workgroups) leave the chip idle:
- * gridDim.y parts then take every gridDim.y-th column of a group's box each,
- * add their sums into gsum (integers: in any order) and k_demig_finish forms
- * the traces.
+ * Few traces leave the chip idle (demig_parts): gridDim.y parts then take every
+ * gridDim.y-th column of a group's box each, add their sums into gsum
+ * (integers: in any order) and k_demig_finish forms the traces.
  * Bound by VALU issue like k_migrate, the image samples' conversion to fixed
  * point and the gates shared by the traces of a column.  48,000 traces x 1501
  * samples, 1600 columns: 23.0 -> 18.9 ms against a test, a branch and a
@@ -2997,12 +2997,70 @@ static int pixel_tables(const ktm_plan *cp, hipStream_t hs)
     return KTM_OK;
 }
 
-/* Workgroups below which a demigration takes its columns in parts (four rounds
- * of the 512 that run at once), the parts at most, and the bound of its
- * workspace (256 MiB) */
-#define DM_TARGET_WGS 2048
+/* The sums of column parts take at most 256 MiB */
 #define DM_MAX_PARTS 16
 #define DM_SUM_MAX_WORDS (32ll << 20)
+
+/* lane shapes by length: K samples per lane, W waves per column */
+typedef void (*demig_fn)(const DemigArgs);
+struct DemigShape { int cap, K, W; demig_fn fn[2]; };   /* fn: reference index, relaxed index */
+template <int K, int W> constexpr DemigShape demig_shape()
+{
+    return {K * W * KTM_WAVE, K, W, {k_demigrate<K, W, false>, k_demigrate<K, W, true>}};
+}
+static const DemigShape demig_shapes[] = {
+    demig_shape<6, 1>(),  demig_shape<8, 1>(),  demig_shape<10, 1>(), demig_shape<12, 1>(),
+    demig_shape<8, 2>(),  demig_shape<10, 2>(), demig_shape<12, 2>(), demig_shape<8, 4>(),
+    demig_shape<10, 4>(), demig_shape<12, 4>(), demig_shape<8, 8>(),  demig_shape<10, 8>(),
+    demig_shape<12, 8>()};                  /* KTM_MAX_NS */
+
+/* columns of an axis within the aperture of a point, at most */
+static int64_t columns_in_reach(const float *col, int n, double aperture)
+{
+    const double step = n > 1 ? fabs((double)col[n - 1] - col[0]) / (n - 1) : 0.0;
+    const double c = step > 0.0 ? 2.0 * aperture / step + 1.0 : (double)n;
+    return c < n ? (int64_t)c : n;
+}
+
+/* how a demigration is laid out: its lanes, traces per workgroup, the columns
+ * that one trace reaches at most, workgroups that run at once */
+struct DemigLayout { const DemigShape *sh; size_t lds; int tb, slots; int64_t cols; };
+
+/* Parts in which n traces take their columns: the cheapest of 1 to
+ * DM_MAX_PARTS if it is 10 % cheaper than 1.  Microseconds: a workgroup costs
+ * its waves 0.27 per slot, trace and column and 3.5 per column (reference index,
+ * four waves per SIMD) and 0.6 per pass over its sums; the chip takes 0.83 of
+ * that time per round of workgroups (some reach fewer columns) and the whole of it
+ * for the last ones; parts cost 34 for two more launches, 1.5e-5 per part and
+ * sample for the 64-bit atomic adds and 3e-5 per sample for clearing and finishing.
+ * Fitted to 1 to 16 parts of 8 to 12,000 traces of 63 to 5000 samples on 4 to 800
+ * columns of a line and 30 x 30 to 120 x 120 of a patch: of the parts tried the
+ * choice is within 0.8 % of the best on average, and at worst 4 % slower than
+ * undivided.
+ * 96 traces x 1001 on 800 columns: 1 part 1096 us, 16 150; 3000: 1 part 1165, 8
+ * 975; 6000 on 4 columns: 1 part 128, 16 254; 3001 x 751 on 61 x 61: 1 part 5.75
+ * ms, 6 3.99, 16 3.86. */
+static int demig_parts(const DemigLayout &l, int64_t n, int ns)
+{
+    const int64_t nblk = (n + l.tb - 1) / l.tb;
+    if (nblk >= 4 * l.slots) return 1;      /* four rounds are even enough */
+    const int64_t per = (l.cols * l.sh->W + 7) / 8;
+    const double col = 0.27 * l.sh->K * (double)(n < l.tb ? n : l.tb) + 3.5;
+    const double sums = 0.6 * l.tb * ns / 512.0, size = (double)n * ns;
+    int best = 1;
+    double tbest = 0.0;
+    for (int p = 1; p <= DM_MAX_PARTS; ++p) {
+        const double rounds = 1.0 + 0.83 * (double)(nblk * p) / l.slots;
+        const double t = rounds * ((double)((per + p - 1) / p) * col + sums) +
+                         (p > 1 ? 34.0 + (1.5e-5 * p + 3e-5) * size : 0.0);
+        if (p == 1) tbest = 0.9 * t;
+        else if (t < tbest) {
+            best = p;
+            tbest = t;
+        }
+    }
+    return best;
+}
 
 /* the demigration trace order of n traces (sorted by k_demig_keys) into
  * plan-owned buffers that grow with n; *order points at the sorted indices */
@@ -3044,17 +3102,21 @@ static int demig_order(const ktm_plan *cp, const ktm_trace_geom *geom, int64_t n
     return KTM_OK;
 }
 
-/* The sums of column parts for calls of up to n traces (tb a workgroup), after
- * everything that a call cannot do without.  They grow with n up to the most
- * traces that take parts, whether or not this call does: a call of no more
- * traces than an earlier one allocates and frees nothing.  Without memory for
- * them calls are not divided until one of more traces asks again. */
-static void demig_sums(ktm_plan *p, int64_t n, int tb)
+/* The sums of column parts for calls of up to n traces, after everything that
+ * a call cannot do without.  They grow with n up to the most traces that take
+ * parts, whether or not this call does: a call of no more traces than an earlier
+ * one allocates and frees nothing.  Without memory for them calls are not
+ * divided until one of more traces asks again. */
+static void demig_sums(ktm_plan *p, const DemigLayout &l, int64_t n)
 {
     if (n <= p->dm_sum_ntr) return;
     p->dm_sum_ntr = n;
-    const int64_t most = (int64_t)DM_TARGET_WGS * tb;
-    int64_t words = (n < most ? n : most) * p->tb.s.ns;
+    const int ns = p->tb.s.ns;
+    int64_t nblk = (n + l.tb - 1) / l.tb;
+    if (nblk > 4 * l.slots) nblk = 4 * l.slots;
+    while (nblk && demig_parts(l, nblk * l.tb, ns) == 1) --nblk;
+    const int64_t most = nblk * l.tb;
+    int64_t words = (n < most ? n : most) * ns;
     if (words > DM_SUM_MAX_WORDS) words = DM_SUM_MAX_WORDS;
     if ((size_t)words <= p->dm_sum_cap) return;
     if (p->d_dm_sum) (void)hipFree(p->d_dm_sum);
@@ -3119,32 +3181,22 @@ static int demigrate(const ktm_plan *p, const float *km, const ktm_trace_geom *g
     hipLaunchKernelGGL(k_absmax, dim3(1024), dim3(256), 0, hs, km, nimg, p->d_dm_amax);
     /* traces per workgroup: DM_TB, fewer so that two workgroups share a CU
      * (g rows of 8 bytes per sample within 76 KB), or one beyond that */
+    DemigLayout l;
     const size_t row = sizeof(unsigned long long) * (size_t)(s->ns + DM_PAD);
-    a.tb = (int)((76 * 1024) / row);
-    if (a.tb < 2) a.tb = (int)((152 * 1024) / row);
-    if (a.tb > DM_TB) a.tb = DM_TB;
-    if (a.tb < 1) return KTM_ERR_UNSUPPORTED;
-    typedef void (*fn_t)(const DemigArgs);
-    fn_t fn;
-    static const struct { int cap; fn_t f[2]; } shapes[] = {
-        {384, {k_demigrate<6, 1, false>, k_demigrate<6, 1, true>}},
-        {512, {k_demigrate<8, 1, false>, k_demigrate<8, 1, true>}},
-        {640, {k_demigrate<10, 1, false>, k_demigrate<10, 1, true>}},
-        {768, {k_demigrate<12, 1, false>, k_demigrate<12, 1, true>}},
-        {1024, {k_demigrate<8, 2, false>, k_demigrate<8, 2, true>}},
-        {1280, {k_demigrate<10, 2, false>, k_demigrate<10, 2, true>}},
-        {1536, {k_demigrate<12, 2, false>, k_demigrate<12, 2, true>}},
-        {2048, {k_demigrate<8, 4, false>, k_demigrate<8, 4, true>}},
-        {2560, {k_demigrate<10, 4, false>, k_demigrate<10, 4, true>}},
-        {3072, {k_demigrate<12, 4, false>, k_demigrate<12, 4, true>}},
-        {4096, {k_demigrate<8, 8, false>, k_demigrate<8, 8, true>}},
-        {5120, {k_demigrate<10, 8, false>, k_demigrate<10, 8, true>}},
-        {KTM_MAX_NS, {k_demigrate<12, 8, false>, k_demigrate<12, 8, true>}}};
-    int sh = 0;
-    while (shapes[sh].cap < s->ns) ++sh;    /* ns <= KTM_MAX_NS by ktm_plan_create */
-    fn = shapes[sh].f[fast ? 1 : 0];
-    const size_t lds = row * (size_t)a.tb;
-    HIP_TRY(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    l.tb = (int)((76 * 1024) / row);
+    l.slots = l.tb < 2 ? KTM_CUS : 2 * KTM_CUS;
+    if (l.tb < 2) l.tb = (int)((152 * 1024) / row);
+    if (l.tb > DM_TB) l.tb = DM_TB;
+    if (l.tb < 1) return KTM_ERR_UNSUPPORTED;
+    a.tb = l.tb;
+    l.lds = row * (size_t)l.tb;
+    l.sh = demig_shapes;
+    while (l.sh->cap < s->ns) ++l.sh;       /* ns <= KTM_MAX_NS by ktm_plan_create */
+    l.cols = columns_in_reach(p->tb.colx, s->nxp, p->cfg.aperture) *
+             columns_in_reach(p->tb.coly, s->nyp, p->cfg.aperture);
+    const demig_fn fn = l.sh->fn[fast ? 1 : 0];
+    HIP_TRY(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)l.lds));
     for (int64_t i0 = 0; i0 < ntr; i0 += 1 << 30) {
         const int64_t n = ntr - i0 < (1 << 30) ? ntr - i0 : (1 << 30);
         DemigArgs b = a;
@@ -3152,18 +3204,16 @@ static int demigrate(const ktm_plan *p, const float *km, const ktm_trace_geom *g
         b.traces = traces + i0 * s->ns;
         b.ntr = n;
         if ((st = demig_order(p, b.geom, n, hs, &b.order)) != KTM_OK) return st;
-        demig_sums(const_cast<ktm_plan *>(p), n, a.tb);
-        const int64_t nblk = (n + a.tb - 1) / a.tb;
-        /* few traces: their columns in parts, where the workspace of sums
-         * holds them */
-        int64_t parts = (DM_TARGET_WGS + nblk - 1) / nblk;
-        if (parts > DM_MAX_PARTS) parts = DM_MAX_PARTS;
+        demig_sums(const_cast<ktm_plan *>(p), l, n);
+        const int64_t nblk = (n + l.tb - 1) / l.tb;
+        /* few traces: their columns in parts, where the sums have their place */
+        int parts = demig_parts(l, n, s->ns);
         if ((size_t)(n * s->ns) > p->dm_sum_cap) parts = 1;
         if (parts > 1) {
             b.gsum = p->d_dm_sum;
             hipLaunchKernelGGL(k_zero_u64, dim3(2048), dim3(256), 0, hs, b.gsum, n * s->ns);
         }
-        hipLaunchKernelGGL(fn, dim3((unsigned)nblk, (unsigned)parts), dim3(8 * KTM_WAVE), lds, hs, b);
+        hipLaunchKernelGGL(fn, dim3((unsigned)nblk, (unsigned)parts), dim3(8 * KTM_WAVE), l.lds, hs, b);
         if (parts > 1)
             hipLaunchKernelGGL(k_demig_finish, dim3((unsigned)n), dim3(256), 0, hs, b);
     }
