@@ -2551,65 +2551,66 @@ static MigShape mig_shape(int accum)
             K, W, NW, C, WN + 1};
 }
 
-/* Relative time of a shape on ncol columns (x offset classes).  A trace costs
- * a wave about MIG_SLOT instructions per slot and MIG_TRACE besides (k_migrate);
- * a SIMD runs its waves' sum, ncol columns in workgroups of NW / W over 256
- * CUs (whole workgroups while there are few), and issues at full rate from
- * four waves.  Against 8 or 12 slots with 2 or 4 waves by length alone: 751
- * samples take 12 x 1 instead of 8 x 2 (a 61 x 61 patch with the relaxed index
- * 5.0 -> 3.3 ms), 1251 10 x 2 instead of 12 x 2 (150 x 150 columns 187 -> 171),
- * 2503 10 x 4 instead of 12 x 4 (12 classes of 500 columns 6.75 -> 5.9), and 32
- * columns of 501 samples 2 x 4 instead of 4 x 2 (60 -> 45 us).  The 800-column,
- * 1001-sample line, chunks of 4 rows: 4 x 4 2.96 ms, 8 x 2 3.92, 2 x 8 3.22. */
-static double mig_cost(int K, int W, int NW, int64_t ncol, bool fast)
+/* every shape, by samples per column; the ring of rows within half of a
+ * CU's LDS (two workgroups of 8 waves) or all of it (one of 16, or one of 8 for
+ * few columns).  Chunks of 8 rows wherever that ring holds two of them, with
+ * windows of up to 16 traces as it allows: half the barriers of chunks of 4 and
+ * twice the rows in flight.  The 800-column, 1001-sample line (4 x 4) 2.80 ->
+ * 2.41 ms, 12,000 traces into 1600 columns x 4 classes of 640 samples (10 x 1)
+ * 3.31 -> 3.13 and of 2001 (8 x 4) 8.90 -> 8.21, 500 samples into 60 columns (2 x
+ * 4) 0.78 -> 0.70; compensated sums and the relaxed index 2 to 13 % as well.
+ * 1280 and 1536 samples and beyond 2048 keep 4 (two chunks of 8 do not fit). */
+static const struct MigRow { int cap; MigShape (*make)(int); } mig_rows[] = {
+    {256, mig_shape<2, 2, 8, 8, 2>},    {384, mig_shape<6, 1, 8, 8, 2>},
+    {512, mig_shape<2, 4, 8, 8, 2>},    {512, mig_shape<4, 2, 8, 8, 2>},
+    {512, mig_shape<8, 1, 8, 8, 2>},    {640, mig_shape<10, 1, 8, 8, 2>},
+    {768, mig_shape<6, 2, 8, 8, 2>},    {768, mig_shape<12, 1, 8, 8, 2>},
+    {1024, mig_shape<2, 8, 8, 8, 1>},   {1024, mig_shape<4, 4, 8, 8, 1>},
+    {1024, mig_shape<8, 2, 8, 8, 1>},   {1280, mig_shape<10, 2, 8, 4, 2>},
+    {1536, mig_shape<6, 4, 8, 4, 2>},   {1536, mig_shape<12, 2, 8, 4, 2>},
+    {2048, mig_shape<8, 4, 16, 8, 1>},  {2048, mig_shape<8, 4, 8, 4, 1>},
+    {2560, mig_shape<10, 4, 16, 4, 2>}, {3072, mig_shape<12, 4, 16, 4, 2>},
+    {4096, mig_shape<8, 8, 16, 2, 2>},  {4096, mig_shape<8, 8, 8, 4, 1>},
+    {5120, mig_shape<10, 8, 16, 2, 2>}, {6144, mig_shape<12, 8, 16, 2, 2>},
+    {6144, mig_shape<12, 8, 8, 2, 2>}};
+
+/* dynamic LDS: the ring of rows, the slots' largest constants, the trace list,
+ * counts */
+static size_t mig_lds(const MigShape &m, int64_t row)
 {
-    static const double rate[5] = {0.0, 0.40, 0.65, 0.85, 1.0};
-    const double per_cu = (double)((ncol * W + NW - 1) / NW) / 256.0;
-    const double whole = per_cu < 8.0 ? ceil(per_cu) : per_cu;
-    const double waves = whole * NW / 4.0;
-    const double r = waves >= 4.0 ? 1.0 : rate[(int)waves] + (waves - (int)waves) *
-                                                                  (rate[(int)waves + 1] - rate[(int)waves]);
-    return waves * (fast ? 8.0 * K + 25.0 : 10.7 * K + 40.0) / r;
+    return sizeof(float) * (size_t)(m.RING * m.C * row + 2 * m.NW * m.K) +
+           sizeof(int) * (size_t)(KTM_WAVE + m.C + m.NW * KTM_WAVE + m.NW);
 }
 
-/* W waves share one image column (each owns K*64 consecutive samples); a
- * workgroup of NW waves covers NW/W columns. */
-static MigShape pick_migrate(int ns, int accum, int64_t ncol)
+/* instructions of a trace, per wave of K slots (k_migrate) */
+static double mig_trace(int K, int accum)
 {
-    /* every shape, by samples per column; the ring of rows within half of a
-     * CU's LDS (two workgroups of 8 waves) or all of it (one of 16).  Chunks
-     * of 8 rows wherever that ring holds two of them, with windows of up to 16
-     * traces as it allows: half the barriers of chunks of 4 and twice the rows
-     * in flight.  The 800-column, 1001-sample line (4 x 4) 2.80 -> 2.41 ms,
-     * 12,000 traces into 1600 columns x 4 classes of 640 samples (10 x 1) 3.31
-     * -> 3.13 and of 2001 (8 x 4) 8.90 -> 8.21, 500 samples into 60 columns (2 x
-     * 4) 0.78 -> 0.70; compensated sums and the relaxed index 2 to 13 % as
-     * well.  1280 and 1536 samples and beyond 2048 keep 4 (two chunks of 8 do
-     * not fit). */
-    static const struct { int cap, K, W, NW; MigShape (*make)(int); } S[] = {
-        {256, 2, 2, 8, mig_shape<2, 2, 8, 8, 2>},    {384, 6, 1, 8, mig_shape<6, 1, 8, 8, 2>},
-        {512, 2, 4, 8, mig_shape<2, 4, 8, 8, 2>},    {512, 4, 2, 8, mig_shape<4, 2, 8, 8, 2>},
-        {512, 8, 1, 8, mig_shape<8, 1, 8, 8, 2>},    {640, 10, 1, 8, mig_shape<10, 1, 8, 8, 2>},
-        {768, 6, 2, 8, mig_shape<6, 2, 8, 8, 2>},    {768, 12, 1, 8, mig_shape<12, 1, 8, 8, 2>},
-        {1024, 2, 8, 8, mig_shape<2, 8, 8, 8, 1>},   {1024, 4, 4, 8, mig_shape<4, 4, 8, 8, 1>},
-        {1024, 8, 2, 8, mig_shape<8, 2, 8, 8, 1>},   {1280, 10, 2, 8, mig_shape<10, 2, 8, 4, 2>},
-        {1536, 6, 4, 8, mig_shape<6, 4, 8, 4, 2>},   {1536, 12, 2, 8, mig_shape<12, 2, 8, 4, 2>},
-        {2048, 8, 4, 16, mig_shape<8, 4, 16, 8, 1>}, {2560, 10, 4, 16, mig_shape<10, 4, 16, 4, 2>},
-        {3072, 12, 4, 16, mig_shape<12, 4, 16, 4, 2>}, {4096, 8, 8, 16, mig_shape<8, 8, 16, 2, 2>},
-        {5120, 10, 8, 16, mig_shape<10, 8, 16, 2, 2>}, {6144, 12, 8, 16, mig_shape<12, 8, 16, 2, 2>}};
-    /* compensated sums of a small image are split along the traces instead */
-    if ((accum & ~KTM_INDEX_FAST) == KTM_ACCUM_KAHAN && ncol < (1 << 20)) ncol = 1 << 20;
-    int best = -1;
-    double tbest = 0.0;
-    for (int i = 0; i < (int)(sizeof S / sizeof S[0]); ++i) {
-        if (S[i].cap < ns) continue;
-        const double t = mig_cost(S[i].K, S[i].W, S[i].NW, ncol, (accum & KTM_INDEX_FAST) != 0);
-        if (best < 0 || t < tbest) {
-            best = i;
-            tbest = t;
-        }
-    }
-    return S[best].make(accum);
+    return accum & KTM_INDEX_FAST ? 8.0 * K + 25.0 : 10.7 * K + 40.0;
+}
+
+/* Relative time of a shape with wgs workgroups (columns x offset classes x
+ * parts of the traces, as if every trace reached all of them) that take `share`
+ * of the traces each: a SIMD runs its waves' sum over the chip's CUs (whole
+ * workgroups while there are few), at full rate from four resident waves.  Two
+ * waves run at 0.65 of that rate (3500 samples into 200 columns: 2.39 ms at four
+ * waves on 100 CUs, 1.74 at two on 200); one and three lie beside it.
+ * Against 8 or 12 slots with 2 or 4 waves by length alone: 751 samples take 12 x 1
+ * instead of 8 x 2 (a 61 x 61 patch with the relaxed index 5.0 -> 3.3 ms), 1251
+ * 10 x 2 instead of 12 x 2 (150 x 150 columns 187 -> 171), 2503 10 x 4 instead of
+ * 12 x 4 (12 classes of 500 columns 6.75 -> 5.9), and 32 columns of 501 samples
+ * 2 x 4 instead of 4 x 2 (60 -> 45 us).  The 800-column, 1001-sample line, chunks
+ * of 4 rows: 4 x 4 2.96 ms, 8 x 2 3.92, 2 x 8 3.22.  Eight waves of long rows
+ * against sixteen: 200 columns of 1700 samples 1.46 ms, 1.75; of 3500 1.74, 2.39; of
+ * 6144 2.50, 2.96; 60 x 60 columns of 3500 5.65, 4.42. */
+static double mig_cost(const MigShape &m, size_t lds, double wgs, double share, int accum)
+{
+    static const double rate[5] = {0.0, 0.40, 0.65, 0.85, 1.0};
+    const double per_cu = wgs / KTM_CUS;
+    const double waves = (per_cu < 8.0 ? ceil(per_cu) : per_cu) * m.NW / 4.0;
+    const double fit = (double)(160 * 1024 / lds) * m.NW / 4.0;    /* resident, by LDS */
+    const double at_once = waves < 4.0 && waves < fit ? waves : fit < 4.0 ? fit : 4.0;
+    const int i = at_once < 4.0 ? (int)at_once : 3;
+    return waves * share * mig_trace(m.K, accum) / (rate[i] + (at_once - i) * (rate[i + 1] - rate[i]));
 }
 
 /* Tiles of the region [rx0,rx1) x [ry0,ry1): ncol columns, a row on a 2-D
@@ -2640,17 +2641,59 @@ static int parts_for(int64_t wgs)
     return n > KTM_MAX_PARTS ? KTM_MAX_PARTS : (int)n;
 }
 
+/* The shape, tiles and parts of a block of ntr traces into the region of a. */
+static MigShape pick_migrate(const ktm_setup *s, int64_t row, int accum, int64_t ntr, int parts_max,
+                             MigArgs *a)
+{
+    const int64_t ncol = (int64_t)(a->rx1 - a->rx0) * (a->ry1 - a->ry0) * s->nh;
+    MigShape best = {};
+    MigArgs with = *a;
+    double tbest = 0.0;
+    for (const MigRow &r : mig_rows) {
+        if (r.cap < s->ns) continue;
+        const MigShape m = r.make(accum);
+        MigArgs b = *a;
+        tile_layout(s, m.NW / m.W, &b);
+        /* compensated sums of a small region: the traces in parts */
+        double share = 1.0;
+        b.nparts = 1;
+        if ((accum & ~KTM_INDEX_FAST) == KTM_ACCUM_KAHAN) {
+            const int64_t chunk = m.NW * KTM_WAVE, nchunks = (ntr + chunk - 1) / chunk;
+            b.nparts = parts_for((int64_t)b.ntiles * s->nh);
+            if (b.nparts > parts_max) b.nparts = parts_max;
+            if (b.nparts > nchunks) b.nparts = nchunks;      /* no part without a chunk */
+            const double most = (double)((nchunks + b.nparts - 1) / b.nparts * chunk) / (double)ntr;
+            if (b.nparts > 1 && most < 1.0) share = most;
+        }
+        const double wgs = (double)((ncol * m.W + m.NW - 1) / m.NW) * (double)b.nparts;
+        const double t = mig_cost(m, mig_lds(m, row), wgs, share, accum);
+        if (!best.fn || t < tbest) {
+            best = m;
+            with = b;
+            tbest = t;
+        }
+    }
+    *a = with;
+    return best;
+}
+
 /* the partial images of the compensated split, sized for the whole image
- * (a job region needs at most that), allocated once with the plan so that
- * neither migration entry point allocates them; none for a large image */
+ * (a job region needs at most that) at the shape of least instructions a trace
+ * (the fewest tiles of those that a block takes, so the most parts), allocated
+ * once with the plan so that neither migration entry point allocates them; none
+ * for a large image */
 static int parts_workspace(ktm_plan *p)
 {
     const ktm_setup *s = &p->tb.s;
     MigArgs a;
     memset(&a, 0, sizeof a);
     a.rx1 = s->nxp; a.ry1 = s->nyp;
-    const MigShape m = pick_migrate(s->ns, KTM_ACCUM_KAHAN,
-                                    (int64_t)s->nxp * s->nyp * s->nh);
+    MigShape m = {};
+    for (const MigRow &r : mig_rows) {
+        if (r.cap < s->ns) continue;
+        const MigShape c = r.make(KTM_ACCUM_KAHAN);
+        if (!m.fn || c.W * mig_trace(c.K, 0) < m.W * mig_trace(m.K, 0)) m = c;
+    }
     tile_layout(s, m.NW / m.W, &a);
     int n = parts_for((int64_t)a.ntiles * s->nh);
     const uint64_t per = 3ull * sizeof(float) * (uint64_t)s->nxp * s->nyp * s->nh * s->ns;
@@ -2817,25 +2860,12 @@ static int migrate_block(const ktm_plan *p, const void *prepared, int dtype, int
         a.rx0 = (job / p->cfg.jobs_y) * s->nx; a.rx1 = a.rx0 + s->nx;
         a.ry0 = (job % p->cfg.jobs_y) * s->ny; a.ry1 = a.ry0 + s->ny;
     }
-    const int64_t ncols_region = (int64_t)(a.rx1 - a.rx0) * (a.ry1 - a.ry0);
-    const MigShape m = pick_migrate(s->ns, accum, ncols_region * s->nh);
-    const mig_fn fn = m.fn;
-    tile_layout(s, m.NW / m.W, &a);
-    const int nthreads = m.NW * KTM_WAVE;
-    /* compensated sums of a small region: the traces in parts */
-    int nparts = 1;
-    a.part_n = ncols_region * s->nh * s->ns;
+    a.part_n = (int64_t)(a.rx1 - a.rx0) * (a.ry1 - a.ry0) * s->nh * s->ns;
     a.parts = p->d_parts;
-    if (acc_mode == KTM_ACCUM_KAHAN && p->parts_max > 1) {
-        nparts = parts_for((int64_t)a.ntiles * s->nh);
-        if (nparts > p->parts_max) nparts = p->parts_max;
-        const int64_t nchunks = (ntr + nthreads - 1) / nthreads;
-        if (nparts > nchunks) nparts = (int)nchunks;     /* no part without a chunk */
-    }
-    a.nparts = nparts;
-    /* the ring of rows, the slots' largest constants, the trace list, counts */
-    const size_t lds = sizeof(float) * (size_t)(m.RING * m.C * p->row + 2 * m.NW * m.K) +
-                       sizeof(int) * (size_t)(KTM_WAVE + m.C + nthreads + m.NW);
+    const MigShape m = pick_migrate(s, p->row, accum, ntr, p->parts_max, &a);
+    const mig_fn fn = m.fn;
+    const int nthreads = m.NW * KTM_WAVE, nparts = (int)a.nparts;
+    const size_t lds = mig_lds(m, p->row);
     if (lds > 160 * 1024) return KTM_ERR_UNSUPPORTED;
     /* runs of a row of tiles, but at least 8 runs per XCD */
     a.run = a.ntiles / 64 < a.tiles_x ? a.ntiles / 64 : a.tiles_x;

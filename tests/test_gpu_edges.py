@@ -330,3 +330,27 @@ def test_traces_without_a_position_add_nothing(cuda, ns, kahan):
         assert float((out[0][0] - out[1][0]).norm() / out[1][0].norm()) <= 1e-6
     else:
         assert torch.equal(out[0][0], out[1][0])
+
+
+# (samples, columns) of every lane layout of ktm_migrate_block, as
+# test_host_launches.py finds them taken
+LANES = [(200, 300), (384, 4200), (512, 40), (512, 1600), (512, 4200), (640, 4200), (768, 1600),
+         (768, 4200), (1024, 40), (1024, 700), (1024, 4200), (1280, 4200), (1536, 40), (1536, 4200),
+         (2048, 1000), (2048, 40), (2560, 1000), (3072, 1000), (4096, 1000), (4096, 40), (5120, 1000),
+         (6144, 1000), (6144, 40)]
+
+
+@pytest.mark.parametrize("ns,ncols", LANES)
+def test_trace_counts_in_every_lane_layout_bitexact(cuda, ns, ncols):
+    """Trace counts around the chunks of rows (2, 4 or 8), the windows (4, 8 or
+    16 traces), the 64 traces whose gates are evaluated at once and the blocks
+    filtered into the list (512 or 1024), the last ones for few columns, at the
+    last sample count of the layout."""
+    sv = small_line(ns, nshots=55, nrecv_side=10, ncols=ncols, jobs_x=1, nh=1, dh=110.0, aperture=400.0)
+    coords = sv.coords[np.random.default_rng(ns).permutation(sv.ntr)]
+    coords[::4, 2] = coords[::4, 0] = 625 * (1 + np.arange(coords[::4].shape[0]) % 7)
+    tr = np.random.default_rng(ncols).standard_normal((sv.ntr, ns)).astype(np.float32)
+    for ntr in [1, 3, 9, 17, 66, 73, 131] + ([515, 1089] if ncols == 40 else []):
+        print(f"case: {ntr} traces x {ns} samples, {ncols} columns", flush=True)
+        sv.coords = np.ascontiguousarray(coords[:ntr])
+        bitexact_case(sv, tr[:ntr].copy(), cuda)

@@ -45,3 +45,69 @@ def test_demigration_divides_its_columns_only_where_that_pays(stand_in):
     assert host_hip.run(__file__, stand_in, "child_demigrate", whole) == [1] * len(whole)
     many = [("line", ns, 800, 96) for ns in (63, 300, 1001, 2600, 5000)] + [("area", 751, 61, 3001)]
     assert min(host_hip.run(__file__, stand_in, "child_demigrate", many)) >= 4
+
+
+# (samples, columns, offset classes) that take each lane layout with plain
+# sums: samples per lane, waves per column and per workgroup
+LAYOUTS = [
+    (200, 300, 1, [2, 2, 8]), (384, 4200, 1, [6, 1, 8]), (512, 40, 1, [2, 4, 8]),
+    (512, 1600, 1, [4, 2, 8]), (512, 4200, 1, [8, 1, 8]), (640, 4200, 1, [10, 1, 8]),
+    (768, 1600, 1, [6, 2, 8]), (768, 4200, 1, [12, 1, 8]), (1024, 40, 1, [2, 8, 8]),
+    (1024, 700, 1, [4, 4, 8]), (1024, 4200, 1, [8, 2, 8]), (1280, 4200, 1, [10, 2, 8]),
+    (1536, 40, 1, [6, 4, 8]), (1536, 4200, 1, [12, 2, 8]), (2048, 1000, 1, [8, 4, 16]),
+    (2048, 40, 1, [8, 4, 8]), (2560, 1000, 1, [10, 4, 16]), (3072, 1000, 1, [12, 4, 16]),
+    (4096, 1000, 1, [8, 8, 16]), (4096, 40, 1, [8, 8, 8]), (5120, 1000, 1, [10, 8, 16]),
+    (6144, 1000, 1, [12, 8, 16]), (6144, 40, 1, [12, 8, 8])]
+
+
+def _shape(hip, sv, ntr, accum, job=-1):
+    plan = hip.plan(sv.cfg, sv.ns, sv.dt, sv.vel)
+    st, launches, _ = hip.migrate(plan, ntr, accum, job)
+    hip.lib.ktm_plan_destroy(plan)
+    (k, (K, W, NW, C, *_, kahan, fast), grid, block, lds), *merge = launches
+    assert st == 0 and k == "k_migrate"
+    assert [kahan, fast] == [accum & 1, accum >> 8] and block == [64 * NW, 1, 1]
+    assert 64 * K * W >= sv.ns and NW % W == NW % C == 0 and lds <= 160 * 1024
+    assert len(merge) == int(grid[2] > 1) and (kahan or grid[2] == 1)
+    return [K, W, NW], grid[2]
+
+
+def child_layouts(hip, layouts):
+    return [_shape(hip, _line(ns, ncols, nh), 100, 0)[0] for ns, ncols, nh, _ in layouts]
+
+
+def test_every_lane_layout_is_taken(stand_in):
+    got = host_hip.run(__file__, stand_in, "child_layouts", LAYOUTS)
+    assert got == [s for *_, s in LAYOUTS]
+    assert len({(s[0], tuple(s[3])) for s in LAYOUTS}) == 23
+
+
+def child_compensated(hip, cases):
+    out = []
+    for ns, ncols, ntr in cases:
+        for fast in (0, 256):
+            sv = _line(ns, ncols)
+            out.append([_shape(hip, sv, ntr, fast), _shape(hip, sv, ntr, fast | 1)])
+    return out
+
+
+def test_compensated_blocks_that_are_not_divided_take_the_lanes_of_plain_ones(stand_in):
+    """A block of one chunk of traces is one part: its lanes spread over the
+    chip as with plain sums (one shot record into 32 columns ran 4 workgroups)."""
+    cases = [(ns, ncols, ntr) for ns in (301, 501, 600, 751, 1001, 1700, 2001, 2600, 3000, 3500, 6144)
+             for ncols, ntr in ((32, 96), (200, 120), (2000, 1))]
+    for plain, kahan in host_hip.run(__file__, stand_in, "child_compensated", cases):
+        assert plain == kahan
+
+
+def child_divided(hip):
+    sv = _line(1501, 1600)
+    return [_shape(hip, sv, 48000, 1), _shape(hip, _line(1700, 200), 1920, 1),
+            _shape(hip, _area(1251, 150), 20000, 1)]
+
+
+def test_compensated_blocks_of_many_traces_are_divided(stand_in):
+    big, few, area = host_hip.run(__file__, stand_in, "child_divided")
+    assert big == [[12, 2, 8], 26]
+    assert few == [[8, 4, 8], 4]                   # chunks of 512 traces
+    assert area[0] == [10, 2, 8] and area[1] == 2
