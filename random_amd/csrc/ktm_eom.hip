@@ -14,12 +14,12 @@
  *
  * k_eom_geometry: per trace h2, CMP and talpha with the reference's float and
  *   double promotions (EOM.c:1245-1272).
- * k_eom_accum: one workgroup = one CSP x one segment of 64 samples, one lane
- *   per sample.  The lane owns its sample of every offset bin of its CSP for
+ * k_eom_accum: one workgroup = one CSP x one segment of 64 or 256 samples, one
+ *   lane per sample.  The lane owns its sample of every offset bin of its CSP for
  *   the whole launch, so it adds into the gather without atomics and in trace
  *   order (the reference's order of additions per bin); the two bins of the
  *   latest trace stay in registers until another trace needs their slot.
- *   Traces stream in chunks of 64: the aperture gate of each is evaluated
+ *   Traces stream in chunks of as many: the aperture gate of each is evaluated
  *   lane-parallel, the passing ones are compacted in order through LDS.
  * k_postfft<PostEom> (ktm_postfft.h; k_postmx<PostEom> of ktm_postmx.h on
  *   the matrix cores beyond 4096 samples): the post filter as a real
@@ -44,8 +44,7 @@
 #include "ktm_postmx.h"
 #include "ktm_postfft.h"
 
-#define EOM_NT 64      /* samples (and lanes) of a workgroup: one wave */
-#define EOM_RUN 64     /* consecutive tiles per XCD run */
+#define EOM_RUN 4096   /* lanes of the consecutive tiles of an XCD's run */
 #define EOM_WAVE 64
 #define EOM_PI 3.14159265359 /* EOM.c:124 */
 
@@ -356,33 +355,35 @@ struct EomArgs {
  * trace (a store and a load of both arrays, 51 GB on the 40-shot line, 4 TB/s;
  * the bins a wave returns to with the next shot, 82 KB, do not fit the L2 at
  * any useful occupancy).  Four waves per SIMD measured faster than five or
- * six (fewer gathers in flight to evict each other), and workgroups of one
- * wave than of four (no barrier, and the segments' unequal counts even out):
- * 14.8 -> 12.2 ms with 7.5e9 -> 5.1e9 VALU instructions, the sample of the
- * next trace loaded ahead and the bins before the taper. */
-template <bool WIDE>
-__global__ void __launch_bounds__(EOM_NT) __attribute__((amdgpu_waves_per_eu(4)))
+ * six (fewer gathers in flight to evict each other), and on that line
+ * workgroups of one wave than of four (no barrier, and the segments' unequal
+ * counts even out; eom_lanes): 14.8 -> 12.2 ms with 7.5e9 -> 5.1e9 VALU
+ * instructions, the sample of the next trace loaded ahead and the bins before
+ * the taper. */
+template <bool WIDE, int NT>
+__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4)))
 k_eom_accum(const EomArgs a)
 {
     /* per passing trace: 4 x2 h2 (exact in double) and RN(x2 + h2), the
      * trace-only terms of EOM.c:1285-1286 */
-    __shared__ double sXH4[EOM_NT];
-    __shared__ float sXpH[EOM_NT];
-    __shared__ int sTa[EOM_NT], sIdx[EOM_NT], sCnt[EOM_NT / EOM_WAVE];
+    __shared__ double sXH4[NT];
+    __shared__ float sXpH[NT];
+    __shared__ int sTa[NT], sIdx[NT], sCnt[NT / EOM_WAVE];
+    constexpr int RUN = EOM_RUN / NT;       /* consecutive tiles per XCD run */
     const int tid = threadIdx.x, lane = tid & (EOM_WAVE - 1), wv = tid / EOM_WAVE;
     /* XCD-aware order: consecutive workgroup ids go to different XCDs; each
-     * XCD takes runs of EOM_RUN consecutive (CSP, segment) tiles (neighbouring
+     * XCD takes runs of RUN consecutive (CSP, segment) tiles (neighbouring
      * CSPs share traces in its L2), and the runs are dealt round-robin so
      * every XCD gets CSPs from the whole survey (the trace count per CSP
      * falls towards the survey's edges) */
     const int ntiles = a.nrx * a.nry * a.nseg;
     const int i = blockIdx.x >> 3;
-    const int tile = (((i / EOM_RUN) << 3) + (int)(blockIdx.x & 7)) * EOM_RUN + i % EOM_RUN;
+    const int tile = (((i / RUN) << 3) + (int)(blockIdx.x & 7)) * RUN + i % RUN;
     if (tile >= ntiles) return;
     const int seg = tile % a.nseg, col = tile / a.nseg;
     const int X = a.rx0 + col / a.nry, Y = a.ry0 + col % a.nry;
     const float cspX = a.cspx[X], cspY = a.cspy[Y];
-    const int t = seg * EOM_NT + tid;
+    const int t = seg * NT + tid;
     const bool tin = t < a.ns;
     const int tc = tin ? t : a.ns - 1;
     /* per-sample constants of this lane */
@@ -409,7 +410,7 @@ k_eom_accum(const EomArgs a)
     /* the lane's sample of two offset bins, held in registers between traces */
     int tagE = -1, tagO = -1;
     float cE = 0.0f, fE = 0.0f, cO = 0.0f, fO = 0.0f;
-    for (int64_t c0 = 0; c0 < a.ntr; c0 += EOM_NT) {
+    for (int64_t c0 = 0; c0 < a.ntr; c0 += NT) {
         /* ---- aperture gate of EOM.c:1268-1270 for 64 traces, in order ---- */
         const int64_t i = c0 + tid;
         bool pass = false;
@@ -429,7 +430,7 @@ k_eom_accum(const EomArgs a)
         __syncthreads();
         int base = 0, total = 0;
 #pragma unroll
-        for (int q = 0; q < EOM_NT / EOM_WAVE; ++q) {
+        for (int q = 0; q < NT / EOM_WAVE; ++q) {
             base += q < wv ? sCnt[q] : 0;
             total += sCnt[q];
         }
@@ -554,6 +555,18 @@ extern "C" int ktm_eom_reset(const ktm_eom_plan *p, float *csp, float *fold, voi
 
 /* Bin a block of traces into the gathers of every slab (job < 0) or one;
  * local: the gathers hold the job's slab only, [nx][ny][nh][ns]. */
+/* Lanes of a workgroup: one wave, or four where all four are needed and a lane
+ * has more than 200 bins, whose traffic the fours' neighbouring bins share (one
+ * wave, four): 720 traces x 2001 samples into 60 CSPs x 1000 bins 2.36 ms, 1.76;
+ * 3600 x 1001 into 300 CSPs x 320 bins 9.86, 8.02; 1200 x 2001 into 800 CSPs x 320
+ * bins 9.50, 8.60, x 1000 bins 18.7, 20.1, x 160 bins 5.20, 5.44; 4800 x 1001 into
+ * 800 CSPs x 160 bins 12.3, 12.8; 3600 x 3000 (47 segments of 64) into 300 CSPs x
+ * 1000 bins 28.1, 34.3. */
+static int eom_lanes(int ns, int nh)
+{
+    return nh > 200 && (ns + 63) / 64 % 4 == 0 ? 256 : 64;
+}
+
 static int eom_block(const ktm_eom_plan *cp, const float *traces, const int32_t *coords,
                      int64_t ntr, int job, bool local, float *csp, float *fold, uint64_t *counter,
                      void *stream)
@@ -584,7 +597,8 @@ static int eom_block(const ktm_eom_plan *cp, const float *traces, const int32_t 
     a.csp = csp; a.fold = fold; a.counter = (unsigned long long *)counter;
     a.aperture2 = p->aperture2; a.dt = s->dt; a.dh = p->cfg.dh; a.oh = p->cfg.oh;
     a.ns = s->ns; a.nh = s->nh;
-    a.nseg = (s->ns + EOM_NT - 1) / EOM_NT;
+    const int nt = eom_lanes(s->ns, s->nh);
+    a.nseg = (s->ns + nt - 1) / nt;
     if (job < 0) {
         a.rx0 = 0; a.ry0 = 0; a.nrx = s->nxp; a.nry = s->nyp;
     } else {   /* the job's slab, EOM.c:1261-1262 */
@@ -598,12 +612,12 @@ static int eom_block(const ktm_eom_plan *cp, const float *traces, const int32_t 
     }
     const int64_t ntiles = (int64_t)a.nrx * a.nry * a.nseg;
     if (ntiles > 0x7fffff00LL) return KTM_ERR_UNSUPPORTED;
-    const int64_t span = 8 * EOM_RUN;   /* tiles per round of runs over the 8 XCDs */
+    const int64_t span = 8 * (EOM_RUN / nt);   /* tiles per round of runs over the 8 XCDs */
     const int64_t nblk = (ntiles + span - 1) / span * span;
-    if ((int64_t)a.nh * a.ns >= (1 << 30) || a.nh >= (1 << 24) || a.ns >= (1 << 22))
-        hipLaunchKernelGGL(k_eom_accum<true>, dim3((unsigned)nblk), dim3(EOM_NT), 0, st, a);
-    else
-        hipLaunchKernelGGL(k_eom_accum<false>, dim3((unsigned)nblk), dim3(EOM_NT), 0, st, a);
+    const bool wide = (int64_t)a.nh * a.ns >= (1 << 30) || a.nh >= (1 << 24) || a.ns >= (1 << 22);
+    void (*fn)(const EomArgs) = nt == 64 ? (wide ? k_eom_accum<true, 64> : k_eom_accum<false, 64>)
+                                         : (wide ? k_eom_accum<true, 256> : k_eom_accum<false, 256>);
+    hipLaunchKernelGGL(fn, dim3((unsigned)nblk), dim3((unsigned)nt), 0, st, a);
     EOM_TRY(hipGetLastError());
     return KTM_OK;
 }

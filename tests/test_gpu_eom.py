@@ -221,3 +221,27 @@ def test_eom_post_long_traces(cuda, ns):
     e = rel_l2(out[:2], ref)
     print(f"  relL2 {e:.2e}", flush=True)
     assert e <= 1e-6
+
+
+@pytest.mark.parametrize("nh", [32, 200, 201, 400])
+@pytest.mark.parametrize("ns", [40, 64, 65, 192, 193, 256, 257, 300, 511, 513, 751])
+def test_eom_workgroups_of_one_and_of_four_waves(cuda, ns, nh):
+    """Sample and bin counts on both sides of every change between workgroups of
+    64 samples and of 256, with more traces than either gates at once."""
+    print(f"case: EOM line, {ns} samples, {nh} bins", flush=True)
+    sv = surveys.line2d(nshots=14, nrecv_side=20, ns=ns, ncols=80, col_dx=12.5, nscat=4, x0=400.0,
+                        t0_range=(0.01, 0.1))
+    _, cfg, _ = line_case()
+    cfg.velocity_start = cfg.velocity_end = 6000.0
+    cfg.nh, cfg.dh = nh, 800.0 / nh
+    tr = np.random.default_rng(ns).standard_normal((sv.ntr, ns)).astype(np.float32)
+    plan = EomPlan(cfg, ns, sv.dt)
+    csp, fold, n = plan.migrate(torch.from_numpy(tr).to(cuda), torch.from_numpy(sv.coords).to(cuda),
+                                block=600)
+    c0, f0, n0 = oracle.eom_all(cfg, ns, np.float32(sv.dt), tr, sv.coords, cfg.velocity(ns))
+    c = csp.cpu().numpy()
+    print(f"  evaluated {n} (oracle {n0}); gathers relL2 {rel_l2(c, c0):.2e}", flush=True)
+    assert n == n0
+    assert np.array_equal(fold.cpu().numpy(), f0)
+    assert rel_l2(c, c0) <= 1e-6
+    assert ns < 64 or np.abs(c0).max() > 0

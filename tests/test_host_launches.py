@@ -111,3 +111,33 @@ def test_compensated_blocks_of_many_traces_are_divided(stand_in):
     assert big == [[12, 2, 8], 26]
     assert few == [[8, 4, 8], 4]                   # chunks of 512 traces
     assert area[0] == [10, 2, 8] and area[1] == 2
+
+
+def child_eom(hip, cases):
+    """(WIDE, lanes) of the binning kernel by samples and bins."""
+    import ctypes as C
+    from random_amd import _lib
+    from random_amd.eom import EomConfig
+    out = []
+    for ns, nh in cases:
+        cfg = EomConfig(ox=0.0, oy=0.0, angle_e_to_n=0.0, oxcsp=0.0, oycsp=0.0, excsp=100.0, eycsp=0.0,
+                        scale_xy=0.01, dcsp_x=12.5, dcsp_y=0.0, dh=1.0, nh=nh, aperture=800.0, jobs_x=1,
+                        jobs_y=1, ntblock=50, velocity_start=2000.0, velocity_end=2000.0)
+        h, c, vel = C.c_void_p(), cfg.to_c(), cfg.velocity(ns)
+        _lib.check(hip.lib.ktm_eom_plan_create(C.byref(h), C.byref(c), ns, 0.004,
+                                               vel.ctypes.data_as(C.c_void_p)), "ktm_eom_plan_create")
+        st, launches, _ = hip.call("ktm_eom_block", h, hip.any, hip.any, 10, -1, hip.any, hip.any, None, None)
+        k, t, grid, block, _ = launches[-1]
+        assert st == 0 and k == "k_eom_accum" and block == [t[1], 1, 1]
+        assert grid[0] >= 8 * -(-ns // t[1])             # 8 CSPs
+        out.append(t)
+        hip.lib.ktm_eom_plan_destroy(h)
+    return out
+
+
+def test_eom_workgroups_by_samples_and_bins(stand_in):
+    cases = {(1001, 160): [0, 64], (1001, 201): [0, 256], (1001, 1000): [0, 256], (2001, 1000): [0, 256],
+             (300, 1000): [0, 64], (3000, 1000): [0, 64], (256, (1 << 22) - 1): [0, 256],
+             (256, 1 << 22): [1, 256], (320, 1 << 22): [1, 64], (4, 1 << 24): [1, 64]}
+    got = host_hip.run(__file__, stand_in, "child_eom", list(cases))
+    assert got == list(cases.values())
