@@ -560,12 +560,20 @@ float ktm_gate_threshold(double A);
  * traveltime path (its error bound is an input of that path's proof). */
 int ktm_selftest_sqrt(const float *x, int64_t n, float *out_hw, void *stream);
 /* in4[n][4] = (dIS2, dIR2, t, v2), t a sample index held as a float (t2
- * is formed as in the traveltime table, Kirchhoff.c:1246-1247): q_fast (fast
- * path), q_ref = RN(dsr/dt) with the arithmetic of Kirchhoff.c:1381-1384,
- * and the sample index the migration kernel selects (t_kernel) vs the
- * reference's (t_ref). */
+ * is formed as in the traveltime table, Kirchhoff.c:1246-1247): q_fast (the
+ * fast form of the demigration and of the relaxed index), q_ref = RN(dsr/dt)
+ * with the arithmetic of Kirchhoff.c:1381-1384, and the sample index the
+ * migration kernel selects (t_kernel) vs the reference's (t_ref). */
 int ktm_selftest_traveltime(const float *in4, int64_t n, float dt, int ns, float *q_fast,
                             float *q_ref, int32_t *t_kernel, int32_t *t_ref, void *stream);
+/* The fast form of the migration's reference index for the same inputs, in
+ * samples, limited to ns + 1/2. */
+int ktm_selftest_limited(const float *in4, int64_t n, float dt, int ns, double *q, void *stream);
+/* taper[i]: the time taper of EOM.c:1290-1292 for the float d[i] = t dt - tc;
+ * root[i]: (float)sqrt((double)x[i]) of EOM.c:1286, both as the binning kernel
+ * forms them. */
+int ktm_selftest_eom(const float *d, const float *x, int64_t n, float *taper, float *root,
+                     void *stream);
 
 #ifdef __cplusplus
 }

@@ -186,6 +186,8 @@ _PROTOS = {
     "ktm_vgrad_velocity": (_i32, [_vp, _vp, _vp, _vp]),
     "ktm_vgrad_eval": (_i32, [_vp, _vp, C.POINTER(C.c_double), _vp, _vp, _vp]),
     "ktm_vgrad_pairs": (_i64, [_vp]),
+    "ktm_selftest_limited": (_i32, [_vp, _i64, _f32, _i32, _vp, _vp]),
+    "ktm_selftest_eom": (_i32, [_vp, _vp, _i64, _vp, _vp, _vp]),
     "ktm_selftest_traveltime": (_i32, [_vp, _i64, _f32, _i32, _vp, _vp, _vp, _vp, _vp]),
 }
 

@@ -1547,6 +1547,28 @@ __global__ void k_selftest_traveltime(const float4 *__restrict__ in, int64_t n, 
     t_ref[i] = qq < nsf ? (int)qq : ns;
 }
 
+/* the exact migration kernel's form of q, p nsh, without a further rounding */
+__global__ void k_selftest_limited(const float4 *__restrict__ in, int64_t n, float dt, int ns,
+                                   double *__restrict__ q)
+{
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const float4 v = in[i];
+    const float nsh = (float)ns + 0.5f;
+    q[i] = (double)fast_p(v.x, v.y, fast_rsn(v.w, dt, nsh), fast_tqn((int)v.z, nsh)) * (double)nsh;
+}
+
+extern "C" int ktm_selftest_limited(const float *in4, int64_t n, float dt, int ns, double *q,
+                                    void *stream)
+{
+    if (n < 0 || (n && (!in4 || !q))) return KTM_ERR_ARG;
+    if (!n) return KTM_OK;
+    hipLaunchKernelGGL(k_selftest_limited, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
+                       (hipStream_t)stream, (const float4 *)in4, n, dt, ns, q);
+    HIP_TRY(hipGetLastError());
+    return KTM_OK;
+}
+
 extern "C" int ktm_selftest_sqrt(const float *x, int64_t n, float *out_hw, void *stream)
 {
     if (n < 0 || (n && (!x || !out_hw))) return KTM_ERR_ARG;

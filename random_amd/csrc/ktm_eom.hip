@@ -321,9 +321,10 @@ __device__ __forceinline__ float eom_taper(float df)
     return (float)(0.5 + div_cr(atan(z), EOM_PI, RPI));
 }
 
-/* RN(sqrt(x)), x >= 0: v_sqrt_f32 to one ulp and the two tests of its
- * neighbours, without the scaling of subnormal radicands unless a lane has
- * one below 2^-96 */
+/* RN(sqrt(x)), x >= 0, from v_sqrt_f32 to one ulp: the correction by the exact
+ * signs of x - s (s -+ ulp), as in the AMDGPU backend's expansion of a correctly
+ * rounded float square root, without that expansion's scaling of subnormal
+ * radicands unless a lane has one below 2^-96 */
 __device__ __forceinline__ float sqrt_rn(float x)
 {
     if (__ballot(x < 0x1p-96f && x > 0.0f)) return __builtin_sqrtf(x);
@@ -332,6 +333,26 @@ __device__ __forceinline__ float sqrt_rn(float x)
     const float up = __uint_as_float(__float_as_uint(s) + 1u);
     const float r = __builtin_fmaf(-dn, s, x) <= 0.0f ? dn : s;
     return __builtin_fmaf(-up, s, x) > 0.0f ? up : r;
+}
+
+__global__ void k_selftest_eom(const float *__restrict__ d, const float *__restrict__ x, int64_t n,
+                               float *__restrict__ taper, float *__restrict__ root)
+{
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    taper[i] = eom_taper(d[i]);
+    root[i] = sqrt_rn(x[i]);
+}
+
+extern "C" int ktm_selftest_eom(const float *d, const float *x, int64_t n, float *taper, float *root,
+                                void *stream)
+{
+    if (n < 0 || (n && (!d || !x || !taper || !root))) return KTM_ERR_ARG;
+    if (!n) return KTM_OK;
+    hipLaunchKernelGGL(k_selftest_eom, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
+                       (hipStream_t)stream, d, x, n, taper, root);
+    EOM_TRY(hipGetLastError());
+    return KTM_OK;
 }
 
 struct EomArgs {

@@ -245,3 +245,34 @@ def test_eom_workgroups_of_one_and_of_four_waves(cuda, ns, nh):
     assert np.array_equal(fold.cpu().numpy(), f0)
     assert rel_l2(c, c0) <= 1e-6
     assert ns < 64 or np.abs(c0).max() > 0
+
+
+@pytest.mark.parametrize("ns,base", [(192, 1400), (256, 1050)])
+def test_eom_gathers_beyond_32_bit_offsets(cuda, ns, base):
+    """A CSP of more than 2^30 samples, its bins of 2^-12 m beyond 4 GiB: the
+    same sums as in a plan whose first bin lies there (shifting by a whole number
+    of bins is exact for a width of a power of two)."""
+    width = 2.0 ** -12
+    shift = int(base / width)
+    bins = (1 << 30) // ns + 400_000
+    assert 4 * shift * ns > 2 ** 32 and bins > shift
+    print(f"case: {bins} bins x {ns} samples, 200 traces", flush=True)
+    rng = np.random.default_rng(ns)
+    coords = np.zeros((200, 4), np.int32)
+    cmp = rng.uniform(base - 60.0, base + 60.0, 200)
+    coords[:, 0] = np.round(100.0 * (cmp - 150.0))
+    coords[:, 2] = np.round(100.0 * (cmp + 150.0))
+    tr = torch.from_numpy(rng.standard_normal((200, ns)).astype(np.float32)).to(cuda)
+    co = torch.from_numpy(coords).to(cuda)
+    out = []
+    for oh, nh in ((0, bins), (base, bins - shift)):
+        cfg = EomConfig(ox=0.0, oy=0.0, angle_e_to_n=0.0, oxcsp=0.0, oycsp=0.0, excsp=0.0, eycsp=0.0,
+                        scale_xy=0.01, dcsp_x=12.5, dcsp_y=0.0, dh=width, nh=nh, oh=oh, aperture=2500.0,
+                        jobs_x=1, jobs_y=1, ntblock=1000, velocity_start=9000.0, velocity_end=9000.0)
+        plan = EomPlan(cfg, ns, 0.004)
+        csp, fold, n = plan.migrate(tr, co)
+        out.append((csp.reshape(nh, ns)[nh - (bins - shift):], fold.reshape(nh, ns)[nh - (bins - shift):], n))
+    (c0, f0, n0), (c1, f1, n1) = out
+    assert n0 == n1 > 0
+    assert bool((f1[1:-1] != 1.0).any()) and bool(c1[1:-1].any())
+    assert torch.equal(c0[1:-1], c1[1:-1]) and torch.equal(f0[1:-1], f1[1:-1])

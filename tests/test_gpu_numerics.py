@@ -7,6 +7,7 @@ That is exact only if |q_fast - q_ref| <= 4.8e-7 (q_ref + 1), which rests on
 v_sqrt_f32 being within one ulp.  Both facts are checked here.
 """
 import ctypes as C
+import math
 
 import numpy as np
 import pytest
@@ -108,3 +109,63 @@ def test_fast_traveltime_near_integers(cuda):
     assert np.sum(dist < 1e-4) > ok.sum() // 4
     assert err.max() <= EPS
     assert np.array_equal(tk, tr)
+
+
+@pytest.mark.parametrize("ns", [4, 63, 501, 1500, 3001, 6144])
+def test_limited_traveltime_bound_and_index(cuda, ns):
+    """The migration's own form, in units of ns + 1/2 and limited to 1, within
+    the same bound; a limited sample is past the trace."""
+    print(f"case: limited fast form vs reference traveltime, 2^22 samples, ns={ns}", flush=True)
+    rng = np.random.default_rng(ns)
+    n = 1 << 22
+    dt = np.float32(0.004)
+    t = rng.integers(0, ns, n)
+    reach = 3000.0 * dt * ns
+    d = (reach * rng.uniform(0.0, 1.0, (n, 2)) ** 2) ** 2
+    d[: n // 16] = 0.0
+    v = rng.uniform(1400.0, 5000.0, n).astype(np.float32)
+    inp = np.ascontiguousarray(np.stack([d[:, 0], d[:, 1], t, v * v], axis=1), np.float32)
+    _, qr, tk, tr = _run_traveltime(cuda, inp, dt, ns)
+    q = torch.empty(n, dtype=torch.float64, device=cuda)
+    _lib.check(_lib.lib().ktm_selftest_limited(_p(torch.from_numpy(inp).to(cuda)), n, dt, ns, _p(q),
+                                               None), "selftest_limited")
+    q = q.cpu().numpy()
+    at_limit = q == ns + 0.5
+    err = np.abs(q - qr)[~at_limit] / (qr.astype(np.float64) + 1.0)[~at_limit]
+    print(f"  max |q - q_ref| / (q_ref + 1) = {err.max():.3e} (bound {EPS}); {at_limit.sum()} at the "
+          f"limit; T mismatches {np.sum(tk != tr)}", flush=True)
+    assert 0 < at_limit.sum() < n // 2
+    assert err.max() <= EPS
+    assert (qr[at_limit] > ns).all()
+    assert np.array_equal(tk, tr)
+
+
+def test_eom_taper_and_square_root_round_as_the_reference(cuda):
+    """EOM.c:1286-1292: the taper's series and its switch to the full double
+    expression (at |d| = 3.2 ms, and where the sum and its error bound round
+    apart), and the float square root down to the subnormals.  The device's double
+    arctangent and the C library's may be two ulps apart, 1.1e-16 of the sum,
+    whose float has an ulp of 8e-8 times its value 1.27e-4 / |d| for d < -1: were
+    all of them that far apart, 10 of these 10^6 floats would differ; 30 may, by
+    one ulp."""
+    rng = np.random.default_rng(3)
+    edge = np.float32(0.0032).view(np.int32) + np.arange(-4000, 4001, dtype=np.int32)
+    d = np.concatenate([edge.astype(np.int32).view(np.float32), [0.0, 1e-30, 0.00319, 0.0033],
+                        10.0 ** rng.uniform(-9.0, 1.4, 490_000)]).astype(np.float32)
+    d = np.concatenate([d, -d])
+    x = np.concatenate([[0.0, 2.0 ** -149, 2.0 ** -126, 2.0 ** -97, 2.0 ** -96, 2.0 ** -95, 1.0, 2.0, 3e38],
+                        2.0 ** rng.uniform(-149.0, 127.0, d.size - 200_009),
+                        rng.integers(1, 1 << 20, 100_000).astype(np.float64) ** 2,
+                        rng.uniform(0.0, 1e8, 100_000)]).astype(np.float32)
+    assert d.size == x.size
+    print(f"case: taper and square root of {d.size} floats", flush=True)
+    d_d, d_x = torch.from_numpy(d).to(cuda), torch.from_numpy(x).to(cuda)
+    taper, root = torch.empty_like(d_d), torch.empty_like(d_x)
+    _lib.check(_lib.lib().ktm_selftest_eom(_p(d_d), _p(d_x), d.size, _p(taper), _p(root), None),
+               "selftest_eom")
+    z = (200.0 * d.astype(np.float64) / 0.080).tolist()
+    want = np.array([0.5 + math.atan(v) / 3.14159265359 for v in z]).astype(np.float32)
+    u = ulp_diff(taper.cpu().numpy(), want)
+    print(f"  taper: {np.sum(u > 0)} differ, by {u.max()} ulp", flush=True)
+    assert u.max() <= 1 and np.sum(u > 0) <= 30
+    assert np.array_equal(root.cpu().numpy().view(np.int32), np.sqrt(x).view(np.int32))
