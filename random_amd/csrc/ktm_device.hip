@@ -739,16 +739,14 @@ __device__ __forceinline__ float finite(float x) { return fminf(x, 3.402823466e3
  * limited to 1 by the clamp modifier of its sum, at no cost (a v_med3 is a
  * quarter-rate instruction): a limited sample has Q > ns for certain, its
  * index is ns, and half a sample from an integer it is never ambiguous.
- * A trace without a position (NaN or infinite in the caller's geometry), or a
- * velocity whose square underflows, has no traveltime: the reference arithmetic
- * gives NaN or infinity, index ns.  So that p is never NaN (which the limit turns
- * into 0, and floor_p into an index of -1), rsn and the squared distances are
- * kept finite: such a sample is past the trace by the limit, or ambiguous (both
- * distances 0). */
+ * p is never NaN (which the limit would turn into 0, and floor_p into an index of
+ * -1): v2 is at least KTM_V2_MIN, so rsn is finite, and the squared distances are
+ * kept finite.  A trace without a position (NaN or infinite in the caller's
+ * geometry), whose index is ns in the reference arithmetic, is so past the trace
+ * by the limit. */
 __device__ __forceinline__ float fast_rsn(float v2, float dt, float nsh)
 {
-    return finite(
-        (float)(1.0 / ((double)v2 * (double)dt * (double)dt * ((double)nsh * (double)nsh))));
+    return (float)(1.0 / ((double)v2 * (double)dt * (double)dt * ((double)nsh * (double)nsh)));
 }
 __device__ __forceinline__ float fast_tqn(int t, float nsh)
 {
@@ -2092,12 +2090,15 @@ __global__ void k_velocity_check(const float *__restrict__ vel, const int32_t *_
     }
 }
 
-/* v -> v^2 in place (Kirchhoff.c:617), one FP32 product each */
+/* v -> v^2 in place (Kirchhoff.c:617), one FP32 product each, at least
+ * KTM_V2_MIN: below it (v < 3e-13 m/s) every sample away from the source and the
+ * receiver is past the trace either way, and 1/(v dt)^2 would overflow */
+#define KTM_V2_MIN 1.0e-25f
 __global__ void k_square(float *__restrict__ v, int64_t n)
 {
     for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < n;
          e += (int64_t)gridDim.x * blockDim.x)
-        v[e] = v[e] * v[e];
+        v[e] = fmaxf(v[e] * v[e], KTM_V2_MIN);
 }
 
 /* ------------------------------------------------------------------------ */

@@ -354,3 +354,16 @@ def test_trace_counts_in_every_lane_layout_bitexact(cuda, ns, ncols):
         print(f"case: {ntr} traces x {ns} samples, {ncols} columns", flush=True)
         sv.coords = np.ascontiguousarray(coords[:ntr])
         bitexact_case(sv, tr[:ntr].copy(), cuda)
+
+
+def test_velocities_whose_inverse_square_overflows(cuda):
+    """Zero-offset traces on a column of a velocity of 1e-20 m/s (1/(v dt)^2
+    overflows in FP32, the reference's 0 / v^2 does not): the reference's index,
+    T = t, in every sample."""
+    print("case: zero-offset traces, velocities down to 1e-20 m/s", flush=True)
+    sv = small_line(301, ncols=1, jobs_x=1)
+    sv.coords[:, 0::2] = 0
+    sv.vel[..., 1::3] = 1.0e-20
+    tr = np.random.default_rng(1).standard_normal((sv.ntr, sv.ns)).astype(np.float32)
+    _, km, _, n = bitexact_case(sv, tr, cuda)
+    assert n > 0 and (km[..., 1::3] != 0).any()
