@@ -649,27 +649,7 @@ __device__ __forceinline__ int exact_T(float dIS2, float dIR2, float t2, float v
     return qq < (float)ns ? (int)qq : ns;
 }
 
-/* Fast path of the traveltime index.  With r = RN(1/v2) and rdt = RN(1/dt),
- *   q = RN( RN( sqrt_hw(fma(dIS2, r, t2)) + sqrt_hw(fma(dIR2, r, t2)) ) * rdt ).
- * Against the reference value Q = RN(dsr/dt) of exact_T (u = 2^-24):
- *   fma vs RN(t2 + RN(dIS2/v2))            relative 4u on the radicand
- *   -> 2u after the square root, plus the hardware sqrt (<= 1 ulp = 2u)
- *   sum rounding vs the double sum rounded to float         2u
- *   RN(1/dt) and the product rounding vs RN(dsr/dt)         3u
- * so |q - Q| <= 9u Q (first order).  KTM_FAST_EPS = 10u = 5.96e-7 rounded up;
- * the 1 ulp figure of v_sqrt_f32 is checked exhaustively on [1, 4) by the GPU
- * tests, the whole bound on random and near-integer inputs. */
-#define KTM_FAST_EPS 6.0e-7f
-
-__device__ __forceinline__ float fast_q(float dIS2, float dIR2, float r, float t2, float rdt)
-{
-    const float a1 = __builtin_fmaf(dIS2, r, t2);
-    const float a2 = __builtin_fmaf(dIR2, r, t2);
-    const float d = __builtin_amdgcn_sqrtf(a1) + __builtin_amdgcn_sqrtf(a2);
-    return d * rdt;
-}
-
-/* The migration kernel's form, in samples from the start: with
+/* The fast form of the traveltime index, in samples from the start: with
  * rs = RN(1/(v2 dt^2)) (product and quotient in double, one rounding) and
  * tq = 0.25 t^2 (exact for t < 4096, else one rounding),
  *   q = RN( sqrt_hw(fma(dIS2, rs, tq)) + sqrt_hw(fma(dIR2, rs, tq)) ).
@@ -679,7 +659,9 @@ __device__ __forceinline__ float fast_q(float dIS2, float dIR2, float r, float t
  * the square root, plus 2u for v_sqrt_f32; the sum's rounding u; the
  * reference's RN(dsr) and RN(dsr/dt) 2u: |q - Q| <= 7u Q to first order;
  * its tolerance KTM_FAST_EPS_S = 8u leaves 1u for the second-order terms.
- * No multiply by 1/dt is left in the hot loop. */
+ * The 1 ulp figure of v_sqrt_f32 is checked exhaustively on [1, 4) by the GPU
+ * tests, the whole bound on random and near-integer inputs.  The demigration and
+ * the relaxed index take this form, the exact migration that of fast_p. */
 #define KTM_FAST_EPS_S 4.8e-7f
 __device__ __forceinline__ float fast_qs(float dIS2, float dIR2, float rs, float tq)
 {
@@ -694,28 +676,19 @@ __device__ __forceinline__ float fast_rs(float v2, float dt)
 }
 __device__ __forceinline__ float fast_tq(int t) { return (float)(0.25 * (double)t * (double)t); }
 
-/* q clamped to nsh = ns + 0.5 (demigration).  q >= 0 (a sum of square
- * roots).  Beyond ns + 0.5 the reference's Q is > ns as well (|q - Q| <=
- * 1e-6 q), so the sample is discarded either way; the clamped value
- * truncates to ns and is half a sample from an integer, hence never
- * ambiguous.  One clamp serves the index and the ambiguity test.  (The
- * migration kernel clamps at ns instead, see there.) */
-__device__ __forceinline__ float fast_clamp(float q, float nsh) { return fminf(q, nsh); }
+/* q >= 0 (a sum of square roots) clamped to lim, half a sample past an integer
+ * T >= ns (demigration).  Beyond lim the reference's Q is > ns as well (|q - Q|
+ * <= 1e-6 q), so the sample is discarded either way; the clamped value truncates
+ * to T and is never ambiguous.  One clamp serves the index and the ambiguity
+ * test. */
+__device__ __forceinline__ float fast_clamp(float q, float lim) { return fminf(q, lim); }
 
-/* An integer within eps*(q+1) of the clamped q: floor(q) may differ from
- * the reference's floor(Q).  eps is the bound of the fast form in use. */
-__device__ __forceinline__ bool fast_ambiguous(float qc, float eps = KTM_FAST_EPS)
-{
-    const float dev = fabsf(qc - __builtin_rintf(qc));
-    return dev <= __builtin_fmaf(qc, eps, eps);
-}
-
-/* floor of the clamped q, in [0, ns] */
+/* floor of the clamped q */
 __device__ __forceinline__ int fast_T(float qc) { return (int)qc; }
 
-/* staged batches whose taps the Kahan variants sum in plain FP32 before one
- * compensated step */
-#define KTM_KAHAN_FOLD 4
+/* chunks of up to 4 staged rows (one of 8 counts twice) whose taps the Kahan
+ * variants sum in plain FP32 before one compensated step: at most 32 terms */
+#define KTM_KAHAN_CHUNKS 8
 
 /* q clamped to [0, hi] in one instruction (v_med3_f32; q >= 0 is a sum of
  * square roots, so this is min(q, hi) without the canonicalisation of
@@ -866,8 +839,8 @@ typedef __attribute__((address_space(1))) const void global_void;
  * 6.75 ms.  12 waves of K = 8 (six per SIMD) measured the same as 8 of K = 12
  * with 1500 samples, 16 waves in one workgroup 15 % slower (all of a CU's waves
  * at one barrier); slot groups of 2, 4 and 6 within 3 % of 3. */
-template <int K, int W, int NW, int C, int WN, int EU, bool KAHAN, bool FASTIDX>
-__global__ void __launch_bounds__(NW * KTM_WAVE) __attribute__((amdgpu_waves_per_eu(EU, EU)))
+template <int K, int W, int NW, int C, int WN, bool KAHAN, bool FASTIDX>
+__global__ void __launch_bounds__(NW * KTM_WAVE) __attribute__((amdgpu_waves_per_eu(4, 4)))
 k_migrate(const MigArgs a)
 {
     constexpr int NT = NW * KTM_WAVE;
@@ -877,7 +850,7 @@ k_migrate(const MigArgs a)
     constexpr int WT = WN * C;              /* traces of a window */
     constexpr int SB = KTM_WAVE / WT * WT;  /* traces whose gates are evaluated at once */
     constexpr int RING = WN + 1;            /* chunks in LDS: a window's and the next */
-    static_assert(NW % C == 0 && WT <= 16 && K < 16 && K % G == 0,
+    static_assert(NW % C == 0 && WT <= 16 && K < 16 && K % G == 0 && (WN & (WN - 1)) == 0,
                   "remembered samples pack the slot and the trace in 4 bits each");
     extern __shared__ float4 lds4[];
     const int ldl = (int)a.row;             /* LDS row = prepared row (floats) */
@@ -941,7 +914,7 @@ k_migrate(const MigArgs a)
             if (KAHAN && col_ok && part == 0) cmp[k] = a.comp[pix + tl];
         } else {
             /* padding lane: q = 0.5, never flagged by the ambiguity test; it
-             * reads F[0] (and V[0]) into values that are not stored */
+             * reads F[0] into a value that is not stored */
             rs[k] = 0.0f;
             tq[k] = FASTIDX ? 0.0625f : 0.0625f / (nsh * nsh);
             acc[k] = 0.0f;
@@ -956,11 +929,11 @@ k_migrate(const MigArgs a)
     }
 
     /* Kahan variants: the taps are summed onto y = -c in plain FP32 over
-     * 2 KTM_KAHAN_FOLD chunks of at most 4 rows or half as many of 8 (error
-     * <= (terms - 1) u times the terms' magnitudes) and added to the image with one
-     * compensated step, which keeps the compensated error bound of order
-     * u * sum |f| at a fraction of the per-tap cost.  Plain variants add
-     * every tap into the image in trace order, as the reference does. */
+     * KTM_KAHAN_CHUNKS chunks (error <= (terms - 1) u times the terms'
+     * magnitudes) and added to the image with one compensated step, which keeps
+     * the compensated error bound of order u * sum |f| at a fraction of the
+     * per-tap cost.  Plain variants add every tap into the image in trace order,
+     * as the reference does. */
     float y[KAHAN ? K : 1];
 #pragma unroll
     for (int k = 0; k < (KAHAN ? K : 1); ++k) y[k] = -cmp[k];
@@ -1090,10 +1063,9 @@ k_migrate(const MigArgs a)
          * index << 8 (-1: none) and the sum before it */
         int qi = -1;
         float qs = 0.0f;
-        int wnext = 0;
         for (int q = 0; q * C < nb; ++q) {
             /* chunk q's place in its window */
-            const int wq = (WN & (WN - 1)) ? wnext : (q & (WN - 1));
+            const int wq = q & (WN - 1);
             /* chunk q has arrived and every wave is done with chunk q - 1,
              * so with the slot that chunk q + 1 goes to */
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -1247,11 +1219,10 @@ k_migrate(const MigArgs a)
                 }
                 qi = -1;
             }
-            if (KAHAN && wend && (nfold += C > 4 ? WN * (C / 4) : WN) >= 2 * KTM_KAHAN_FOLD) {
+            if (KAHAN && wend && (nfold += C > 4 ? WN * (C / 4) : WN) >= KTM_KAHAN_CHUNKS) {
                 nfold = 0;
                 fold_y();
             }
-            wnext = wq == WN - 1 ? 0 : wq + 1;
             slot = nslot;
         }
         head += nb;
@@ -2568,9 +2539,9 @@ static MigShape mig_shape(int accum)
 {
     const bool kahan = (accum & ~KTM_INDEX_FAST) == KTM_ACCUM_KAHAN;
     if (accum & KTM_INDEX_FAST)         /* no window to keep */
-        return {kahan ? k_migrate<K, W, NW, C, 1, 4, true, true> : k_migrate<K, W, NW, C, 1, 4, false, true>,
+        return {kahan ? k_migrate<K, W, NW, C, 1, true, true> : k_migrate<K, W, NW, C, 1, false, true>,
                 K, W, NW, C, 2};
-    return {kahan ? k_migrate<K, W, NW, C, WN, 4, true, false> : k_migrate<K, W, NW, C, WN, 4, false, false>,
+    return {kahan ? k_migrate<K, W, NW, C, WN, true, false> : k_migrate<K, W, NW, C, WN, false, false>,
             K, W, NW, C, WN + 1};
 }
 
@@ -2640,7 +2611,7 @@ static double mig_cost(const MigShape &m, size_t lds, double wgs, double share, 
  * line, as square as possible in 3-D. */
 static void tile_layout(const ktm_setup *s, int ncol, MigArgs *a)
 {
-    a->tx_cols = s->nyp == 1 ? ncol : (ncol == 8 ? 4 : ncol == 6 ? 3 : ncol == 4 ? 2 : ncol);
+    a->tx_cols = s->nyp == 1 ? ncol : (ncol == 8 ? 4 : ncol == 4 ? 2 : ncol);
     a->ty_cols = ncol / a->tx_cols;
     a->tiles_x = (a->rx1 - a->rx0 + a->tx_cols - 1) / a->tx_cols;
     const int tiles_y = (a->ry1 - a->ry0 + a->ty_cols - 1) / a->ty_cols;
