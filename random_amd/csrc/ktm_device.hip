@@ -269,7 +269,7 @@ __device__ __forceinline__ float load_sample(const TraceSrc &s, int64_t i, int t
  * per tile.
  * Bound by the recurrence's chain for few traces and by memory for a full
  * block: 50,000 IBM records of 1500 samples 319 -> 170 us (3.6 TB/s), 96
- * traces of 501 74 -> 20 us, against one wave that did all of it with a full
+ * traces of 501 74 -> 32 us, against one wave that did all of it with a full
  * double division per sample.  Of the same block with 4 helper waves 180 us,
  * 8 200, tiles of 16 steps 250, and with the division in the recurrence wave
  * and tiles of 64 steps 350. */
@@ -818,7 +818,8 @@ typedef __attribute__((address_space(1))) const void global_void;
  * next of the same source: traces in shot order, which most surveys come in,
  * cost one root per sample instead of two (12 offset classes x 2503 samples:
  * 6.3 -> 5.6 ms, the pair L, L^T of the 200-shot line 39.0 -> 36.5 ms), sources
- * at random 2 % more for the roots computed apart.
+ * at random 2 % more for the roots computed apart; with 12 slots and compensated
+ * sums the roots do not fit the registers (33 of them in scratch).
  * A sample past the trace reads the zero F[ns] and does not count for fold.
  * With the gates each lane bounds, for its trace and every slot of the wave,
  * the largest q (the traveltime at the slot's largest constants): slots before
@@ -833,10 +834,10 @@ typedef __attribute__((address_space(1))) const void global_void;
  * add into the image, and 2/3 of an instruction for the test (14.5 in all with
  * the gates, the staging and the ambiguous samples).  Against rows staged
  * through registers between two barriers and every sample past the trace on
- * the rare path: 16,000 traces x 1500 samples into 400 x 400 columns 295 ->
- * 253 ms, 20,000 BF16-stored x 1251 into 150 x 150 222 -> 187 ms, the
- * 40-shot line 3.75 -> 2.85 ms (2.40 with chunks of 8 rows), 12 classes x 2503 samples x 500 columns 10.9 ->
- * 6.75 ms.  12 waves of K = 8 (six per SIMD) measured the same as 8 of K = 12
+ * the rare path, the lane shapes and the kept root included: 16,000 traces x 1500
+ * samples into 400 x 400 columns 298 -> 263 ms, 20,000 BF16-stored x 1251 into 150
+ * x 150 222 -> 171 ms, the 40-shot line 3.91 -> 2.39 ms, 12 classes x 2503 samples
+ * x 500 columns 11.5 -> 5.5 ms.  12 waves of K = 8 (six per SIMD) measured the same as 8 of K = 12
  * with 1500 samples, 16 waves in one workgroup 15 % slower (all of a CU's waves
  * at one barrier); slot groups of 2, 4 and 6 within 3 % of 3. */
 template <int K, int W, int NW, int C, int WN, bool KAHAN, bool FASTIDX>
@@ -1032,16 +1033,16 @@ k_migrate(const MigArgs a)
             const float ax = IX - g0.x, ay = IY - g0.y, bx = IX - g0.z, by = IY - g0.w;
             g_is = ax * ax + ay * ay;
             g_ir = bx * bx + by * by;
-            if (SPEC) {
-                g_is = finite(g_is);
-                g_ir = finite(g_ir);
-            }
             const float cx = IX - g1.x, cy = IY - g1.y;
             const float ex = scx - g1.x, ey = scy - g1.y;
             gp = ex * ex + ey * ey < sthr && cx * cx + cy * cy < a.ap_x2thr;
         }
         const uint64_t pm = col_ok ? __ballot(gp) : 0ull;
         npass += __popcll(pm);
+        if (SPEC) {
+            g_is = finite(g_is);
+            g_ir = finite(g_ir);
+        }
         /* the slots that cannot reach the end of lane j's trace, the first
          * kend: their largest q (FMA and v_sqrt_f32 to 1 ulp each, so 1e-5
          * covers their rounding) is below ns - 1; and the trace's ambiguity

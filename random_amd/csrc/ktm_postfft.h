@@ -30,9 +30,9 @@
  * last one writes t < ns <= N / 2; both with consecutive lanes on consecutive
  * samples.  LDS rows are padded by one double2 per 16 so that lanes 16 points
  * apart spread over the banks.
- * 160,000 traces of 1500 samples: 1.3 ms (2.1 before, with a Stockham
- * reordering and two barriers in every pass), 2.2 TB/s of traces and fold in
- * and image out.  It is bound by FP64 instructions (about 1500 per lane, 0.9
+ * 160,000 traces of 1500 samples: 1.3 to 1.7 ms, 1.39 on average (2.1 before,
+ * with a Stockham reordering and two barriers in every pass), 2.1 TB/s of traces
+ * and fold in and image out.  It is bound by FP64 instructions (about 1500 per lane, 0.9
  * ms at one per four cycles) and by LDS latency at the three waves per SIMD
  * that 52 KB per workgroup leave: without its input loads it takes 1.2 ms.
  */

@@ -16,12 +16,10 @@ from random_amd.lsm import Operator, dot_test
 
 pytestmark = pytest.mark.gpu
 
-# sample counts at and around the lane-layout boundaries of ktm_migrate_block
-# (K samples per lane x W waves per column: 8x1 <= 512 < 8x2 <= 1024 < 12x2
-# <= 1536 < 8x4 <= 2048 < 12x4 <= 3072 < 8x8 <= 4096 < 12x8 <= 6144; images
-# too small for two workgroups per CU take 4x2 and 4x4 below 1025 samples,
-# as the 40-column line here does -- test_wide_image_layouts_bitexact keeps
-# the default ones covered)
+# sample counts on both sides of capacities of the lane layouts of
+# ktm_migrate_block (64 K W samples of K per lane and W waves per column), for
+# the 40-column line here and a 4104-column one; LANES below names a size for
+# every layout
 NS_CASES = [4, 63, 512, 513, 1024, 1025, 1536, 1537, 2048, 2049, 3072, 3073, 4096, 4097, 6144]
 
 
@@ -257,9 +255,9 @@ def test_prepared_rows_at_any_float(cuda):
     assert bool(km.any()) and torch.equal(km, km2) and torch.equal(fold, fold2)
 
 
-# both sides of every boundary of the lane layouts by samples per lane and
-# waves per column (2, 4, 6, 8, 10 or 12 x 64 x 1, 2, 4 or 8); the 4104-column
-# image takes the widest lanes of its length, the 40-column one the narrowest
+# both sides of the remaining capacities of the lane layouts by samples per lane
+# and waves per column (2, 4, 6, 8, 10 or 12 x 64 x 1, 2, 4 or 8); the
+# 4104-column image takes wide lanes, the 40-column one narrow ones
 LAYOUT_NS = [256, 257, 384, 385, 640, 641, 768, 769, 1280, 1281, 2560, 2561, 5120, 5121]
 
 
