@@ -176,7 +176,7 @@ def valu_probe(dev, modes=tuple(VALU_MODES), waves_per_simd=(8,), target_ms=40.0
 # v_sqrt_f32, CVT = conversions, INT32 = v_add_u32 and v_lshl_add_u32;
 # v_min/v_med3, v_rndne, v_cmp, v_cndmask, v_readlane are in no class.
 KMIG_COUNTS = {
-    "exact": {"kernel": "k_migrate<12, 2, 8, 4, 2, 4, false, false>",
+    "exact": {"kernel": "k_migrate<12, 2, 8, 4, 2, false, false>",
               "contributions": 1806379368000,
               "launch_ms": 830.31, "clock_ghz": 2.382, "valu": 399382949703,
               "fma_f32": 123061932252, "add_f32": 98669530749, "mul_f32": 3665208252,
@@ -184,7 +184,7 @@ KMIG_COUNTS = {
               "fma_f64": 6214502668, "add_f64": 407006653, "mul_f64": 1808376454,
               "trans_f64": 900188227, "int64": 3643298780, "salu": 144148207394,
               "lds": 30424527558},
-    "fast_kahan": {"kernel": "k_migrate<12, 2, 8, 4, 1, 4, true, true>",
+    "fast_kahan": {"kernel": "k_migrate<12, 2, 8, 4, 1, true, true>",
                    "contributions": 1806379368000,
                    "launch_ms": 555.53, "clock_ghz": 2.381, "valu": 270874098032,
                    "fma_f32": 58724046808, "add_f32": 65307199744, "mul_f32": 910043424,
