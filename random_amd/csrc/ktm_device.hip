@@ -3114,7 +3114,9 @@ static int demig_order(const ktm_plan *cp, const ktm_trace_geom *geom, int64_t n
         if (p->d_dm_tmp) HIP_TRY(hipFree(p->d_dm_tmp));
         p->d_dm_tmp = nullptr;
         p->dm_tmp_bytes = 0;
-        if (plan_alloc(p, (char **)&p->d_dm_tmp, need) != KTM_OK) return KTM_ERR_NOMEM;
+        char *tmp = nullptr;
+        if (plan_alloc(p, &tmp, need) != KTM_OK) return KTM_ERR_NOMEM;
+        p->d_dm_tmp = tmp;
         p->dm_tmp_bytes = need;
     }
     hipLaunchKernelGGL(k_demig_keys, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, hs, geom, n,
